@@ -142,9 +142,15 @@ void* scratch_on_current_device(hipError_t* err) {
 // owner, (device, stream) -- launches on one stream run in order, launches on different streams may
 // overlap -- and an event recorded behind the last launches that used it.  A buffer changes hands
 // (a buffer its owner outgrew, or the least recently used one when all MAX_HELD entries are
-// taken) by making the new owner's stream wait for that event: no host synchronisation, no free
-// and no allocation inside a matmul call beyond the first ones.  Memory goes back to the device
-// only through adr_release_held_workspace*, which wait for the event first.
+// taken) by making the new owner's stream wait for that event: no free and no allocation inside a
+// call beyond the first ones.  Memory goes back to the device only through
+// adr_release_held_workspace*, which wait for the event first.
+// An event costs the stream 3 us (a barrier packet and the flush behind it: a 41.5 us kernel launched
+// again and again takes 44.4 us with one behind each) and the host 1.4 us, so none is recorded behind a
+// use until it can be of use: while entries are free no buffer that has an owner changes hands, a
+// buffer is outgrown or released with its owner's stream at hand (recorded then), and only the pool
+// filling up asks for events of uses that are over -- of streams that may not exist any more.  That
+// waits for the device, once; from then on every use records its event.
 constexpr int MAX_HELD = 16;
 constexpr int64_t HELD_FLOOR = (int64_t)16 << 20;
 struct Held {
@@ -153,7 +159,8 @@ struct Held {
   bool owned;
   void* ptr;
   int64_t bytes;
-  hipEvent_t last_use;  // recorded on the owner's stream behind the last launches that used ptr
+  hipEvent_t last_use;  // recorded on the owner's stream behind the last launches that used ptr ...
+  bool pending;         // ... unless this is set: nothing has been recorded behind them yet
   uint64_t tick;        // value of held_clock at the last use
 };
 std::mutex held_mutex;
@@ -179,9 +186,33 @@ bool held_allowed(hipStream_t stream) {
   return st == hipStreamCaptureStatusNone;
 }
 
+// Records the event behind the last use of an entry whose owner's stream is at hand.
+bool held_record(Held* h) {
+  if (h->pending && hipEventRecord(h->last_use, h->stream) == hipSuccess) h->pending = false;
+  if (h->pending) (void)hipGetLastError();
+  return !h->pending;
+}
+
+// Waits until no launch on the current device uses any buffer (see above).  In relaxed capture mode: it
+// must not disturb a capture that another stream of the process is in.
+bool held_wait_for_device(int dev) {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  const hipError_t e = hipDeviceSynchronize();
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  for (int i = 0; i < held_count; i++)
+    if (held[i].device == dev) held[i].pending = false;
+  return true;
+}
+
 // `stream` takes over entry h: everything the previous owner launched on the buffer is ordered
 // before whatever `stream` launches next.
 bool held_take_over(Held* h, hipStream_t stream) {
+  if (h->pending && !held_wait_for_device(h->device)) return false;
   if (hipStreamWaitEvent(stream, h->last_use, 0) != hipSuccess) {
     (void)hipGetLastError();
     return false;
@@ -189,6 +220,13 @@ bool held_take_over(Held* h, hipStream_t stream) {
   h->stream = stream;
   h->owned = true;
   return true;
+}
+
+// Entry h, which its owner has outgrown, is free to be taken over.
+void held_outgrown(Held* h) {
+  if (!h) return;
+  held_record(h);
+  h->owned = false;
 }
 
 // A buffer of at least `want` bytes for (current device, stream), or null (then the caller runs
@@ -212,7 +250,7 @@ Held* held_buffer(hipStream_t stream, int64_t want) {
   // a buffer some stream outgrew that is large enough
   for (int i = 0; i < held_count; i++)
     if (!held[i].owned && held[i].device == dev && held[i].bytes >= want && held_take_over(&held[i], stream)) {
-      if (mine) mine->owned = false;
+      held_outgrown(mine);
       return &held[i];
     }
   if (held_count < MAX_HELD) {
@@ -235,9 +273,9 @@ Held* held_buffer(hipStream_t stream, int64_t want) {
       (void)hipGetLastError();  // out of memory: the product runs without a workspace
       return declined();
     }
-    if (mine) mine->owned = false;  // outgrown: stays in the pool for a stream that wants less
+    held_outgrown(mine);  // stays in the pool for a stream that wants less
     Held* h = &held[held_count++];
-    *h = Held{dev, stream, true, p, size, ev, 0};
+    *h = Held{dev, stream, true, p, size, ev, false, 0};
     held_total += size;
     return h;
   }
@@ -248,7 +286,7 @@ Held* held_buffer(hipStream_t stream, int64_t want) {
         (!lru || held[i].tick < lru->tick))
       lru = &held[i];
   if (lru && held_take_over(lru, stream)) {
-    if (mine) mine->owned = false;
+    held_outgrown(mine);
     return lru;
   }
   return declined();
@@ -257,11 +295,20 @@ Held* held_buffer(hipStream_t stream, int64_t want) {
 // behind the launches that used h->ptr on its owner's stream
 void held_used(Held* h) {
   h->tick = ++held_clock;
-  if (hipEventRecord(h->last_use, h->stream) != hipSuccess) (void)hipGetLastError();
+  h->pending = true;
+  if (held_count == MAX_HELD) held_record(h);
 }
 
-// Frees entry i (waits for its last use first) and closes the gap.  held_mutex is held.
-void held_free(int i) {
+// Frees entry i (waits for its last use first) and closes the gap.  held_mutex is held.  `alive`: its
+// owner's stream certainly exists.
+void held_free(int i, bool alive) {
+  if (!(alive && held_record(&held[i])) && held[i].pending) {
+    int dev = held[i].device;
+    (void)hipGetDevice(&dev);
+    if (dev != held[i].device) (void)hipSetDevice(held[i].device);
+    (void)hipDeviceSynchronize();
+    if (dev != held[i].device) (void)hipSetDevice(dev);
+  }
   (void)hipEventSynchronize(held[i].last_use);
   (void)hipEventDestroy(held[i].last_use);
   (void)hipFree(held[i].ptr);
@@ -349,13 +396,13 @@ int adr_release_held_workspace(adr_stream_t stream) {
   if (hipError_t e = hipGetDevice(&dev)) return (int)e;
   std::lock_guard<std::mutex> lock(held_mutex);
   for (int i = held_count - 1; i >= 0; i--)
-    if (held[i].device == dev && (!held[i].owned || held[i].stream == (hipStream_t)stream)) held_free(i);
+    if (held[i].device == dev && (!held[i].owned || held[i].stream == (hipStream_t)stream)) held_free(i, held[i].owned);
   return ADR_OK;
 }
 
 int adr_release_held_workspace_all(void) {
   std::lock_guard<std::mutex> lock(held_mutex);
-  while (held_count > 0) held_free(held_count - 1);
+  while (held_count > 0) held_free(held_count - 1, false);
   return ADR_OK;
 }
 

@@ -154,14 +154,15 @@ int adr_matmul_f16_noalloc(adr_stream_t stream, uint16_t* output, const uint16_t
  * reference).  Those entry points keep the reference's argument tuples and so have no workspace
  * argument; where a workspace pays -- the products adr_matmul_f16_ws splits along K -- they take
  * one from a pool inside the library.  A buffer belongs to a (device, stream) pair: it is allocated
- * with hipMalloc at the first call on that stream that wants one (16 MiB doubling up to the limit)
- * and carries an event recorded behind the last launches that used it.  When a stream wants more
- * than its buffer holds it gets a larger one and the old buffer stays in the pool for any stream
- * that wants less; when all 16 entries of the pool are taken, a stream without a buffer takes over
- * the least recently used one that is large enough.  A buffer changes hands by making the new
- * owner's stream wait for the buffer's event (hipStreamWaitEvent): nothing is freed, allocated or
- * synchronised inside a matmul call beyond those first allocations, and the pool never holds more
- * than 16 buffers of at most the limit each.  Calls on one stream share a buffer and run in stream
+ * with hipMalloc at the first call on that stream that wants one (16 MiB doubling up to the limit).
+ * When a stream wants more than its buffer holds it gets a larger one and the old buffer stays in
+ * the pool for any stream that wants less; when all 16 entries of the pool are taken, a stream
+ * without a buffer takes over the least recently used one that is large enough.  A buffer changes
+ * hands by making the new owner's stream wait for an event behind the buffer's last use
+ * (hipStreamWaitEvent).  Those events cost more than they order, so they are recorded only once all
+ * 16 entries are taken; the first call that takes over a buffer used before that waits for the device.
+ * Beyond that and the first allocations nothing is freed, allocated or synchronised inside a call,
+ * and the pool never holds more than 16 buffers of at most the limit each.  Calls on one stream share a buffer and run in stream
  * order; the pool is locked while a call that uses it launches, so any thread may call on any
  * stream.  No buffer is used or allocated -- the call runs exactly as with a limit of 0 -- while
  * the stream is being captured into a graph (the launches would tie the buffer to a graph that may
@@ -175,11 +176,11 @@ int adr_matmul_f16_noalloc(adr_stream_t stream, uint16_t* output, const uint16_t
  * adr_set_held_workspace_limit: bytes per buffer (default ADR_HELD_WORKSPACE_DEFAULT_BYTES =
  * 128 MiB); 0 switches the pool off for later calls (buffers already allocated stay until
  * released).  adr_held_workspace_bytes: bytes the pool holds now.
- * adr_release_held_workspace(stream): waits for the last launches that used them (the buffers'
- * events, not the device) and frees, on the current device, the buffers `stream` owns and those no
- * stream owns any more; call it before destroying a stream.  adr_release_held_workspace_all: the
- * same for every buffer on every device.  (hipFree itself may wait for other work on the device:
- * these two are not for the hot path.)  Later calls allocate afresh.
+ * adr_release_held_workspace(stream): waits for what `stream` has been given so far and frees, on the
+ * current device, the buffers it owns and those no stream owns any more; call it before destroying
+ * a stream.  adr_release_held_workspace_all: frees every buffer on every device, waiting for the
+ * devices.  (hipFree itself may wait for other work on the device: these two are not for the hot
+ * path.)  Later calls allocate afresh.
  * Callers that must not allocate at all use adr_matmul_f16_noalloc or the _ws forms, which never
  * touch the pool.
  *
