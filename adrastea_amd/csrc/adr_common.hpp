@@ -335,7 +335,10 @@ hipError_t launch_error_stats(hipStream_t stream, float* out, const void* lhs, c
 hipError_t launch_attention(hipStream_t stream, half_t* out, const half_t* q, const half_t* k,
                             const half_t* v, int heads, int m, int n, int d, int so_y, int so_z,
                             int sq_y, int sq_z, int sk_y, int sk_z, int sv_y, int sv_z, float scale,
-                            float temp, uint32_t mask);
+                            float temp, uint32_t mask, void* workspace, int64_t workspace_bytes);
+// Scratch bytes that launch would use when at most `avail` can be had (0: no keys are split).
+int64_t attention_workspace_bytes(int heads, int m, int n, int d, int sq_y, int sk_y, int sv_y, uint32_t mask,
+                                  int64_t avail);
 hipError_t launch_softmax_rows(hipStream_t stream, half_t* out, const half_t* in, int64_t rows,
                                int w, float temp);
 
