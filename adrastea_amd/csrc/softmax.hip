@@ -5,9 +5,9 @@
 //   out_i = fp16( expf(v_i - max_j v_j) / sum_j expf(v_j - max_j v_j) )
 // The operation is bound by reading and writing the tensor once each.  Rows of up to 4096
 // elements are held in registers by one wavefront (one pass over memory, shuffle reductions):
-// 16-byte accesses where the rows are 16-byte aligned, shifted dword accesses where they start
-// at any even address (a row length that is no multiple of 8); longer rows take a three-pass
-// kernel with one workgroup per row.
+// 16-byte accesses of the row's own elements where the rows are 16-byte aligned, of the aligned
+// pieces a row touches where they start at any even address (a row length that is no multiple of
+// 8); longer rows take a three-pass kernel with one workgroup per row.
 #include "adr_common.hpp"
 
 namespace adr {
@@ -94,12 +94,99 @@ __global__ __launch_bounds__(256) void softmax_rows_reg_kernel(half_t* out, cons
   }
 }
 
-// The same for rows that start at any even address and hold any number of elements (w <= 512 * NV):
-// a sequence length that is no multiple of 8 (Whisper's 1500 positions, CLIP's 77 and 257, any odd
-// prompt length).  Chunks of eight halves counted from the row's first element, moved with
-// load8_any / store8_any; the row's last, partial chunk is stored element by element.
+// The same for rows that start at any even address and hold any number of elements: a sequence
+// length that is no multiple of 8 (Whisper's 1500 positions, CLIP's 77 and 257, any odd prompt
+// length).  Bound by memory once its requests are whole: chunks are the 16-byte pieces of the address
+// space the row touches, not of the row, so every load is one aligned 16-byte access -- the first
+// and the last chunk of a row bring elements of the rows beside it, which are replaced by -inf -- and
+// so is every store where `out` lies as `in` does (in place always); a row's end pieces go out as
+// the dwords and halves that are its own.  Chunks counted from the row's first element had to be
+// shifted into place, a second request per chunk: 48000 rows of 1500 80 -> 64 us = 4.5 TB/s, 30000 of
+// them 52.7 -> 42.5, 32016 of 2001 65.8 -> 52.5, 24008 of 3001 76.4 -> 59.7, 32760 of 4095 119.5 -> 103,
+// 12240 of 1530 22.7 -> 19.1; 19232 of 601 19.7 and 16352 of 2044 29.7 either way.  (Cached stores
+// instead of streaming ones, and a contiguous piece of the tensor for each die, change nothing.)
+// NV: chunks per lane; every row of the tensor touches at most 64 NV chunks (see the launch).
 template <int NV>
 __global__ __launch_bounds__(256) void softmax_rows_anyrow_kernel(half_t* out, const half_t* in,
+                                                                  int64_t rows, int w, float temp) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t row = (int64_t)blockIdx.x * 4 + wave;
+  if (row >= rows) return;
+  const half_t* src = in + row * w;
+  half_t* dst = out + row * w;
+  const uintptr_t base = (uintptr_t)src & ~(uintptr_t)15;
+  const int lead = (int)((uintptr_t)src & 15) >> 1;  // elements of the first chunk before the row
+  const int chunks = (lead + w + 7) >> 3;
+  const bool same = (((uintptr_t)dst ^ (uintptr_t)src) & 15) == 0;
+  half8_t x[NV];
+  // (the tensor's own first and last row alone can have chunks that reach outside of it: those rows
+  // are read element by element)
+  if (base >= (uintptr_t)in && base + 16 * (uintptr_t)chunks <= (uintptr_t)(in + rows * w)) {
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+      x[i] = *(const ADR_GLOBAL_AS half8_t*)(base + 16 * (uintptr_t)min(i * 64 + lane, chunks - 1));
+  } else {
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+#pragma unroll
+      for (int e = 0; e < 8; e++)
+        x[i][e] = src[min(max((i * 64 + lane) * 8 - lead + e, 0), w - 1)];
+  }
+  float v[NV][8];
+  float mx = -INFINITY;
+  const bool unit_temp = temp == 1.0f;
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    const int c = (i * 64 + lane) * 8 - lead;  // the chunk's first element, as counted from the row's
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[i][e] = unit_temp ? (float)x[i][e] : (float)x[i][e] / temp;
+    if (i == 0 || (i + 1) * 64 >= chunks) {  // (whole chunks for all lanes in between)
+#pragma unroll
+      for (int e = 0; e < 8; e++) v[i][e] = (unsigned)(c + e) < (unsigned)w ? v[i][e] : -INFINITY;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) mx = fmaxf(mx, v[i][e]);
+  }
+  mx = wave_max(mx);
+  float sum = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NV; i++)
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      v[i][e] = exp_neg(v[i][e] - mx);  // (-inf - mx: 0 for the elements beside the row)
+      sum += v[i][e];
+    }
+  sum = wave_sum(sum);
+  const float rs = 1.0f / sum;
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    const int c = (i * 64 + lane) * 8 - lead;
+    half8_t r;
+#pragma unroll
+    for (int e = 0; e < 8; e++) r[e] = (half_t)(v[i][e] * rs);
+    if (c >= 0 && c + 8 <= w) {
+      if (same) __builtin_nontemporal_store(r, (half8_t*)(dst + c));
+      else store8_any(dst + c, r);
+    } else if (c < w) {
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        const bool first = (unsigned)(c + e) < (unsigned)w, second = (unsigned)(c + e + 1) < (unsigned)w;
+        if (first && second && same) *(half2_t*)(dst + c + e) = half2_t{r[e], r[e + 1]};
+        else {
+          if (first) dst[c + e] = r[e];
+          if (second) dst[c + e + 1] = r[e + 1];
+        }
+      }
+    }
+  }
+}
+
+// The same on chunks counted from the row's first element, moved with load8_any / store8_any: for the
+// few lengths just short of 512 or 1024 whose aligned pieces are one more per lane, which there costs
+// more than the shifting (8168 rows of 1021 11.7 us against 13.5, 8144 of 509 6.9 against 10.0; from
+// 1500 on it no longer does: 16376 of 2047 32.6 against 33.0).
+template <int NV>
+__global__ __launch_bounds__(256) void softmax_rows_shifted_kernel(half_t* out, const half_t* in,
                                                                   int64_t rows, int w, float temp) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t row = (int64_t)blockIdx.x * 4 + wave;
@@ -196,14 +283,27 @@ hipError_t launch_softmax_rows(hipStream_t stream, half_t* out, const half_t* in
     const int64_t blocks = (rows + 3) / 4;
     if (blocks > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     const dim3 grid((unsigned)blocks), block(256);
-    if (w <= 512)
-      hipLaunchKernelGGL(softmax_rows_anyrow_kernel<1>, grid, block, 0, stream, out, in, rows, w, temp);
-    else if (w <= 1024)
-      hipLaunchKernelGGL(softmax_rows_anyrow_kernel<2>, grid, block, 0, stream, out, in, rows, w, temp);
-    else if (w <= 2048)
-      hipLaunchKernelGGL(softmax_rows_anyrow_kernel<4>, grid, block, 0, stream, out, in, rows, w, temp);
-    else
-      hipLaunchKernelGGL(softmax_rows_anyrow_kernel<8>, grid, block, 0, stream, out, in, rows, w, temp);
+    // Chunks per lane as the row that starts worst needs them: rows start at `in` plus multiples of w,
+    // so their first chunks hold as many elements of other rows as `in` does modulo the largest power
+    // of two in w (or 8), and at most that much short of a chunk more.
+    const int g = w % 2 ? 1 : w % 4 ? 2 : w % 8 ? 4 : 8;
+    const int lead = 8 - g + (int)(((uintptr_t)in & 15) >> 1) % g;
+    const int per_lane = ((lead + w + 7) / 8 + 63) / 64;
+    if (per_lane == 2 && w <= 512)
+      hipLaunchKernelGGL(softmax_rows_shifted_kernel<1>, grid, block, 0, stream, out, in, rows, w, temp);
+    else if (per_lane == 3 && w <= 1024)
+      hipLaunchKernelGGL(softmax_rows_shifted_kernel<2>, grid, block, 0, stream, out, in, rows, w, temp);
+    else switch (per_lane) {
+      case 1: hipLaunchKernelGGL(softmax_rows_anyrow_kernel<1>, grid, block, 0, stream, out, in, rows, w, temp); break;
+      case 2: hipLaunchKernelGGL(softmax_rows_anyrow_kernel<2>, grid, block, 0, stream, out, in, rows, w, temp); break;
+      case 3: hipLaunchKernelGGL(softmax_rows_anyrow_kernel<3>, grid, block, 0, stream, out, in, rows, w, temp); break;
+      case 4: hipLaunchKernelGGL(softmax_rows_anyrow_kernel<4>, grid, block, 0, stream, out, in, rows, w, temp); break;
+      case 5: hipLaunchKernelGGL(softmax_rows_anyrow_kernel<5>, grid, block, 0, stream, out, in, rows, w, temp); break;
+      case 6: hipLaunchKernelGGL(softmax_rows_anyrow_kernel<6>, grid, block, 0, stream, out, in, rows, w, temp); break;
+      case 7: hipLaunchKernelGGL(softmax_rows_anyrow_kernel<7>, grid, block, 0, stream, out, in, rows, w, temp); break;
+      case 8: hipLaunchKernelGGL(softmax_rows_anyrow_kernel<8>, grid, block, 0, stream, out, in, rows, w, temp); break;
+      default: hipLaunchKernelGGL(softmax_rows_anyrow_kernel<9>, grid, block, 0, stream, out, in, rows, w, temp); break;
+    }
   } else {
     if (rows > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL(softmax_rows_general_kernel, dim3((unsigned)rows), dim3(256), 0, stream, out,
