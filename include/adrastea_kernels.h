@@ -10,7 +10,7 @@
  * with any other device current, every launching entry point returns ADR_EUNSUPPORTED_DEVICE
  * (the device's architecture, compute-unit and die counts are queried once per device and
  * cached).  Beside that cache the library keeps one piece of state: the pool of workspaces that
- * adr_matmul_f16, adr_matmul_nt_f16 and (on request) adr_matmul_nt_fp16u8 draw from, grown on
+ * adr_matmul_f16, adr_matmul_nt_f16, adr_attention_f16 and (on request) adr_matmul_nt_fp16u8 draw from, grown on
  * demand and given back through adr_release_held_workspace* (adr_set_held_workspace_limit below;
  * 0 switches it off).
  *
@@ -153,7 +153,8 @@ int adr_matmul_f16_noalloc(adr_stream_t stream, uint16_t* output, const uint16_t
  * The workspaces that adr_matmul_f16 and adr_matmul_nt_f16 hold themselves (no counterpart in the
  * reference).  Those entry points keep the reference's argument tuples and so have no workspace
  * argument; where a workspace pays -- the products adr_matmul_f16_ws splits along K -- they take
- * one from a pool inside the library.  A buffer belongs to a (device, stream) pair: it is allocated
+ * one from a pool inside the library, and so does adr_attention_f16 where its query blocks are fewer
+ * than the compute units and workgroups share their keys.  A buffer belongs to a (device, stream) pair: it is allocated
  * with hipMalloc at the first call on that stream that wants one (16 MiB doubling up to the limit).
  * When a stream wants more than its buffer holds it gets a larger one and the old buffer stays in
  * the pool for any stream that wants less; when all 16 entries of the pool are taken, a stream
