@@ -116,6 +116,10 @@ template <int N>
 __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
 }
+// (A barrier alone: it does not wait for LDS reads in flight.  Whoever reads what another wavefront may
+// overwrite behind the next barrier waits for the reads first.  Those issued ahead at the end of a half
+// tile, read_v(cV, 0) and read_k(cK, 0) below, need not: they are used, hence waited for, before the
+// next barrier, and their buffers are refilled behind that one.)
 __device__ __forceinline__ void barrier() {
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("s_barrier" ::: "memory");
@@ -321,7 +325,9 @@ __global__ __launch_bounds__(256 * G, 2) void attention_fwd_kernel(AttnArgs a) {
     wait_vm<2 * NI>();  // Q has landed
 #pragma unroll
     for (int ds = 0; ds < DS; ds++) qf[ds] = *(const half8_t*)(sm + 2 * TILE + w * (32 * ROWB) + offK[ds]);
-    wait_vm<NI>();      // and the first K tile
+    // The first K tile has landed too, and the fragments are read before the barrier behind which any
+    // wavefront may transfer the first V tile over them (one without rows of its own does so at once).
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(NI) : "memory");
   }
   // V (transposing read): in each group of 16 lanes, lanes 4r..4r+3 address 16 consecutive
   // halves of tile row r, and lane i of the group receives column i of that 4 x 16 block.
