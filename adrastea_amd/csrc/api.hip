@@ -140,17 +140,18 @@ void* scratch_on_current_device(hipError_t* err) {
 // and therefore no workspace argument.  Where a workspace pays (K split over workgroups; on request
 // the u8 matrix dequantised once) they take it from a pool that grows on demand.  A buffer has an
 // owner, (device, stream) -- launches on one stream run in order, launches on different streams may
-// overlap -- and an event recorded behind the last launches that used it.  A buffer changes hands
-// (a buffer its owner outgrew, or the least recently used one when all MAX_HELD entries are
-// taken) by making the new owner's stream wait for that event: no free and no allocation inside a
-// call beyond the first ones.  Memory goes back to the device only through
-// adr_release_held_workspace*, which wait for the event first.
+// overlap -- and an event behind the last launches that used it.  A buffer changes hands (a buffer its
+// owner outgrew, or the least recently used one when all MAX_HELD entries are taken) by making the
+// new owner's stream wait for that event: no synchronisation, no free and no allocation inside a call
+// beyond the first ones.  Memory goes back to the device only through adr_release_held_workspace*,
+// which wait for the last launches first.
 // An event costs the stream 3 us (a barrier packet and the flush behind it: a 41.5 us kernel launched
-// again and again takes 44.4 us with one behind each) and the host 1.4 us, so none is recorded behind a
-// use until it can be of use: while entries are free no buffer that has an owner changes hands, a
-// buffer is outgrown or released with its owner's stream at hand (recorded then), and only the pool
-// filling up asks for events of uses that are over -- of streams that may not exist any more.  That
-// waits for the device, once; from then on every use records its event.
+// again and again takes 44.4 us with one behind each) and the host 1.4 us.  So none is recorded behind
+// a use while one stream is the only owner of a buffer, as in most programs: there is nobody to hand it
+// to.  Such an entry is `pending` and keeps its owner until the event has been recorded after all:
+// at the owner's next use beside others, or when it outgrows or releases the buffer (its stream is
+// at hand then).  A stream that is gone without a release can so keep the one buffer it had alone, and no
+// call ever waits for work whose stream it cannot name.
 constexpr int MAX_HELD = 16;
 constexpr int64_t HELD_FLOOR = (int64_t)16 << 20;
 struct Held {
@@ -193,26 +194,10 @@ bool held_record(Held* h) {
   return !h->pending;
 }
 
-// Waits until no launch on the current device uses any buffer (see above).  In relaxed capture mode: it
-// must not disturb a capture that another stream of the process is in.
-bool held_wait_for_device(int dev) {
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  (void)hipThreadExchangeStreamCaptureMode(&mode);
-  const hipError_t e = hipDeviceSynchronize();
-  (void)hipThreadExchangeStreamCaptureMode(&mode);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
-  for (int i = 0; i < held_count; i++)
-    if (held[i].device == dev) held[i].pending = false;
-  return true;
-}
-
 // `stream` takes over entry h: everything the previous owner launched on the buffer is ordered
 // before whatever `stream` launches next.
 bool held_take_over(Held* h, hipStream_t stream) {
-  if (h->pending && !held_wait_for_device(h->device)) return false;
+  if (h->pending) return false;
   if (hipStreamWaitEvent(stream, h->last_use, 0) != hipSuccess) {
     (void)hipGetLastError();
     return false;
@@ -282,7 +267,7 @@ Held* held_buffer(hipStream_t stream, int64_t want) {
   // every entry is taken: the least recently used buffer of this device that is large enough
   Held* lru = nullptr;
   for (int i = 0; i < held_count; i++)
-    if (held[i].device == dev && held[i].bytes >= want && &held[i] != mine &&
+    if (held[i].device == dev && held[i].bytes >= want && &held[i] != mine && !held[i].pending &&
         (!lru || held[i].tick < lru->tick))
       lru = &held[i];
   if (lru && held_take_over(lru, stream)) {
@@ -296,7 +281,9 @@ Held* held_buffer(hipStream_t stream, int64_t want) {
 void held_used(Held* h) {
   h->tick = ++held_clock;
   h->pending = true;
-  if (held_count == MAX_HELD) held_record(h);
+  int owners = 0;
+  for (int i = 0; i < held_count; i++) owners += held[i].owned;
+  if (owners > 1) held_record(h);
 }
 
 // Frees entry i (waits for its last use first) and closes the gap.  held_mutex is held.  `alive`: its

@@ -10,9 +10,9 @@
  * with any other device current, every launching entry point returns ADR_EUNSUPPORTED_DEVICE
  * (the device's architecture, compute-unit and die counts are queried once per device and
  * cached).  Beside that cache the library keeps one piece of state: the pool of workspaces that
- * adr_matmul_f16, adr_matmul_nt_f16, adr_attention_f16 and (on request) adr_matmul_nt_fp16u8 draw from, grown on
- * demand and given back through adr_release_held_workspace* (adr_set_held_workspace_limit below;
- * 0 switches it off).
+ * adr_matmul_f16, adr_matmul_nt_f16, adr_attention_f16 and (on request) adr_matmul_nt_fp16u8 draw
+ * from, grown on demand and given back through adr_release_held_workspace*
+ * (adr_set_held_workspace_limit below; 0 switches it off).
  *
  * fp16 data is passed as uint16_t bit patterns (Rust `half::f16` is repr(transparent) u16).
  * All strides are in ELEMENTS.  `x` is the last tensor dimension, `y` the second to last,
@@ -154,16 +154,17 @@ int adr_matmul_f16_noalloc(adr_stream_t stream, uint16_t* output, const uint16_t
  * reference).  Those entry points keep the reference's argument tuples and so have no workspace
  * argument; where a workspace pays -- the products adr_matmul_f16_ws splits along K -- they take
  * one from a pool inside the library, and so does adr_attention_f16 where its query blocks are fewer
- * than the compute units and workgroups share their keys.  A buffer belongs to a (device, stream) pair: it is allocated
- * with hipMalloc at the first call on that stream that wants one (16 MiB doubling up to the limit).
- * When a stream wants more than its buffer holds it gets a larger one and the old buffer stays in
- * the pool for any stream that wants less; when all 16 entries of the pool are taken, a stream
- * without a buffer takes over the least recently used one that is large enough.  A buffer changes
- * hands by making the new owner's stream wait for an event behind the buffer's last use
- * (hipStreamWaitEvent).  Those events cost more than they order, so they are recorded only once all
- * 16 entries are taken; the first call that takes over a buffer used before that waits for the device.
- * Beyond that and the first allocations nothing is freed, allocated or synchronised inside a call,
- * and the pool never holds more than 16 buffers of at most the limit each.  Calls on one stream share a buffer and run in stream
+ * than the compute units and workgroups share their keys.  A buffer belongs to a (device, stream)
+ * pair: it is allocated with hipMalloc at the first call on that stream that wants one (16 MiB
+ * doubling up to the limit).  When a stream wants more than its buffer holds it gets a larger one
+ * and the old buffer stays in the pool for any stream that wants less; when all 16 entries of the
+ * pool are taken, a stream without a buffer takes over the least recently used one that is large
+ * enough.  A buffer changes hands by making the new owner's stream wait for an event behind the
+ * buffer's last use (hipStreamWaitEvent).  Such an event costs a call 2-3 us, so it is left out while
+ * one stream is the only owner of a buffer; a buffer used so is handed on only after its owner has
+ * used it beside others, outgrown it or released it.  Nothing is freed, allocated or synchronised
+ * inside a call beyond those first allocations, and the pool never holds more than 16 buffers of at
+ * most the limit each.  Calls on one stream share a buffer and run in stream
  * order; the pool is locked while a call that uses it launches, so any thread may call on any
  * stream.  No buffer is used or allocated -- the call runs exactly as with a limit of 0 -- while
  * the stream is being captured into a graph (the launches would tie the buffer to a graph that may
