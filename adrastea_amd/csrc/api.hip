@@ -187,6 +187,14 @@ bool held_allowed(hipStream_t stream) {
   return st == hipStreamCaptureStatusNone;
 }
 
+// While one of these lives, the calling thread's "unsafe" calls (allocating, freeing, waiting) leave alone
+// a capture in global mode that some stream of the process may be in: they touch no stream.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // Records the event behind the last use of an entry whose owner's stream is at hand.
 bool held_record(Held* h) {
   if (h->pending && hipEventRecord(h->last_use, h->stream) == hipSuccess) h->pending = false;
@@ -242,18 +250,17 @@ Held* held_buffer(hipStream_t stream, int64_t want) {
     int64_t size = HELD_FLOOR;
     while (size < want) size *= 2;
     if (size > limit) size = limit;
-    // (an allocation is an "unsafe" call for a capture in global mode that some other stream of the
-    // process may be in; it touches no stream, so it is made in relaxed mode)
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
     void* p = nullptr;
     hipEvent_t ev = nullptr;
-    hipError_t e = hipMalloc(&p, (size_t)size);
-    if (e == hipSuccess && p) {
-      e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-      if (e != hipSuccess) (void)hipFree(p);
+    hipError_t e;
+    {
+      RelaxedCapture relaxed;
+      e = hipMalloc(&p, (size_t)size);
+      if (e == hipSuccess && p) {
+        e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+        if (e != hipSuccess) (void)hipFree(p);
+      }
     }
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
     if (e != hipSuccess || !p) {
       (void)hipGetLastError();  // out of memory: the product runs without a workspace
       return declined();
@@ -286,22 +293,34 @@ void held_used(Held* h) {
   if (owners > 1) held_record(h);
 }
 
-// Frees entry i (waits for its last use first) and closes the gap.  held_mutex is held.  `alive`: its
+// Waits until the last launches that used entry h are over; after an error they may not be.  `alive`: its
 // owner's stream certainly exists.
-void held_free(int i, bool alive) {
-  if (!(alive && held_record(&held[i])) && held[i].pending) {
-    int dev = held[i].device;
-    (void)hipGetDevice(&dev);
-    if (dev != held[i].device) (void)hipSetDevice(held[i].device);
-    (void)hipDeviceSynchronize();
-    if (dev != held[i].device) (void)hipSetDevice(dev);
+hipError_t held_wait(Held* h, bool alive) {
+  if (alive) held_record(h);
+  if (!h->pending) return hipEventSynchronize(h->last_use);
+  int dev = -1;
+  if (hipError_t e = hipGetDevice(&dev)) return e;
+  if (dev != h->device)
+    if (hipError_t e = hipSetDevice(h->device)) return e;
+  const hipError_t e = hipDeviceSynchronize();
+  if (dev != h->device) (void)hipSetDevice(dev);
+  return e;
+}
+
+// Frees entry i once its last use is over and closes the gap; an entry that cannot be waited for
+// stays as it is.  held_mutex is held.
+hipError_t held_free(int i, bool alive) {
+  RelaxedCapture relaxed;
+  hipError_t e = held_wait(&held[i], alive);
+  if (e == hipSuccess) e = hipFree(held[i].ptr);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return e;
   }
-  (void)hipEventSynchronize(held[i].last_use);
   (void)hipEventDestroy(held[i].last_use);
-  (void)hipFree(held[i].ptr);
-  (void)hipGetLastError();
   held_total -= held[i].bytes;
   held[i] = held[--held_count];
+  return hipSuccess;
 }
 
 // run_matmul for the entry points without a workspace argument.
@@ -381,16 +400,27 @@ int64_t adr_held_workspace_declined(void) { return held_declined.load(std::memor
 int adr_release_held_workspace(adr_stream_t stream) {
   int dev = -1;
   if (hipError_t e = hipGetDevice(&dev)) return (int)e;
+  // Not while the stream is being captured: an event recorded now would be a node of the graph and say
+  // nothing of the launches before it, and any wait for them, or for the device, would end the capture.
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  const hipError_t known = hipStreamIsCapturing((hipStream_t)stream, &st);
+  if (known != hipSuccess) (void)hipGetLastError();
+  if (known == hipErrorStreamCaptureImplicit) return (int)known;  // (the null stream beside a capture)
+  if (st != hipStreamCaptureStatusNone) return (int)hipErrorStreamCaptureUnsupported;
   std::lock_guard<std::mutex> lock(held_mutex);
+  int rc = ADR_OK;
   for (int i = held_count - 1; i >= 0; i--)
-    if (held[i].device == dev && (!held[i].owned || held[i].stream == (hipStream_t)stream)) held_free(i, held[i].owned);
-  return ADR_OK;
+    if (held[i].device == dev && (!held[i].owned || held[i].stream == (hipStream_t)stream))
+      if (hipError_t e = held_free(i, held[i].owned && known == hipSuccess)) rc = (int)e;
+  return rc;
 }
 
 int adr_release_held_workspace_all(void) {
   std::lock_guard<std::mutex> lock(held_mutex);
-  while (held_count > 0) held_free(held_count - 1, false);
-  return ADR_OK;
+  int rc = ADR_OK;
+  for (int i = held_count - 1; i >= 0; i--)
+    if (hipError_t e = held_free(i, false)) rc = (int)e;
+  return rc;
 }
 
 int adr_set_u8_dequantise_first(int enabled) {

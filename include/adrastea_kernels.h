@@ -180,9 +180,11 @@ int adr_matmul_f16_noalloc(adr_stream_t stream, uint16_t* output, const uint16_t
  * released).  adr_held_workspace_bytes: bytes the pool holds now.
  * adr_release_held_workspace(stream): waits for what `stream` has been given so far and frees, on the
  * current device, the buffers it owns and those no stream owns any more; call it before destroying
- * a stream.  adr_release_held_workspace_all: frees every buffer on every device, waiting for the
- * devices.  (hipFree itself may wait for other work on the device: these two are not for the hot
- * path.)  Later calls allocate afresh.
+ * a stream.  Not while that stream is being captured (hipErrorStreamCaptureUnsupported, and nothing is
+ * freed): waiting would end the capture.  adr_release_held_workspace_all: frees every buffer on every
+ * device, waiting for the devices where it must; not while anything on them is being captured.  A
+ * buffer that cannot be waited for is kept, and the error returned.  (hipFree itself may wait for
+ * other work on the device: these two are not for the hot path.)  Later calls allocate afresh.
  * Callers that must not allocate at all use adr_matmul_f16_noalloc or the _ws forms, which never
  * touch the pool.
  *

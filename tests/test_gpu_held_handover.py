@@ -1,6 +1,8 @@
 """A buffer of the library's workspace pool that changes hands while its last owner's launches are still
 running: whoever takes it over runs behind them (the two with operands and results of their own), and
 the call that takes it over returns at once, whatever the device is doing."""
+import contextlib
+
 import pytest
 import torch
 
@@ -193,3 +195,64 @@ def test_a_stream_s_buffer_serves_products_and_attention_in_turn(pool):
     want = (torch.softmax(scores, 1) * v.double()).sum(1, keepdim=True)
     # fp16 output and probabilities: 2^-11 of the largest value each, doubled
     assert ((outs[8].double() - want).abs().max() / want.abs().max()).item() <= 2e-3
+
+
+@contextlib.contextmanager
+def captured(stream):
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        graph.capture_begin()
+        try:
+            yield graph
+        finally:
+            graph.capture_end()
+
+
+def replays(graph, a):
+    for i in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert (a == 2 + i).all()
+
+
+@pytest.mark.parametrize("alone", [True, False])
+def test_release_on_a_stream_that_is_being_captured(pool, alone):
+    """The buffer cannot be waited for then: the call says so, the buffer stays, and the capture goes on."""
+    load, s = Load(), streams(2)
+    product = Product(pool, SMALL, 60)
+    a = torch.ones(256, dtype=torch.float16, device="cuda")
+    if not alone:
+        product.run(s[1])
+    load.put(s[0])
+    product.run(s[0])                                 # (alone in the pool this use leaves no event)
+    before = pool.adr_held_workspace_bytes()
+    with captured(s[0]) as graph:
+        rc = pool.adr_release_held_workspace(s[0].cuda_stream)
+        held = pool.adr_held_workspace_bytes()
+        a.add_(1)
+    assert rc > 0 and held == before
+    replays(graph, a)
+    assert product.right()
+    assert pool.adr_release_held_workspace(s[0].cuda_stream) == 0
+    assert pool.adr_held_workspace_bytes() == before - 16 * MIB
+
+
+@pytest.mark.parametrize("alone", [True, False])
+def test_release_while_another_stream_is_being_captured(pool, alone):
+    load, s = Load(), streams(3)
+    product = Product(pool, SMALL, 61)
+    a = torch.ones(256, dtype=torch.float16, device="cuda")
+    if not alone:
+        product.run(s[2])
+    load.put(s[0])
+    product.run(s[0])
+    done = mark(s[0])
+    before = pool.adr_held_workspace_bytes()
+    with captured(s[1]) as graph:
+        rc = pool.adr_release_held_workspace(s[0].cuda_stream)
+        held = pool.adr_held_workspace_bytes()
+        a.add_(1)
+    over = done.query()                               # (40 ms of work are not over by chance)
+    assert rc == 0 and held == before - 16 * MIB and over
+    assert product.right()
+    replays(graph, a)
