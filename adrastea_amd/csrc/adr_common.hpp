@@ -332,13 +332,25 @@ hipError_t launch_microbench_read(hipStream_t stream, const void* p, int64_t byt
                                   uint32_t* sink);
 hipError_t launch_error_stats(hipStream_t stream, float* out, const void* lhs, const void* rhs,
                               int64_t length, int64_t sl, int64_t sr, bool f32);
-hipError_t launch_attention(hipStream_t stream, half_t* out, const half_t* q, const half_t* k,
-                            const half_t* v, int heads, int m, int n, int d, int so_y, int so_z,
-                            int sq_y, int sq_z, int sk_y, int sk_z, int sv_y, int sv_z, float scale,
-                            float temp, uint32_t mask, void* workspace, int64_t workspace_bytes);
-// Scratch bytes that launch would use when at most `avail` can be had (0: no keys are split).
-int64_t attention_workspace_bytes(int heads, int m, int n, int d, int sq_y, int sk_y, int sv_y, uint32_t mask,
-                                  int64_t avail);
+// Fused attention (attention.hip): the shape of a call, and which kernel runs it on a device of `cus`
+// compute units.  splits > 1: that many workgroups share the keys of a query block, and their parts
+// pass through workspace_bytes bytes of scratch, of which at most `avail` may be asked for.
+struct AttentionShape {
+  int heads, m, n, d;  // query rows, key/value rows, head dimension
+  int so_y, so_z, sq_y, sq_z, sk_y, sk_z, sv_y, sv_z;
+  uint32_t mask;
+};
+struct AttentionPlan {
+  bool rows;   // attention_rows_kernel
+  bool wide;   // 64-bit addresses (attention_fwd_kernel)
+  int groups;  // of four wavefronts (attention_fwd_kernel)
+  int splits;
+  int cus;
+  int64_t workspace_bytes;
+};
+AttentionPlan attention_plan(const AttentionShape& t, int cus, int64_t avail);
+hipError_t launch_attention(hipStream_t stream, half_t* out, const half_t* q, const half_t* k, const half_t* v,
+                            const AttentionShape& t, const AttentionPlan& p, float scale, float temp, void* workspace);
 hipError_t launch_softmax_rows(hipStream_t stream, half_t* out, const half_t* in, int64_t rows,
                                int w, float temp);
 

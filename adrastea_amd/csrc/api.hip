@@ -759,26 +759,28 @@ int adr_attention_f16(adr_stream_t stream, uint16_t* output, const uint16_t* que
     return ADR_EUNSUPPORTED_LAYOUT;
   if (!(scale > 0.0f) || !(temp > 0.0f)) return ADR_EUNSUPPORTED_LAYOUT;
   // largest element offsets stay within int64 trivially; rows are addressed with 64-bit products
-  if (int rc = check_device()) return rc;
-  auto launch = [&](void* workspace, int64_t bytes) {
-    return (int)launch_attention((hipStream_t)stream, (half_t*)output, (const half_t*)query,
-                                 (const half_t*)key, (const half_t*)value, heads, m, n, d,
-                                 stride_oy, stride_oz, stride_qy, stride_qz, stride_ky, stride_kz,
-                                 stride_vy, stride_vz, scale, temp, mask, workspace, bytes);
+  const DeviceInfo dev = device_info();
+  if (dev.status) return dev.status;
+  const AttentionShape t = {heads, m, n, d, stride_oy, stride_oz, stride_qy, stride_qz,
+                            stride_ky, stride_kz, stride_vy, stride_vz, mask};
+  auto launch = [&](const AttentionPlan& plan, void* workspace) {
+    return (int)launch_attention((hipStream_t)stream, (half_t*)output, (const half_t*)query, (const half_t*)key,
+                                 (const half_t*)value, t, plan, scale, temp, workspace);
   };
   // (fewer query blocks than compute units: the keys of a block are shared by several workgroups,
   // whose parts pass through a buffer of the pool)
   const int64_t limit = held_limit.load(std::memory_order_relaxed);
-  const int64_t need = limit > 0 ? attention_workspace_bytes(heads, m, n, d, stride_qy, stride_ky, stride_vy, mask, limit) : 0;
-  if (need > 0 && held_allowed((hipStream_t)stream)) {
+  const AttentionPlan plan = attention_plan(t, dev.cus, limit);
+  if (plan.workspace_bytes == 0) return launch(plan, nullptr);
+  if (held_allowed((hipStream_t)stream)) {
     std::lock_guard<std::mutex> lock(held_mutex);
-    if (Held* h = held_buffer((hipStream_t)stream, need)) {
-      const int rc = launch(h->ptr, h->bytes);
+    if (Held* h = held_buffer((hipStream_t)stream, plan.workspace_bytes)) {
+      const int rc = launch(plan, h->ptr);
       held_used(h);
       return rc;
     }
   }
-  return launch(nullptr, 0);
+  return launch(attention_plan(t, dev.cus, 0), nullptr);
 }
 
 static int error_stats_common(adr_stream_t stream, adr_tensor_desc output, adr_tensor_desc lhs,

@@ -879,47 +879,37 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(AttnArgs a) {
 
 }  // namespace
 
-// Which kernel runs, and how many workgroups share the keys of one query block.  Fewer query blocks than
-// compute units leave units idle, so the keys are then shared: by two groups of wavefronts inside the
-// workgroup, or by several workgroups, whose parts a second launch adds up.
-struct AttnPlan {
-  bool rows;   // attention_rows_kernel
-  int groups;  // of four wavefronts (attention_fwd_kernel)
-  int splits;
-};
-
 // The buffer transfers count the bytes of a head, and of two tiles, in 31 bits, and take rows to be no
 // closer than they are long.
-static bool attention_wide(int m, int n, int d, int sq_y, int sk_y, int sv_y) {
-  const int64_t far = sk_y > sv_y ? sk_y : sv_y;
-  return sq_y < d || sk_y < d || sv_y < d || far >= 1 << 22 || n * far >= (int64_t)1 << 30 ||
-         (int64_t)m * sq_y >= (int64_t)1 << 30;
+static bool attention_wide(const AttentionShape& t) {
+  const int64_t far = t.sk_y > t.sv_y ? t.sk_y : t.sv_y;
+  return t.sq_y < t.d || t.sk_y < t.d || t.sv_y < t.d || far >= 1 << 22 || t.n * far >= (int64_t)1 << 30 ||
+         (int64_t)t.m * t.sq_y >= (int64_t)1 << 30;
 }
 
-static int64_t attention_part_bytes(int heads, int m, int d) { return (int64_t)heads * m * (d * 4 + 8); }
-
-static AttnPlan attention_plan(int heads, int m, int n, int d, int sq_y, int sk_y, int sv_y, uint32_t mask,
-                               int64_t avail) {
-  AttnPlan p;
-  const bool wide = attention_wide(m, n, d, sq_y, sk_y, sv_y);
-  p.rows = m <= 16 && mask == ADR_MASK_NONE && !wide;
-  const int cus = device_info_for_plan().cus;
-  const int64_t part = attention_part_bytes(heads, m, d), blocks = (int64_t)heads * ((m + BM - 1) / BM);
+// Fewer query blocks than compute units leave units idle, so the keys are then shared: by two groups of
+// wavefronts inside the workgroup, or by several workgroups, whose parts a second launch adds up.
+AttentionPlan attention_plan(const AttentionShape& t, int cus, int64_t avail) {
+  AttentionPlan p;
+  p.cus = cus;
+  p.wide = attention_wide(t);
+  p.rows = t.m <= 16 && t.mask == ADR_MASK_NONE && !p.wide;
+  const int64_t part = (int64_t)t.heads * t.m * (t.d * 4 + 8), blocks = (int64_t)t.heads * ((t.m + BM - 1) / BM);
   // One workgroup per compute unit at most: two groups take 9.5 us per 1000 keys where one takes 14
   // (two such workgroups per unit take as long as one of two groups), and half a microsecond to merge,
   // which pays from six tiles on (20 heads of 64, 1500 x 1500: 25.3 -> 21.2 us, 12 x 1000 causal
   // 15.3 -> 12.7; 12 x 256 6.2 -> 6.3).
-  p.groups = !p.rows && !wide && blocks <= cus && n > 5 * BN ? 2 : 1;
+  p.groups = !p.rows && !p.wide && blocks <= cus && t.n > 5 * BN ? 2 : 1;
   p.splits = 1;
   // Times beyond what every launch takes, in us, fitted to 40 shapes of 12-40 heads, 1-448 query rows
   // and 64-8192 keys with every number of parts: the rows kernel reads 69 GB/s per compute unit; parts
   // cost a launch (and the host its issue: more than a short read takes) and their way through memory.
   double best = 1e30;
-  for (int s = 1; s <= MAX_SPLITS && s * 64 <= n + 63 && (s == 1 || s * part <= avail); s++) {
-    const double keys = (double)n / s;
+  for (int s = 1; s <= MAX_SPLITS && s * 64 <= t.n + 63 && (s == 1 || s * part <= avail); s++) {
+    const double keys = (double)t.n / s;
     double us;
     if (p.rows) {
-      us = ceil((double)heads * s / cus) * keys * d * (4.0 / 69e3);
+      us = ceil((double)t.heads * s / cus) * keys * t.d * (4.0 / 69e3);
       if (s > 1) us += 4.0;
     } else if (s == 1 && p.groups == 2) {
       us = keys * 0.0095 + 0.5;
@@ -931,20 +921,15 @@ static AttnPlan attention_plan(int heads, int m, int n, int d, int sq_y, int sk_
     if (us < best * 0.97) best = us, p.splits = s;
   }
   if (p.splits > 1) p.groups = 1;
+  p.workspace_bytes = p.splits > 1 ? p.splits * part : 0;
   return p;
 }
 
-int64_t attention_workspace_bytes(int heads, int m, int n, int d, int sq_y, int sk_y, int sv_y, uint32_t mask,
-                                  int64_t avail) {
-  const AttnPlan p = attention_plan(heads, m, n, d, sq_y, sk_y, sv_y, mask, avail);
-  return p.splits > 1 ? p.splits * attention_part_bytes(heads, m, d) : 0;
-}
-
 template <int HD>
-static void attention_launches(hipStream_t stream, const AttnArgs& a, const AttnPlan& p, bool wide) {
+static void attention_launches(hipStream_t stream, const AttnArgs& a, const AttentionPlan& p) {
   const dim3 block(256), grid((unsigned)(a.heads * (p.rows ? 1 : a.qblocks) * a.splits));
   if (p.rows) hipLaunchKernelGGL(attention_rows_kernel<HD>, grid, block, 0, stream, a);
-  else if (wide) hipLaunchKernelGGL(HIP_KERNEL_NAME(attention_fwd_kernel<HD, 1, true>), grid, block, 0, stream, a);
+  else if (p.wide) hipLaunchKernelGGL(HIP_KERNEL_NAME(attention_fwd_kernel<HD, 1, true>), grid, block, 0, stream, a);
   else if (p.groups == 2) hipLaunchKernelGGL(HIP_KERNEL_NAME(attention_fwd_kernel<HD, 2, false>), grid, dim3(512), 0, stream, a);
   else hipLaunchKernelGGL(HIP_KERNEL_NAME(attention_fwd_kernel<HD, 1, false>), grid, block, 0, stream, a);
   if (a.splits > 1) {
@@ -953,29 +938,25 @@ static void attention_launches(hipStream_t stream, const AttnArgs& a, const Attn
   }
 }
 
-hipError_t launch_attention(hipStream_t stream, half_t* out, const half_t* q, const half_t* k,
-                            const half_t* v, int heads, int m, int n, int d, int so_y, int so_z,
-                            int sq_y, int sq_z, int sk_y, int sk_z, int sv_y, int sv_z, float scale,
-                            float temp, uint32_t mask, void* workspace, int64_t workspace_bytes) {
-  const AttnPlan p = attention_plan(heads, m, n, d, sq_y, sk_y, sv_y, mask, workspace ? workspace_bytes : 0);
+hipError_t launch_attention(hipStream_t stream, half_t* out, const half_t* q, const half_t* k, const half_t* v,
+                            const AttentionShape& t, const AttentionPlan& p, float scale, float temp, void* workspace) {
   AttnArgs a;
   a.out = out; a.q = q; a.k = k; a.v = v;
-  a.heads = heads; a.m = m; a.n = n;
-  a.so_y = so_y; a.so_z = so_z; a.sq_y = sq_y; a.sq_z = sq_z;
-  a.sk_y = sk_y; a.sk_z = sk_z; a.sv_y = sv_y; a.sv_z = sv_z;
+  a.heads = t.heads; a.m = t.m; a.n = t.n;
+  a.so_y = t.so_y; a.so_z = t.so_z; a.sq_y = t.sq_y; a.sq_z = t.sq_z;
+  a.sk_y = t.sk_y; a.sk_z = t.sk_z; a.sv_y = t.sv_y; a.sv_z = t.sv_z;
   // the three-call sequence multiplies by the scale rounded to fp16 (matmul.cu:60-74)
   a.c = (float)(half_t)scale * 1.44269504088896340736f / temp;
-  a.mask = mask;
+  a.mask = t.mask;
   a.splits = p.splits;
-  const int64_t rows = (int64_t)heads * m;
+  const int64_t rows = (int64_t)t.heads * t.m;
   a.part_o = (float*)workspace;
-  a.part_ml = (float2*)((float*)workspace + (a.splits > 1 ? a.splits * rows * d : 0));
-  a.qblocks = (m + BM - 1) / BM;
-  a.upper = (int64_t)heads * a.qblocks * a.splits <= 2 * device_info().cus ? (a.qblocks + 1) / 2 : a.qblocks;
+  a.part_ml = (float2*)((float*)workspace + (a.splits > 1 ? a.splits * rows * t.d : 0));
+  a.qblocks = (t.m + BM - 1) / BM;
+  a.upper = (int64_t)t.heads * a.qblocks * a.splits <= 2 * p.cus ? (a.qblocks + 1) / 2 : a.qblocks;
   if (rows * a.splits > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-  const bool wide = attention_wide(m, n, d, sq_y, sk_y, sv_y);
-  if (d == 128) attention_launches<128>(stream, a, p, wide);
-  else attention_launches<64>(stream, a, p, wide);
+  if (t.d == 128) attention_launches<128>(stream, a, p);
+  else attention_launches<64>(stream, a, p);
   return hipGetLastError();
 }
 
