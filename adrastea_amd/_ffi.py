@@ -18,7 +18,8 @@ SYMBOLS = (
     "adr_matmul_nt_fp16u8", "adr_matmul_nt_fp16u8_ws", "adr_matmul_nt_fp16u8_workspace_bytes",
     "adr_dequantize_absmax_u8", "adr_quantize_absmax_u8",
     "adr_dequantize_absmax_uint8", "adr_quantize_absmax_uint8", "adr_matmul_f16_plan",
-    "adr_matmul_nt_fp16u8_plan", "adr_softmax_rows", "adr_error_stats_f16", "adr_error_stats_f32", "adr_attention_f16", "adr_embed_uint8",
+    "adr_matmul_nt_fp16u8_plan", "adr_softmax_rows", "adr_error_stats_f16", "adr_error_stats_f32", "adr_attention_f16",
+    "adr_attention_f16_ws", "adr_attention_f16_workspace_bytes", "adr_embed_uint8",
     "adr_debug_knob", "adr_microbench_empty", "adr_microbench_mfma_f16", "adr_microbench_stream_read",
     "adr_strerror", "adr_abi_version",
 )
@@ -93,6 +94,8 @@ def lib():
     L.adr_error_stats_f16.argtypes = [vp, TensorDesc, TensorDesc, TensorDesc]
     L.adr_error_stats_f32.argtypes = [vp, TensorDesc, TensorDesc, TensorDesc]
     L.adr_attention_f16.argtypes = [vp, vp, vp, vp, vp] + [i32] * 16 + [f32, f32, u32]
+    L.adr_attention_f16_ws.argtypes = L.adr_attention_f16.argtypes + [vp, C.c_int64]
+    L.adr_attention_f16_workspace_bytes.argtypes = [i32] * 16 + [u32]
     L.adr_embed_uint8.argtypes = [vp, i32, i32, vp, vp, vp, vp, i32]
     L.adr_strerror.argtypes = [C.c_int]
     L.adr_strerror.restype = C.c_char_p
@@ -101,6 +104,7 @@ def lib():
         if name not in ("adr_strerror",):
             getattr(L, name).restype = C.c_int
     L.adr_matmul_f16_workspace_bytes.restype = C.c_int64
+    L.adr_attention_f16_workspace_bytes.restype = C.c_int64
     L.adr_held_workspace_limit.restype = C.c_int64
     L.adr_held_workspace_bytes.restype = C.c_int64
     L.adr_held_workspace_declined.restype = C.c_int64

@@ -736,41 +736,49 @@ int adr_softmax_rows(adr_stream_t stream, uint16_t* output, const uint16_t* inpu
                                   (int64_t)heads * h, w, temp);
 }
 
-int adr_attention_f16(adr_stream_t stream, uint16_t* output, const uint16_t* query,
-                      const uint16_t* key, const uint16_t* value, int32_t heads, int32_t m,
-                      int32_t n, int32_t d, int32_t stride_ox, int32_t stride_oy,
-                      int32_t stride_oz, int32_t stride_qx, int32_t stride_qy, int32_t stride_qz,
-                      int32_t stride_kx, int32_t stride_ky, int32_t stride_kz, int32_t stride_vx,
-                      int32_t stride_vy, int32_t stride_vz, float scale, float temp,
-                      uint32_t mask) {
+// What the attention entry points cover; *nothing_to_do where the call has no output elements.
+static int validate_attention(int32_t heads, int32_t m, int32_t n, int32_t d, const int32_t (&x)[4],
+                              const int32_t (&yz)[8], uint32_t mask, bool* nothing_to_do) {
+  *nothing_to_do = false;
   if (heads < 0 || m < 0 || n < 0 || d < 0) return ADR_EINVAL_SHAPE;
   if (mask > ADR_MASK_CAUSAL) return ADR_EINVAL_ENUM;
-  if (heads == 0 || m == 0 || d == 0) return ADR_OK;
+  if (heads == 0 || m == 0 || d == 0) {
+    *nothing_to_do = true;
+    return ADR_OK;
+  }
   if (n == 0) return ADR_EINVAL_SHAPE;
-  if (!output || !query || !key || !value) return ADR_ENULL;
   if (d != 64 && d != 128) return ADR_EUNSUPPORTED_LAYOUT;
-  if (stride_ox != 1 || stride_qx != 1 || stride_kx != 1 || stride_vx != 1)
-    return ADR_EUNSUPPORTED_LAYOUT;
-  const int32_t st[8] = {stride_oy, stride_oz, stride_qy, stride_qz,
-                         stride_ky, stride_kz, stride_vy, stride_vz};
+  for (int i = 0; i < 4; i++)
+    if (x[i] != 1) return ADR_EUNSUPPORTED_LAYOUT;
   for (int i = 0; i < 8; i++)
-    if (st[i] < 0 || st[i] % 8 != 0) return ADR_EUNSUPPORTED_LAYOUT;
+    if (yz[i] < 0 || yz[i] % 8 != 0) return ADR_EUNSUPPORTED_LAYOUT;
+  return ADR_OK;
+}
+
+static int attention(adr_stream_t stream, uint16_t* output, const uint16_t* query, const uint16_t* key,
+                     const uint16_t* value, int32_t heads, int32_t m, int32_t n, int32_t d, const int32_t (&x)[4],
+                     const int32_t (&yz)[8], float scale, float temp, uint32_t mask, bool held, void* workspace,
+                     int64_t workspace_bytes) {
+  bool nothing;
+  const int covered = validate_attention(heads, m, n, d, x, yz, mask, &nothing);
+  if ((covered && covered != ADR_EUNSUPPORTED_LAYOUT) || nothing) return covered;
+  if (!output || !query || !key || !value) return ADR_ENULL;
+  if (covered) return covered;
   if (((uintptr_t)output | (uintptr_t)query | (uintptr_t)key | (uintptr_t)value) % 16 != 0)
     return ADR_EUNSUPPORTED_LAYOUT;
   if (!(scale > 0.0f) || !(temp > 0.0f)) return ADR_EUNSUPPORTED_LAYOUT;
   // largest element offsets stay within int64 trivially; rows are addressed with 64-bit products
   const DeviceInfo dev = device_info();
   if (dev.status) return dev.status;
-  const AttentionShape t = {heads, m, n, d, stride_oy, stride_oz, stride_qy, stride_qz,
-                            stride_ky, stride_kz, stride_vy, stride_vz, mask};
-  auto launch = [&](const AttentionPlan& plan, void* workspace) {
+  const AttentionShape t = {heads, m, n, d, yz[0], yz[1], yz[2], yz[3], yz[4], yz[5], yz[6], yz[7], mask};
+  auto launch = [&](const AttentionPlan& plan, void* scratch) {
     return (int)launch_attention((hipStream_t)stream, (half_t*)output, (const half_t*)query, (const half_t*)key,
-                                 (const half_t*)value, t, plan, scale, temp, workspace);
+                                 (const half_t*)value, t, plan, scale, temp, scratch);
   };
   // (fewer query blocks than compute units: the keys of a block are shared by several workgroups,
-  // whose parts pass through a buffer of the pool)
-  const int64_t limit = held_limit.load(std::memory_order_relaxed);
-  const AttentionPlan plan = attention_plan(t, dev.cus, limit);
+  // whose parts pass through the caller's workspace or a buffer of the pool)
+  if (!held) return launch(attention_plan(t, dev.cus, workspace_bytes), workspace);
+  const AttentionPlan plan = attention_plan(t, dev.cus, held_limit.load(std::memory_order_relaxed));
   if (plan.workspace_bytes == 0) return launch(plan, nullptr);
   if (held_allowed((hipStream_t)stream)) {
     std::lock_guard<std::mutex> lock(held_mutex);
@@ -781,6 +789,44 @@ int adr_attention_f16(adr_stream_t stream, uint16_t* output, const uint16_t* que
     }
   }
   return launch(attention_plan(t, dev.cus, 0), nullptr);
+}
+
+int adr_attention_f16(adr_stream_t stream, uint16_t* output, const uint16_t* query,
+                      const uint16_t* key, const uint16_t* value, int32_t heads, int32_t m,
+                      int32_t n, int32_t d, int32_t stride_ox, int32_t stride_oy,
+                      int32_t stride_oz, int32_t stride_qx, int32_t stride_qy, int32_t stride_qz,
+                      int32_t stride_kx, int32_t stride_ky, int32_t stride_kz, int32_t stride_vx,
+                      int32_t stride_vy, int32_t stride_vz, float scale, float temp,
+                      uint32_t mask) {
+  return attention(stream, output, query, key, value, heads, m, n, d, {stride_ox, stride_qx, stride_kx, stride_vx},
+                   {stride_oy, stride_oz, stride_qy, stride_qz, stride_ky, stride_kz, stride_vy, stride_vz}, scale, temp,
+                   mask, true, nullptr, 0);
+}
+
+int adr_attention_f16_ws(adr_stream_t stream, uint16_t* output, const uint16_t* query,
+                         const uint16_t* key, const uint16_t* value, int32_t heads, int32_t m,
+                         int32_t n, int32_t d, int32_t stride_ox, int32_t stride_oy,
+                         int32_t stride_oz, int32_t stride_qx, int32_t stride_qy, int32_t stride_qz,
+                         int32_t stride_kx, int32_t stride_ky, int32_t stride_kz, int32_t stride_vx,
+                         int32_t stride_vy, int32_t stride_vz, float scale, float temp,
+                         uint32_t mask, void* workspace, int64_t workspace_bytes) {
+  if (workspace_bytes < 0 || (workspace_bytes > 0 && !workspace)) return ADR_ENULL;
+  if ((uintptr_t)workspace % 16 != 0) return ADR_EINVAL_SHAPE;
+  return attention(stream, output, query, key, value, heads, m, n, d, {stride_ox, stride_qx, stride_kx, stride_vx},
+                   {stride_oy, stride_oz, stride_qy, stride_qz, stride_ky, stride_kz, stride_vy, stride_vz}, scale, temp,
+                   mask, false, workspace, workspace_bytes);
+}
+
+int64_t adr_attention_f16_workspace_bytes(int32_t heads, int32_t m, int32_t n, int32_t d, int32_t stride_ox,
+                                          int32_t stride_oy, int32_t stride_oz, int32_t stride_qx, int32_t stride_qy,
+                                          int32_t stride_qz, int32_t stride_kx, int32_t stride_ky, int32_t stride_kz,
+                                          int32_t stride_vx, int32_t stride_vy, int32_t stride_vz, uint32_t mask) {
+  const int32_t yz[8] = {stride_oy, stride_oz, stride_qy, stride_qz, stride_ky, stride_kz, stride_vy, stride_vz};
+  bool nothing;
+  if (int rc = validate_attention(heads, m, n, d, {stride_ox, stride_qx, stride_kx, stride_vx}, yz, mask, &nothing)) return rc;
+  if (nothing) return 0;
+  const AttentionShape t = {heads, m, n, d, yz[0], yz[1], yz[2], yz[3], yz[4], yz[5], yz[6], yz[7], mask};
+  return attention_plan(t, device_info_for_plan().cus, INT64_MAX).workspace_bytes;
 }
 
 static int error_stats_common(adr_stream_t stream, adr_tensor_desc output, adr_tensor_desc lhs,

@@ -121,7 +121,7 @@ class GpuKernels : public CommonKernels {
  public:
   // `workspace`: optional device buffer (16-byte aligned) the caller owns for as long as this
   // object lives; with it, products with few output tiles and a long K are split over K
-  // (adr_matmul_f16_ws).  Calls on one object must not overlap in time when it is set.
+  // (adr_matmul_f16_ws) and the keys of few query rows shared (adr_attention_f16_ws).  Calls on one object must not overlap in time when it is set.
   explicit GpuKernels(adr_stream_t stream = nullptr, void* workspace = nullptr, int64_t workspace_bytes = 0)
       : stream_(stream), workspace_(workspace), workspace_bytes_(workspace ? workspace_bytes : 0) {}
   void matmul_f16(TensorView<f16>& o, const TensorView<const f16>& l, const TensorView<const f16>& r,
@@ -156,12 +156,15 @@ class GpuKernels : public CommonKernels {
         (rank == 3 && ((int32_t)o.size(-3) != heads || (int32_t)k.size(-3) != heads || (int32_t)v.size(-3) != heads)))
       throw std::logic_error("attention_f16: shape mismatch");
     auto z = [&](const TensorLayout& l) { return rank == 3 ? (int32_t)l.stride(-3) : 0; };
-    int rc = adr_attention_f16(stream_, o.ptr, q.ptr, k.ptr, v.ptr, heads, m, n, d,
-                               (int32_t)o.layout.stride(-1), (int32_t)o.layout.stride(-2), z(o.layout),
-                               (int32_t)q.layout.stride(-1), (int32_t)q.layout.stride(-2), z(q.layout),
-                               (int32_t)k.layout.stride(-1), (int32_t)k.layout.stride(-2), z(k.layout),
-                               (int32_t)v.layout.stride(-1), (int32_t)v.layout.stride(-2), z(v.layout),
-                               scale, temperature, (uint32_t)mask);
+    auto call = [&](auto fn, auto... workspace) {
+      return fn(stream_, o.ptr, q.ptr, k.ptr, v.ptr, heads, m, n, d,
+                (int32_t)o.layout.stride(-1), (int32_t)o.layout.stride(-2), z(o.layout),
+                (int32_t)q.layout.stride(-1), (int32_t)q.layout.stride(-2), z(q.layout),
+                (int32_t)k.layout.stride(-1), (int32_t)k.layout.stride(-2), z(k.layout),
+                (int32_t)v.layout.stride(-1), (int32_t)v.layout.stride(-2), z(v.layout),
+                scale, temperature, (uint32_t)mask, workspace...);
+    };
+    int rc = workspace_bytes_ > 0 ? call(adr_attention_f16_ws, workspace_, workspace_bytes_) : call(adr_attention_f16);
     if (rc) throw AdrasteaError(rc, "attention_f16");
   }
   // kernels.rs:717-751: both operands flattened with shape_cast(&[-1]); equal lengths

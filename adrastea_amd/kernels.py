@@ -189,8 +189,9 @@ class GpuKernels(CommonKernels):
     `workspace_bytes` > 0 gives the instance a scratch buffer of that size, owned like any other
     tensor of the host (in the reference: one more GpuBuffer held by GpuKernels); matmul_f16 then
     goes through adr_matmul_f16_ws, which may split K over workgroups for products with few
-    output tiles and a long K.  The buffer carries nothing between calls; one instance must not
-    be used from streams that run concurrently.  Without it (the default) the library takes such
+    output tiles and a long K, and attention_f16 through adr_attention_f16_ws, which may share keys
+    over workgroups for few query rows.  The buffer carries nothing between calls; one instance must
+    not be used from streams that run concurrently.  Without it (the default) the library takes such
     a buffer from its own per-stream cache (set_held_workspace_limit)."""
 
     def __init__(self, workspace_bytes: int = 0):
@@ -236,7 +237,7 @@ class GpuKernels(CommonKernels):
     def attention_f16(self, output, query, key, value, scale: float, temperature: float = 1.0,
                       mask: int = MatmulMask.NONE):
         """The three calls of llama.rs:541-554 (QK^T with Scale and the mask, softmax_rows_inplace,
-        P.V) as one launch that keeps the scores out of memory.  `query`/`output` are
+        P.V) as one call that keeps the scores out of memory.  `query`/`output` are
         [heads, m, d] views, `key`/`value` [heads, n, d] views (rank 2 = one head).  Raises
         AdrasteaError with code ADR_EUNSUPPORTED_LAYOUT for head dimensions or strides the fused
         kernel does not cover; the three-call sequence remains available for those."""
@@ -252,11 +253,12 @@ class GpuKernels(CommonKernels):
         if rank == 3:
             heads, zo, zq, zk, zv = dq[0], so[0], sq[0], sk[0], sv[0]
             assert do[0] == heads and dk[0] == heads and dv[0] == heads
-        rc = self._lib.adr_attention_f16(_current_stream(), output.data_ptr(), query.data_ptr(),
-                                         key.data_ptr(), value.data_ptr(), heads, m, n, d,
-                                         so[-1], so[-2], zo, sq[-1], sq[-2], zq,
-                                         sk[-1], sk[-2], zk, sv[-1], sv[-2], zv,
-                                         float(scale), float(temperature), int(mask))
+        args = (_current_stream(), output.data_ptr(), query.data_ptr(), key.data_ptr(), value.data_ptr(), heads, m, n, d,
+                so[-1], so[-2], zo, sq[-1], sq[-2], zq, sk[-1], sk[-2], zk, sv[-1], sv[-2], zv,
+                float(scale), float(temperature), int(mask))
+        ws = self._workspace
+        rc = (self._lib.adr_attention_f16(*args) if ws is None else
+              self._lib.adr_attention_f16_ws(*args, ws.data_ptr(), ws.numel()))
         if rc != 0:
             raise AdrasteaError(rc, "attention_f16")
 
@@ -373,9 +375,22 @@ def matmul_workspace_bytes(output: TensorLayout, left: TensorLayout, right: Tens
     return int(n)
 
 
+def attention_workspace_bytes(output: TensorLayout, query: TensorLayout, key: TensorLayout, value: TensorLayout,
+                              mask: int = MatmulMask.NONE) -> int:
+    """Scratch bytes adr_attention_f16_ws would use for these layouts (0: it would share no keys)."""
+    layouts, dims = (output, query, key, value), query.dims
+    rank = len(dims)
+    strides = [s for l in layouts for s in (l.strides[-1], l.strides[-2], l.strides[0] if rank == 3 else 0)]
+    n = _ffi.lib().adr_attention_f16_workspace_bytes(dims[0] if rank == 3 else 1, dims[-2], key.dims[-2], dims[-1],
+                                                     *strides, int(mask))
+    if n < 0:
+        raise AdrasteaError(int(n), "attention_f16_workspace_bytes")
+    return int(n)
+
+
 def set_held_workspace_limit(nbytes: int) -> None:
-    """Bytes per buffer of the workspace pool that adr_matmul_f16 and adr_matmul_nt_f16 (and, on
-    request, adr_matmul_nt_fp16u8) draw from, one buffer per (device, stream); 0 switches it off."""
+    """Bytes per buffer of the workspace pool that adr_matmul_f16, adr_matmul_nt_f16 and
+    adr_attention_f16 (and, on request, adr_matmul_nt_fp16u8) draw from, one buffer per (device, stream); 0 switches it off."""
     rc = _ffi.lib().adr_set_held_workspace_limit(int(nbytes))
     if rc != 0:
         raise AdrasteaError(int(rc), "set_held_workspace_limit")
@@ -398,7 +413,8 @@ def held_workspace_declined() -> int:
 def release_held_workspace(stream=None) -> None:
     """Frees the pool's buffers of `stream` (a raw stream handle; default: torch's current stream)
     and those no stream owns any more, after waiting for the last launches that used them.  Call it
-    before destroying a stream.  `stream="all"`: every buffer on every device."""
+    before destroying a stream, not while it is being captured.  `stream="all"`: every buffer on
+    every device."""
     L = _ffi.lib()
     rc = (L.adr_release_held_workspace_all() if stream == "all" else
           L.adr_release_held_workspace(_current_stream() if stream is None else stream))

@@ -172,8 +172,8 @@ int adr_matmul_f16_noalloc(adr_stream_t stream, uint16_t* output, const uint16_t
  * pool is full and holds no buffer large enough; a product that wants more than the limit is split
  * into fewer pieces instead.  adr_held_workspace_declined counts the calls that wanted a buffer and
  * ran without one.
- * Results: the split products sum K in pieces, so on inexact data the last bits may differ from
- * the unsplit launch (both within the stated tolerance).
+ * Results: the split products sum K in pieces, and attention adds up parts of its keys, so on inexact
+ * data the last bits may differ from the unsplit launch (both within the stated tolerance).
  *
  * adr_set_held_workspace_limit: bytes per buffer (default ADR_HELD_WORKSPACE_DEFAULT_BYTES =
  * 128 MiB); 0 switches the pool off for later calls (buffers already allocated stay until
@@ -185,8 +185,8 @@ int adr_matmul_f16_noalloc(adr_stream_t stream, uint16_t* output, const uint16_t
  * device, waiting for the devices where it must; not while anything on them is being captured.  A
  * buffer that cannot be waited for is kept, and the error returned.  (hipFree itself may wait for
  * other work on the device: these two are not for the hot path.)  Later calls allocate afresh.
- * Callers that must not allocate at all use adr_matmul_f16_noalloc or the _ws forms, which never
- * touch the pool.
+ * Callers that must not allocate at all use adr_matmul_f16_noalloc or the _ws forms (of products and
+ * of attention), which never touch the pool.
  *
  * adr_set_u8_dequantise_first(1): lets adr_matmul_nt_fp16u8 take the route of
  * adr_matmul_nt_fp16u8_ws by itself, with the dequantised matrix (n * p * 2 bytes, which must fit
@@ -354,6 +354,31 @@ int adr_attention_f16(adr_stream_t stream, uint16_t* output, const uint16_t* que
                       int32_t stride_kx, int32_t stride_ky, int32_t stride_kz, int32_t stride_vx,
                       int32_t stride_vy, int32_t stride_vz, float scale, float temp,
                       uint32_t mask);
+
+/*
+ * adr_attention_f16 with a caller-provided scratch buffer.  With few query rows (token generation,
+ * cross attention) the keys of a query block are shared by several workgroups, whose fp32 parts pass
+ * through scratch memory and are added by a second launch.  adr_attention_f16 takes that memory from
+ * the library's pool and so shares no keys where the pool cannot be used (under capture, with the
+ * limit at 0, ...): the sums are then in another order, and one row against 2047 keys takes twice the
+ * time.  Here the keys are shared through `workspace` (device memory, 16-byte aligned, of
+ * workspace_bytes bytes) in every context alike, and nothing is allocated; with less than
+ * adr_attention_f16_workspace_bytes reports they are cut into fewer parts, and with workspace_bytes ==
+ * 0 not at all: one launch, the same bits eagerly and under capture.  The workspace carries nothing
+ * from call to call; calls sharing one must not overlap in time.
+ */
+int adr_attention_f16_ws(adr_stream_t stream, uint16_t* output, const uint16_t* query,
+                         const uint16_t* key, const uint16_t* value, int32_t heads, int32_t m,
+                         int32_t n, int32_t d, int32_t stride_ox, int32_t stride_oy,
+                         int32_t stride_oz, int32_t stride_qx, int32_t stride_qy, int32_t stride_qz,
+                         int32_t stride_kx, int32_t stride_ky, int32_t stride_kz, int32_t stride_vx,
+                         int32_t stride_vy, int32_t stride_vz, float scale, float temp,
+                         uint32_t mask, void* workspace, int64_t workspace_bytes);
+/* Bytes (>= 0; 0: the keys would not be shared) or a negative ADR_E* code; touches no device memory. */
+int64_t adr_attention_f16_workspace_bytes(int32_t heads, int32_t m, int32_t n, int32_t d, int32_t stride_ox,
+                                          int32_t stride_oy, int32_t stride_oz, int32_t stride_qx, int32_t stride_qy,
+                                          int32_t stride_qz, int32_t stride_kx, int32_t stride_ky, int32_t stride_kz,
+                                          int32_t stride_vx, int32_t stride_vy, int32_t stride_vz, uint32_t mask);
 
 /*
  * Diagnostics (no counterpart in the reference).
