@@ -894,7 +894,10 @@ AttentionPlan attention_plan(const AttentionShape& t, int cus, int64_t avail) {
   p.cus = cus;
   p.wide = attention_wide(t);
   p.rows = t.m <= 16 && t.mask == ADR_MASK_NONE && !p.wide;
-  const int64_t part = (int64_t)t.heads * t.m * (t.d * 4 + 8), blocks = (int64_t)t.heads * ((t.m + BM - 1) / BM);
+  const int64_t rows = (int64_t)t.heads * t.m, blocks = (int64_t)t.heads * ((t.m + BM - 1) / BM);
+  // (rows beyond what all parts of can be counted in 31 bits fill the chip many times over)
+  const int most = rows <= 0x7fffffff / MAX_SPLITS ? MAX_SPLITS : 1;
+  const int64_t part = most > 1 ? rows * (t.d * 4 + 8) : 0;
   // One workgroup per compute unit at most: two groups take 9.5 us per 1000 keys where one takes 14
   // (two such workgroups per unit take as long as one of two groups), and half a microsecond to merge,
   // which pays from six tiles on (20 heads of 64, 1500 x 1500: 25.3 -> 21.2 us, 12 x 1000 causal
@@ -905,7 +908,7 @@ AttentionPlan attention_plan(const AttentionShape& t, int cus, int64_t avail) {
   // and 64-8192 keys with every number of parts: the rows kernel reads 69 GB/s per compute unit; parts
   // cost a launch (and the host its issue: more than a short read takes) and their way through memory.
   double best = 1e30;
-  for (int s = 1; s <= MAX_SPLITS && s * 64 <= t.n + 63 && (s == 1 || s * part <= avail); s++) {
+  for (int s = 1; s <= most && s * 64 <= t.n + 63 && (s == 1 || s * part <= avail); s++) {
     const double keys = (double)t.n / s;
     double us;
     if (p.rows) {
@@ -954,7 +957,8 @@ hipError_t launch_attention(hipStream_t stream, half_t* out, const half_t* q, co
   a.part_ml = (float2*)((float*)workspace + (a.splits > 1 ? a.splits * rows * t.d : 0));
   a.qblocks = (t.m + BM - 1) / BM;
   a.upper = (int64_t)t.heads * a.qblocks * a.splits <= 2 * p.cus ? (a.qblocks + 1) / 2 : a.qblocks;
-  if (rows * a.splits > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+  // (parts are shared only where their rows can be counted: no product here runs over)
+  if ((int64_t)t.heads * a.qblocks * a.splits > 0x7fffffffLL) return hipErrorInvalidConfiguration;
   if (t.d == 128) attention_launches<128>(stream, a, p);
   else attention_launches<64>(stream, a, p);
   return hipGetLastError();

@@ -42,3 +42,12 @@ def test_workspace_argument_is_checked():
     assert lib.adr_attention_f16_ws(*args, None, 64) == _ffi.ADR_ENULL
     assert lib.adr_attention_f16_ws(*args, 64, -1) == _ffi.ADR_ENULL
     assert lib.adr_attention_f16_ws(*args, 72, 1 << 20) == _ffi.ADR_EINVAL_SHAPE
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("heads,m", [(2**31 - 1, 2**31 - 1), (2**31 - 1, 1), (2**20, 2**31 - 1), (2**24, 128)])
+def test_more_rows_than_parts_are_counted_for(heads, m, d):
+    """Query rows by the thousands of millions (rows may overlap): the keys are not shared, and no count of
+    rows, parts and bytes runs over on the way to saying so."""
+    strides = [1, d, 0] * 4
+    assert _ffi.lib().adr_attention_f16_workspace_bytes(heads, m, 4096, d, *strides, 0) == 0
