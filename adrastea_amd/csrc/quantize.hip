@@ -201,9 +201,10 @@ hipError_t launch_quantize(hipStream_t stream, adr_tensor_desc out, adr_tensor_d
     int log2_bs = 3;
     while ((1 << log2_bs) < block_size) log2_bs++;
     const int64_t all = (int64_t)rows * cols;
-    // one long row: rows without gaps, and scales too
+    // one long row: rows without gaps, and scales too, as long as a launch takes its lanes along x (2^32)
     const bool flat = in.strides[1] == cols && out.strides[1] == cols &&
-                      (uint64_t)scales.strides[1] == (uint64_t)scales.strides[0] * blocks_per_row;
+                      (uint64_t)scales.strides[1] == (uint64_t)scales.strides[0] * blocks_per_row &&
+                      (all - 1) / (2048 * QV_CHUNKS) < 0xffffff;
     const int64_t len = flat ? all : cols;
     const int64_t groups = (len + 2048 * QV_CHUNKS - 1) / (2048 * QV_CHUNKS);
     hipLaunchKernelGGL(quantize_vec_kernel,

@@ -65,3 +65,29 @@ def test_rows_with_gaps(cols, bs, gap_in, gap_q, gap_s):
     assert np.array_equal(s[:, :cols // bs].cpu().numpy().view(np.uint16), want_s.view(np.uint16))
     assert np.array_equal(q[:, :cols].cpu().numpy(), want_q)
     assert (q[:, cols:] == 7).all() and (s[:, cols // bs:] == 7).all()
+
+
+def test_more_values_than_one_launch_counts_along_x():
+    """2^36 values: as one long row they would be 2^24 workgroups of 256 lanes, one lane more than a launch takes."""
+    rows, cols = 1 << 20, 1 << 16
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    need = rows * cols * 3 + rows * (cols // 32) * 2
+    if torch.cuda.mem_get_info()[0] < need + (8 << 30):
+        pytest.skip("less than 219 GB of device memory free")
+    x = torch.ones(rows, cols, dtype=torch.float16, device="cuda")
+    ends = [0, 1, 2, 3, rows - 2, rows - 1]
+    x[ends] = torch.randn(len(ends), cols, dtype=torch.float16, device="cuda")
+    q = torch.zeros(rows, cols, dtype=torch.uint8, device="cuda")
+    s = torch.zeros(rows, cols // 32, dtype=torch.float16, device="cuda")
+    try:
+        GpuKernels().quantize_absmax_uint8(q, s, x)
+        want_q, want_s = oracle.quantize_absmax_u8(x[ends].cpu().numpy(), 32)
+        assert np.array_equal(q[ends].cpu().numpy(), want_q)
+        assert np.array_equal(s[ends].cpu().numpy().view(np.uint16), want_s.view(np.uint16))
+        one_q, one_s = oracle.quantize_absmax_u8(np.ones((1, 32), np.float16), 32)
+        assert all((q[r:r + 65536] == int(one_q[0, 0])).all() for r in range(65536, rows - 65536, 65536))
+        assert all((s[r:r + 65536] == float(one_s[0, 0])).all() for r in range(65536, rows - 65536, 65536))
+    finally:
+        del x, q, s
+        torch.cuda.empty_cache()
