@@ -922,6 +922,11 @@ AttentionPlan attention_plan(const AttentionShape& t, int cus, int64_t avail) {
     }
     if (s > 1) us += s * part / 1.35e6;
     if (us < best * 0.97) best = us, p.splits = s;
+    // Under some 500 keys the second launch is time the host does not have: a call of two takes it 10 us,
+    // and one walk over all keys is over before (17 rows, 16 heads of 64: 257 keys 7.3 us unshared, 10.2
+    // shared; 500 keys 8.0, 10.2; at 640 8.1, 9.9, but 8.1, 7.4 on the device; 2 heads of 128: 384 keys 8.6,
+    // 10.0; 500 9.9, 10.0; 640 10.9, 9.9).
+    if (!p.rows && s == 1 && us < 5.5) break;
   }
   if (p.splits > 1) p.groups = 1;
   p.workspace_bytes = p.splits > 1 ? p.splits * part : 0;

@@ -19,6 +19,9 @@ def test_workspace_bytes():
     assert need(32, 2048, 2048, 128) == 0                     # query blocks enough
     assert need(32, 1, 64, 128) == 0                          # keys too few
     assert need(1, 40, 2000, 128) > 0
+    # parts pay for a second launch: not where the keys of one are read in the time that takes
+    assert all(need(heads, 17, n, 64) == 0 for heads in (1, 12, 16) for n in (257, 384, 500))
+    assert need(2, 512, 512, 64, 1) == 0
 
 
 @pytest.mark.parametrize("bad,code", [(dict(d=96), _ffi.ADR_EUNSUPPORTED_LAYOUT), (dict(n=-1), _ffi.ADR_EINVAL_SHAPE),

@@ -105,7 +105,7 @@ def test_keys_shared_by_workgroups(heads, m, n, d):
         K.release_held_workspace("all")
 
 
-@pytest.mark.parametrize("heads,m,n,d", [(2, 512, 512, 64), (1, 700, 700, 64), (2, 130, 640, 128), (1, 1000, 1000, 128),
+@pytest.mark.parametrize("heads,m,n,d", [(2, 900, 900, 64), (1, 700, 700, 64), (2, 130, 640, 128), (1, 1000, 1000, 128),
                                          (3, 129, 2000, 64)])
 def test_keys_shared_by_workgroups_under_the_mask(heads, m, n, d):
     """A query block's tiles end at the diagonal: parts of unequal length, and parts of the first blocks
@@ -125,7 +125,7 @@ def test_more_workgroups_than_fit():
 @pytest.mark.parametrize("m,causal", [(1, False), (33, False), (130, True)])
 def test_keys_that_overlap(m, causal, shared):
     """A window over a signal: key rows of 64 elements, 8 apart (rows closer than they are long)."""
-    n, d = 300, 64
+    n, d = 600, 64
     g = torch.Generator(device="cuda").manual_seed(3)
     signal = torch.randn(n * 8 + d, device="cuda", dtype=torch.float16, generator=g)
     v = torch.randn(n, d, device="cuda", dtype=torch.float16, generator=g)
@@ -143,9 +143,9 @@ def test_keys_that_overlap(m, causal, shared):
 
 # (query rows, keys, elements between query rows, between key and value rows)
 FAR = [(40, 70, 1 << 22, 1 << 22),             # rows of 8 MiB: two tiles do not fit the offsets
-       (40, 300, 1 << 21, (1 << 22) - 64),     # a head of 2^30 elements and more
+       (40, 600, 1 << 21, 1 << 21),            # a head of 2^30 elements and more
        (3, 70, 512, 1 << 22),
-       (257, 300, 1 << 22, 512)]               # query rows alone
+       (257, 600, 1 << 22, 512)]               # query rows alone
 
 
 @pytest.mark.parametrize("shared", [False, True])
