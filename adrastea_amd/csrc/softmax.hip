@@ -103,7 +103,7 @@ __global__ __launch_bounds__(256) void softmax_rows_reg_kernel(half_t* out, cons
 // the dwords and halves that are its own.  Chunks counted from the row's first element had to be
 // shifted into place, a second request per chunk: 48000 rows of 1500 80 -> 64 us = 4.5 TB/s, 30000 of
 // them 52.7 -> 42.5, 32016 of 2001 65.8 -> 52.5, 24008 of 3001 76.4 -> 59.7, 32760 of 4095 119.5 -> 103,
-// 12240 of 1530 22.7 -> 19.1; 19232 of 601 19.7 and 16352 of 2044 29.7 either way.  (Cached stores
+// 12240 of 1530 22.7 -> 19.1; 16352 of 2044 29.7 either way.  (Cached stores
 // instead of streaming ones, and a contiguous piece of the tensor for each die, change nothing.)
 // NV: chunks per lane; every row of the tensor touches at most 64 NV chunks (see the launch).
 template <int NV>
@@ -181,10 +181,13 @@ __global__ __launch_bounds__(256) void softmax_rows_anyrow_kernel(half_t* out, c
   }
 }
 
-// The same on chunks counted from the row's first element, moved with load8_any / store8_any: for the
-// few lengths just short of 512 or 1024 whose aligned pieces are one more per lane, which there costs
-// more than the shifting (8168 rows of 1021 11.7 us against 13.5, 8144 of 509 6.9 against 10.0; from
-// 1500 on it no longer does: 16376 of 2047 32.6 against 33.0).
+// The same on chunks counted from the row's first element, moved with load8_any / store8_any.  Up to 1024
+// elements, one or two chunks per lane, the second request is cheaper than the masks of the pieces at
+// both ends (544714 rows of 77 218 us against 238, 163202 of 257 69.2 against 75.6, 125955 of 333 54.9 against
+// 59.7; 436 of 601 3.7 against 3.9, 69788 of them 57.6 either way; at 1100 238 rows take 4.6 against 4.0 and
+// 38130 58 against 45).  So it is for the lengths just short of 2048 whose aligned pieces are one more
+// per lane, unless the tensor is large (4098 rows of 2047 11.5 against 12.6, 8196 17.8 against 19.5, 20490
+// 42.5 against 40.1).
 template <int NV>
 __global__ __launch_bounds__(256) void softmax_rows_shifted_kernel(half_t* out, const half_t* in,
                                                                   int64_t rows, int w, float temp) {
@@ -289,13 +292,13 @@ hipError_t launch_softmax_rows(hipStream_t stream, half_t* out, const half_t* in
     const int g = w % 2 ? 1 : w % 4 ? 2 : w % 8 ? 4 : 8;
     const int lead = 8 - g + (int)(((uintptr_t)in & 15) >> 1) % g;
     const int per_lane = ((lead + w + 7) / 8 + 63) / 64;
-    if (per_lane == 2 && w <= 512)
+    if (w <= 512)
       hipLaunchKernelGGL(softmax_rows_shifted_kernel<1>, grid, block, 0, stream, out, in, rows, w, temp);
-    else if (per_lane == 3 && w <= 1024)
+    else if (w <= 1024)
       hipLaunchKernelGGL(softmax_rows_shifted_kernel<2>, grid, block, 0, stream, out, in, rows, w, temp);
+    else if (per_lane == 5 && w < 2048 && rows <= 12288)
+      hipLaunchKernelGGL(softmax_rows_shifted_kernel<4>, grid, block, 0, stream, out, in, rows, w, temp);
     else switch (per_lane) {
-      case 1: hipLaunchKernelGGL(softmax_rows_anyrow_kernel<1>, grid, block, 0, stream, out, in, rows, w, temp); break;
-      case 2: hipLaunchKernelGGL(softmax_rows_anyrow_kernel<2>, grid, block, 0, stream, out, in, rows, w, temp); break;
       case 3: hipLaunchKernelGGL(softmax_rows_anyrow_kernel<3>, grid, block, 0, stream, out, in, rows, w, temp); break;
       case 4: hipLaunchKernelGGL(softmax_rows_anyrow_kernel<4>, grid, block, 0, stream, out, in, rows, w, temp); break;
       case 5: hipLaunchKernelGGL(softmax_rows_anyrow_kernel<5>, grid, block, 0, stream, out, in, rows, w, temp); break;

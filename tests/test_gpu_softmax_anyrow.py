@@ -12,7 +12,7 @@ from helpers import rng, ulp_diff_f16
 
 pytestmark = pytest.mark.gpu
 
-WIDTHS = [1, 2, 7, 9, 505, 506, 512, 513, 1017, 1018, 1024, 1500, 1529, 1530, 2041, 2042, 2048, 3065, 3066,
+WIDTHS = [1, 2, 7, 9, 505, 506, 512, 513, 1017, 1018, 1024, 1500, 1529, 1530, 2041, 2042, 2043, 2047, 2048, 3065, 3066,
           4082, 4089, 4095, 4096]
 
 
@@ -43,3 +43,15 @@ def test_edges_of_rows_and_chunks(w):
         inplace = to_np(buf)
         assert np.array_equal(inplace[start_in:start_in + n], got[start_out:start_out + n])
         assert np.all(np.isinf(inplace[:start_in])) and np.all(np.isinf(inplace[start_in + n:]))
+
+
+@pytest.mark.parametrize("rows", [12288, 12289])
+@pytest.mark.parametrize("w", [2043, 2046, 2047])
+def test_one_more_piece_per_lane_in_few_rows_and_in_many(w, rows):
+    g = torch.Generator(device="cuda").manual_seed(w + rows)
+    x = torch.randn(1, rows, w, dtype=torch.float16, device="cuda", generator=g) * 4
+    want = torch.softmax(x.double(), -1).half()
+    s = torch.cuda.current_stream().cuda_stream
+    assert _ffi.lib().adr_softmax_rows(s, x.data_ptr(), x.data_ptr(), 1, rows, w, 1.0) == 0
+    steps = (x.view(torch.int16).int() - want.view(torch.int16).int()).abs().max()   # (no signs: all are >= 0)
+    assert int(steps) <= 1
