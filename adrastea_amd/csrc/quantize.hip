@@ -110,26 +110,30 @@ __device__ __forceinline__ u32x2_t quantize8_div(half8_t v, float fs) {
   return u32x2_t{w[0], w[1]};
 }
 
-// Contiguous rows, block sizes 8 * 2^k <= 512: a lane takes QV_CHUNKS groups of 8 consecutive values
+// Contiguous rows, block sizes 8 * 2^k <= 512: a lane takes CHUNKS groups of 8 consecutive values
 // (one 16-byte load and one 8-byte store each, all loads issued first), the bs/8 lanes of a block
 // find the absmax with xor shuffles.  Same results, bit for bit, as quantize_kernel.  Tensors
 // without gaps between their rows arrive as one long row, so that no lane idles behind a row's end.
-constexpr int QV_CHUNKS = 2;
+// Two chunks are for large ones, from memory (11008 x 4096 27.5 us against 28.2 with one, 13824 x 5120 39.6
+// against 40.3; 4096 x 4096 13.1 against 12.5, 5120 x 1280 7.4 against 6.7): the second keeps more in flight
+// and halves the workgroups that fill the chip.  Rows with gaps end too often for it (50000 rows of 64
+// 31.3 against 20.6).
+template <int CHUNKS>
 __global__ __launch_bounds__(256) void quantize_vec_kernel(uint8_t* out, half_t* scales, const half_t* in,
                                                            int64_t cols, int64_t out_stride, int64_t scale_row,
                                                            int64_t scale_stride, int64_t in_stride, int log2_bs,
                                                            int chunks_on_x) {
   const int64_t row = chunks_on_x ? 0 : blockIdx.x;
-  const int64_t c0 = ((int64_t)(chunks_on_x ? blockIdx.x : blockIdx.y) * (256 * QV_CHUNKS) + threadIdx.x) * 8;
+  const int64_t c0 = ((int64_t)(chunks_on_x ? blockIdx.x : blockIdx.y) * (256 * CHUNKS) + threadIdx.x) * 8;
   const half_t* x = in + row * in_stride;
-  half8_t v[QV_CHUNKS];
+  half8_t v[CHUNKS];
 #pragma unroll
-  for (int j = 0; j < QV_CHUNKS; j++) {
+  for (int j = 0; j < CHUNKS; j++) {
     const int64_t c = c0 + j * 2048;  // cols % block_size == 0, so a block is all live or all dead
     v[j] = *(const half8_t*)(x + (c < cols ? c : 0));  // (unconditional: all in flight together)
   }
 #pragma unroll
-  for (int j = 0; j < QV_CHUNKS; j++) {
+  for (int j = 0; j < CHUNKS; j++) {
     const int64_t c = c0 + j * 2048;
     float absmax = 0.0f;
 #pragma unroll
@@ -204,10 +208,11 @@ hipError_t launch_quantize(hipStream_t stream, adr_tensor_desc out, adr_tensor_d
     // one long row: rows without gaps, and scales too, as long as a launch takes its lanes along x (2^32)
     const bool flat = in.strides[1] == cols && out.strides[1] == cols &&
                       (uint64_t)scales.strides[1] == (uint64_t)scales.strides[0] * blocks_per_row &&
-                      (all - 1) / (2048 * QV_CHUNKS) < 0xffffff;
+                      (all - 1) / 4096 < 0xffffff;
     const int64_t len = flat ? all : cols;
-    const int64_t groups = (len + 2048 * QV_CHUNKS - 1) / (2048 * QV_CHUNKS);
-    hipLaunchKernelGGL(quantize_vec_kernel,
+    const int chunks = flat && all >= 32 << 20 ? 2 : 1;
+    const int64_t groups = (len + 2048 * chunks - 1) / (2048 * chunks);
+    hipLaunchKernelGGL(chunks == 2 ? quantize_vec_kernel<2> : quantize_vec_kernel<1>,
                        flat ? dim3((uint32_t)groups, 1, 1) : dim3(rows, (uint32_t)groups, 1), dim3(256, 1, 1), 0,
                        stream, (uint8_t*)out.ptr, (half_t*)scales.ptr, (const half_t*)in.ptr, len,
                        (int64_t)out.strides[1], (int64_t)scales.strides[1], (int64_t)scales.strides[0],
