@@ -156,6 +156,11 @@ __device__ __forceinline__ void barrier() {
 // 2048 and under the mask (twice the MFMAs to issue, and registers spilled in the prologue); two
 // groups half a tile apart, one in the MFMAs of a whole tile while the other is in its softmax, took
 // 82 us: alone on its SIMD's vector ALU a wavefront issues at half the rate.
+// HD = 128 keeps 22 vector registers in scratch memory (WIDE 42), HD = 64 none: all of them in the
+// straight-line halves behind the main loop, none in it.  One tile of keys takes 0.2-0.7 us
+// more than it did without the overlap (32 heads of 128, 17 rows against 64 keys 3.9 -> 4.6): the code of
+// all halves, and Q and the output by way of LDS.  Asking whether a tile is left before its transfers
+// there, or for a single tile's V together with its K, made it 0.1-0.2 us longer still.
 template <int HD, int G, bool WIDE>
 __global__ __launch_bounds__(256 * G, 2) void attention_fwd_kernel(AttnArgs a) {
   constexpr int CPR = HD / 8;
@@ -667,8 +672,8 @@ __global__ __launch_bounds__(256 * G, 2) void attention_fwd_kernel(AttnArgs a) {
 // that of the kernel above on 16x16x32 MFMAs: S^T = K Q^T, so that a lane holds scores of one query
 // row, and O^T = V^T P^T.  The four partial results meet in LDS.
 // Bound by the path into a compute unit (69 GB/s) where one workgroup has a head to itself, by memory
-// where the parts fill the chip: 32 heads of 128, one row against 2047 keys 41.0 -> 11.7 us in eight
-// parts (19.5 in one; 33.5 MB), against 500 keys 10 -> 6.6 in one, against 8192 105 -> 31.
+// where the parts fill the chip: 32 heads of 128, K and V from HBM, one row against 2047 keys 42 -> 12.7 us
+// in eight parts (27 in one; 33.5 MB), against 500 keys 13.2 -> 9.9 in one, against 8192 156 -> 31.
 template <int HD>
 __global__ __launch_bounds__(256) void attention_rows_kernel(AttnArgs a) {
   constexpr int CPR = HD / 8, KEYS = 32;

@@ -83,8 +83,8 @@ __global__ __launch_bounds__(256) void quantize_kernel(adr_tensor_desc out, adr_
 // 2 * 31743^2 finite operand pairs give the same bytes as the division).  floor(v + 0.5) is roundf(v)
 // where v >= 0 -- v is a multiple of 2^-18 there -- and below zero either one clamps to 0.  The byte
 // conversion saturates and takes NaN to 0.  Eight instructions a value where the division and
-// roundf take some thirty: at 4 cycles an instruction those were the time of the kernel (11008 x 4096 39 us,
-// now 25 us = 5.5 TB/s).
+// roundf take some thirty: at 4 cycles an instruction those were the time of the kernel (11008 x 4096 from
+// memory 42-45 us, now 27-28 = 5 TB/s).
 __device__ __forceinline__ u32x2_t quantize8(half8_t v, float fs, float r) {
   uint32_t w[2] = {0, 0};
 #pragma unroll

