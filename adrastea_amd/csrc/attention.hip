@@ -7,6 +7,7 @@
 // bit for bit.
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "adr_common.hpp"
@@ -908,6 +909,8 @@ AttentionPlan attention_plan(const AttentionShape& t, int cus, int64_t avail) {
   AttentionPlan p;
   p.cus = cus;
   p.wide = attention_wide(t);
+  // (no row sees a key past the last row's own)
+  const int n = t.mask == ADR_MASK_CAUSAL ? std::min(t.n, t.m) : t.n;
   p.rows = t.m <= 16 && t.mask == ADR_MASK_NONE && !p.wide;
   const int64_t rows = (int64_t)t.heads * t.m, blocks = (int64_t)t.heads * ((t.m + BM - 1) / BM);
   // (rows beyond what all parts of can be counted in 31 bits fill the chip many times over)
@@ -917,14 +920,14 @@ AttentionPlan attention_plan(const AttentionShape& t, int cus, int64_t avail) {
   // (two such workgroups per unit take as long as one of two groups), and half a microsecond to merge,
   // which pays from six tiles on (20 heads of 64, 1500 x 1500: 25.3 -> 21.2 us, 12 x 1000 causal
   // 15.3 -> 12.7; 12 x 256 6.2 -> 6.3).
-  p.groups = !p.rows && !p.wide && blocks <= cus && t.n > 5 * BN ? 2 : 1;
+  p.groups = !p.rows && !p.wide && blocks <= cus && n > 5 * BN ? 2 : 1;
   p.splits = 1;
   // Times beyond what every launch takes, in us, fitted to 40 shapes of 12-40 heads, 1-448 query rows
   // and 64-8192 keys with every number of parts: the rows kernel reads 69 GB/s per compute unit; parts
   // cost a launch (and the host its issue: more than a short read takes) and their way through memory.
   double best = 1e30;
-  for (int s = 1; s <= most && s * 64 <= t.n + 63 && (s == 1 || s * part <= avail); s++) {
-    const double keys = (double)t.n / s;
+  for (int s = 1; s <= most && s * 64 <= n + 63 && (s == 1 || s * part <= avail); s++) {
+    const double keys = (double)n / s;
     double us;
     if (p.rows) {
       us = ceil((double)t.heads * s / cus) * keys * t.d * (4.0 / 69e3);

@@ -22,6 +22,9 @@ def test_workspace_bytes():
     # parts pay for a second launch: not where the keys of one are read in the time that takes
     assert all(need(heads, 17, n, 64) == 0 for heads in (1, 12, 16) for n in (257, 384, 500))
     assert need(2, 512, 512, 64, 1) == 0
+    # nor for keys that no row sees
+    assert all(need(32, m, 2000, 128, 1) == 0 for m in (40, 64, 130))
+    assert need(2, 700, 2000, 64, 1) == need(2, 700, 700, 64, 1) > 0
 
 
 @pytest.mark.parametrize("bad,code", [(dict(d=96), _ffi.ADR_EUNSUPPORTED_LAYOUT), (dict(n=-1), _ffi.ADR_EINVAL_SHAPE),

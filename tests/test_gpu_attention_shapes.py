@@ -105,8 +105,8 @@ def test_keys_shared_by_workgroups(heads, m, n, d):
         K.release_held_workspace("all")
 
 
-@pytest.mark.parametrize("heads,m,n,d", [(2, 900, 900, 64), (1, 700, 700, 64), (2, 130, 640, 128), (1, 1000, 1000, 128),
-                                         (3, 129, 2000, 64)])
+@pytest.mark.parametrize("heads,m,n,d", [(2, 900, 900, 64), (1, 700, 700, 64), (1, 700, 600, 128), (1, 600, 600, 64),
+                                         (2, 700, 2000, 64), (1, 1000, 600, 64)])
 def test_keys_shared_by_workgroups_under_the_mask(heads, m, n, d):
     """A query block's tiles end at the diagonal: parts of unequal length, and parts of the first blocks
     without any tile, whose sums of nothing must not count."""
@@ -122,7 +122,7 @@ def test_more_workgroups_than_fit():
 
 
 @pytest.mark.parametrize("shared", [False, True])
-@pytest.mark.parametrize("m,causal", [(1, False), (33, False), (130, True)])
+@pytest.mark.parametrize("m,causal", [(1, False), (33, False), (500, True)])
 def test_keys_that_overlap(m, causal, shared):
     """A window over a signal: key rows of 64 elements, 8 apart (rows closer than they are long)."""
     n, d = 600, 64
