@@ -342,6 +342,7 @@ struct AttentionShape {
 };
 struct AttentionPlan {
   bool rows;   // attention_rows_kernel
+  bool tile;   // attention_tile_kernel
   bool wide;   // 64-bit addresses (attention_fwd_kernel)
   int groups;  // of four wavefronts (attention_fwd_kernel)
   int splits;

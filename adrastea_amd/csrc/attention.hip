@@ -158,10 +158,7 @@ __device__ __forceinline__ void barrier() {
 // groups half a tile apart, one in the MFMAs of a whole tile while the other is in its softmax, took
 // 82 us: alone on its SIMD's vector ALU a wavefront issues at half the rate.
 // HD = 128 keeps 22 vector registers in scratch memory (WIDE 42), HD = 64 none: all of them in the
-// straight-line halves behind the main loop, none in it.  One tile of keys takes 0.2-0.7 us
-// more than it did without the overlap (32 heads of 128, 17 rows against 64 keys 3.9 -> 4.6): the code of
-// all halves, and Q and the output by way of LDS.  Asking whether a tile is left before its transfers
-// there, or for a single tile's V together with its K, made it 0.1-0.2 us longer still.
+// straight-line halves behind the main loop, none in it.
 template <int HD, int G, bool WIDE>
 __global__ __launch_bounds__(256 * G, 2) void attention_fwd_kernel(AttnArgs a) {
   constexpr int CPR = HD / 8;
@@ -666,6 +663,119 @@ __global__ __launch_bounds__(256 * G, 2) void attention_fwd_kernel(AttnArgs a) {
   }
 }
 
+// A single tile of keys and few rows: the same arithmetic, in the same order (so the same bits), with
+// nothing to overlap -- a workgroup per head, one trip to memory for Q, K and V together, one barrier,
+// any strides.  Bound by that trip and the launch.  In the kernel above such a call passes the code of all
+// four kinds of halves, waits for V behind the scores and takes Q and the output by way of LDS, which
+// pays from about 96 rows on: in a graph, us, this kernel against that one: 32 heads of 128, 64 keys, 17
+// rows 3.9 / 4.6, 64 4.7 / 4.9, 96 5.3 / 5.0, 300 6.1 / 5.5; 12 heads of 64 3.1 / 3.7, 3.5 / 3.8, 3.8 / 3.8, 4.1 / 3.9.
+template <int HD>
+__global__ __launch_bounds__(256, 2) void attention_tile_kernel(AttnArgs a) {
+  constexpr int CPR = HD / 8, ROWB = HD * 2, TILE = BN * ROWB, NI = TILE / 1024 / 4, DS = HD / 16, DT = HD / 32;
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * TILE];  // K, V
+
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int frow = lane & 31, g = lane >> 5;
+  const int head = blockIdx.x, qi = w * 32 + frow;
+  const bool causal = a.mask == ADR_MASK_CAUSAL;
+
+  half8_t qf[DS];
+  const half_t* const qrow = a.q + (int64_t)head * a.sq_z + (int64_t)min(qi, a.m - 1) * a.sq_y + g * 8;
+#pragma unroll
+  for (int ds = 0; ds < DS; ds++) qf[ds] = *(const half8_t*)(qrow + ds * 16);
+  // (rows past the last key fetch that one; their scores are masked)
+  const uint32_t lds0 = (uint32_t)(uintptr_t)ADR_LDS_PTR(smem) + w * (NI * 1024);
+#pragma unroll
+  for (int j = 0; j < NI; j++) {
+    int row, kc;
+    k_chunk_inv<CPR>((w * NI + j) * 64 + lane, row, kc);
+    dma_global(lds0 + j * 1024, a.k + (int64_t)head * a.sk_z + (int64_t)min(row, a.n - 1) * a.sk_y + kc * 8);
+  }
+#pragma unroll
+  for (int j = 0; j < NI; j++) {
+    const int phys = (w * NI + j) * 64 + lane, row = phys / CPR, c = (phys % CPR) ^ v_swz<CPR>(row);
+    dma_global(lds0 + TILE + j * 1024, a.v + (int64_t)head * a.sv_z + (int64_t)min(row, a.n - 1) * a.sv_y + c * 8);
+  }
+  int offV[DT];
+  {
+    const int c = lane & 15, b = (lane >> 4) & 1, row = 4 * g + (c >> 2);
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+      offV[dt] = row * ROWB + (((4 * dt + 2 * b + ((c & 3) >> 1)) ^ v_swz<CPR>(row)) << 4) + (c & 1) * 8;
+  }
+#pragma unroll
+  for (int ds = 0; ds < DS; ds++) asm volatile("" : "+v"(qf[ds]));
+  wait_vm<0>();
+  barrier();
+  if (w * 32 >= a.m) return;
+
+  float16_t s[2], o[DT];
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    s[0][r] = s[1][r] = 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++) o[dt][r] = 0.0f;
+  }
+#pragma unroll
+  for (int c = 0; c < DS; c++) {
+    const int ds = c ^ 1;
+#pragma unroll
+    for (int kt = 1; kt >= 0; kt--) {
+      const half8_t kf = *(const half8_t*)(smem + k_chunk_off<CPR>(frow, ds * 2 + g) + kt * 32 * ROWB);
+      s[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[ds], s[kt], 0, 0, 0);
+    }
+  }
+  float mx = -1.0e30f;
+  const int end = (causal ? min(a.n, qi + 1) : a.n) - 4 * g;  // this lane's first masked key
+#pragma unroll
+  for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      if (32 * kt + 8 * (r >> 2) + (r & 3) >= end) s[kt][r] = -INFINITY;
+      mx = fmaxf(mx, s[kt][r]);
+    }
+  const float m_row = fmaxf(-1.0e30f, pair_max(mx) * a.c);
+  float sum[2] = {0.0f, 0.0f};
+  u32x4_t pf[2][2];
+#pragma unroll
+  for (int x = 0; x < 32; x += 2) {
+    float2_t e;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      e[j] = __builtin_amdgcn_exp2f(fmaf(s[x >> 4][(x & 15) + j], a.c, -m_row));
+      sum[j] += e[j];
+    }
+    pf[x >> 4][x >> 3 & 1][(x & 7) / 2] = __builtin_bit_cast(uint32_t, __builtin_convertvector(e, half2_t));
+  }
+  typedef short short4_t __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) short4_t lds_short4_t;
+#pragma unroll
+  for (int x = 0; x < 4; x++) {
+    const int y = HD == 64 ? x ^ 1 : x, kt = y >> 1, t = y & 1;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++) {
+      const unsigned char* const p0 = smem + TILE + offV[dt] + (32 * kt + 16 * t) * ROWB;
+      const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)ADR_LDS_PTR(p0));
+      const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)ADR_LDS_PTR(p0 + 8 * ROWB));
+      const half8_t vf = __builtin_shufflevector(__builtin_bit_cast(half4_t, lo), __builtin_bit_cast(half4_t, hi),
+                                                 0, 1, 2, 3, 4, 5, 6, 7);
+      o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, __builtin_bit_cast(half8_t, pf[kt][t]), o[dt], 0, 0, 0);
+    }
+  }
+  const float inv = 1.0f / pair_sum(sum[0] + sum[1]);
+  if (qi >= a.m) return;
+  half_t* const orow = a.out + (int64_t)head * a.so_z + (int64_t)qi * a.so_y + 4 * g;
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      half4_t r;
+#pragma unroll
+      for (int j = 0; j < 4; j++) r[j] = (half_t)(o[dt][4 * i + j] * inv);
+      *(half4_t*)(orow + 32 * dt + 8 * i) = r;
+    }
+}
+
 // At most sixteen query rows (generation, cross attention) against all keys, no mask: a read of K and
 // V.  A workgroup takes one head and one of `splits` parts of its keys; its four wavefronts walk
 // tiles of 32 keys in turn, each through two tiles' worth of LDS of its own, so that up to 128 KiB of
@@ -909,9 +1019,10 @@ AttentionPlan attention_plan(const AttentionShape& t, int cus, int64_t avail) {
   AttentionPlan p;
   p.cus = cus;
   p.wide = attention_wide(t);
+  p.rows = t.m <= 16 && t.mask == ADR_MASK_NONE && !p.wide;
   // (no row sees a key past the last row's own)
   const int n = t.mask == ADR_MASK_CAUSAL ? std::min(t.n, t.m) : t.n;
-  p.rows = t.m <= 16 && t.mask == ADR_MASK_NONE && !p.wide;
+  p.tile = !p.rows && n <= BN && t.m <= 80;  // (between 65 rows, where that kernel still is ahead, and 96)
   const int64_t rows = (int64_t)t.heads * t.m, blocks = (int64_t)t.heads * ((t.m + BM - 1) / BM);
   // (rows beyond what all parts of can be counted in 31 bits fill the chip many times over)
   const int most = rows <= 0x7fffffff / MAX_SPLITS ? MAX_SPLITS : 1;
@@ -955,6 +1066,7 @@ template <int HD>
 static void attention_launches(hipStream_t stream, const AttnArgs& a, const AttentionPlan& p) {
   const dim3 block(256), grid((unsigned)(a.heads * (p.rows ? 1 : a.qblocks) * a.splits));
   if (p.rows) hipLaunchKernelGGL(attention_rows_kernel<HD>, grid, block, 0, stream, a);
+  else if (p.tile) hipLaunchKernelGGL(attention_tile_kernel<HD>, grid, block, 0, stream, a);
   else if (p.wide) hipLaunchKernelGGL(HIP_KERNEL_NAME(attention_fwd_kernel<HD, 1, true>), grid, block, 0, stream, a);
   else if (p.groups == 2) hipLaunchKernelGGL(HIP_KERNEL_NAME(attention_fwd_kernel<HD, 2, false>), grid, dim3(512), 0, stream, a);
   else hipLaunchKernelGGL(HIP_KERNEL_NAME(attention_fwd_kernel<HD, 1, false>), grid, block, 0, stream, a);

@@ -116,6 +116,16 @@ def test_keys_shared_by_workgroups_under_the_mask(heads, m, n, d):
         assert torch.equal(shared, run(heads, m, n, d, True))
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("m", [17, 31, 33, 64, 65, 79, 80, 81])
+def test_one_tile_of_keys(m, d):
+    for n in (1, 5, 31, 33, 63, 64, 65):
+        run(3, m, n, d, False)
+        run(3, m, n, d, True)
+    run(2, min(m, 64), 200, d, True)   # more keys, but only a tile of them is seen
+    run(2, 7, 64, d, True)
+
+
 def test_more_workgroups_than_fit():
     run(40, 1700, 1700, 128, True)   # 560 blocks: dealt out from the longest to the shortest
     run(32, 1100, 300, 64, False)
@@ -142,7 +152,8 @@ def test_keys_that_overlap(m, causal, shared):
 
 
 # (query rows, keys, elements between query rows, between key and value rows)
-FAR = [(40, 70, 1 << 22, 1 << 22),             # rows of 8 MiB: two tiles do not fit the offsets
+FAR = [(40, 50, 1 << 22, 1 << 25),             # one tile; a head of 2^30 elements and more
+       (40, 70, 1 << 22, 1 << 22),             # rows of 8 MiB: two tiles do not fit the offsets
        (40, 600, 1 << 21, 1 << 21),            # a head of 2^30 elements and more
        (3, 70, 512, 1 << 22),
        (257, 600, 1 << 22, 512)]               # query rows alone
@@ -181,6 +192,7 @@ def test_rows_far_apart(m, n, far_q, far_k, d, shared):
 @pytest.mark.parametrize("shared", [False, True])
 @pytest.mark.parametrize("heads,m,n,d", [(4, 3, 2048, 128),   # at most sixteen rows, its four wavefronts; parts
                                          (3, 16, 1000, 64),
+                                         (2, 40, 64, 128),    # one tile
                                          (2, 40, 300, 64),    # one group
                                          (2, 130, 640, 64),   # two groups; parts
                                          (2, 40, 2000, 128)])
