@@ -39,6 +39,7 @@
 // 16-byte chunks of output rows, applying the store operator, the bias and the causal mask on
 // the way.
 #include <stdint.h>
+#include <stdio.h>
 #include <type_traits>
 
 #include "adr_common.hpp"
@@ -605,7 +606,7 @@ __global__ __launch_bounds__(WM* WN * 64, MINB) void gemm_nt_dma_kernel(MatmulAr
   constexpr int FM = WTM / MI, FN = WTN / MI;  // MFMA blocks of the wavefront's sub-tile
   constexpr int TN2 = WTN / 16;                // the sub-tile's width in 16-column blocks
   constexpr int SLOT = 32 * (TN2 * 32 + 16);
-  static_assert(!MI16 || (!NN && !SPLIT), "16x16x32: plain NT products");
+  static_assert(!MI16 || !NN, "16x16x32: NT products");
   static_assert(BM * CPR % (NWD * 64) == 0 && BN * CPR % (NWD * 64) == 0,
                 "slices must split evenly over lanes");
   static_assert(WTM % 32 == 0 && WTN % (MI16 ? 16 : 32) == 0,
@@ -619,7 +620,7 @@ __global__ __launch_bounds__(WM* WN * 64, MINB) void gemm_nt_dma_kernel(MatmulAr
                 "epilogue slots must fit in the stage buffers");
   static_assert(NSTAGE == 2 || NSTAGE == 3 || NSTAGE == 6 || NSTAGE == 7,
                 "2 or 3 LDS stages, or 6: two stages of the left and four of the right operand");
-  static_assert(NSTAGE < 6 || (!NN && !SPLIT && NW % 2 == 0), "role split: plain NT products");
+  static_assert(NSTAGE < 6 || (!NN && NW % 2 == 0), "role split: NT products");
   static_assert(!NN || BN == 128, "the N-contiguous right operand is staged as [64][128] tiles");
   // Separate objects per stage: the compiler's alias analysis then knows that the asynchronous
   // LDS writes of one stage cannot touch the stage being read, and does not serialise them.
@@ -956,6 +957,7 @@ __global__ __launch_bounds__(WM* WN * 64, MINB) void gemm_nt_dma_kernel(MatmulAr
   wait_dma_barrier(std::integral_constant<int, 0>{});
 
   if constexpr (SPLIT) {
+    // (a 32 x 32 block of results is four float4 a lane; splitk_reduce_kernel sums block by block)
     float4_t* const ws = (float4_t*)a.workspace +
                          ((int64_t)piece * map.total + tile_id) * (TM * TN * 4) * NT + tid;
 #pragma unroll
@@ -964,8 +966,11 @@ __global__ __launch_bounds__(WM* WN * 64, MINB) void gemm_nt_dma_kernel(MatmulAr
       for (int j = 0; j < TN; j++)
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-          const float4_t v = {acc[i][j][4 * c], acc[i][j][4 * c + 1], acc[i][j][4 * c + 2],
-                              acc[i][j][4 * c + 3]};
+          float4_t v;
+          if constexpr (MI16)
+            v = acc[2 * i + c / 2][2 * j + c % 2];
+          else
+            v = float4_t{acc[i][j][4 * c], acc[i][j][4 * c + 1], acc[i][j][4 * c + 2], acc[i][j][4 * c + 3]};
           ws[(int64_t)((i * TN + j) * 4 + c) * NT] = v;
         }
     return;
@@ -993,49 +998,65 @@ __global__ __launch_bounds__(WM* WN * 64, MINB) void gemm_nt_dma_kernel(MatmulAr
 #endif
 }
 
-// Second launch of a split product: one workgroup per tile, with the geometry of the kernel that
-// wrote the pieces.  Every thread sums its accumulator registers over the pieces (always in the
-// order 0, 1, 2, ...: the result does not depend on which workgroup finished first) and the
-// epilogue of the unsplit kernel stores the tile.
-template <int BM, int BN, int WM, int WN>
-__global__ __launch_bounds__(WM* WN * 64) void splitk_reduce_kernel(MatmulArgs a, TileMap map) {
+// Second launch of a split product: every wavefront sums one 32 x 32 block of results over the pieces
+// (always in the order 0, 1, 2, ...: the result does not depend on which workgroup finished first)
+// and the epilogue of the unsplit kernel stores the block.  A block is four float4 a lane and piece;
+// four pieces' worth are requested before the first is added.  (One workgroup per tile, with
+// the geometry of the kernel that wrote the pieces, had 32 workgroups walk 16 MB for K11008 N4096 m=128.)
+template <int BM, int BN, int WM, int WN, bool MI16>
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(MatmulArgs a, TileMap map) {
   constexpr int NW = WM * WN, NT = NW * 64;
   constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
-  constexpr int SLOT = 32 * (TN * 64 + 16);
-  __shared__ __attribute__((aligned(1024))) unsigned char slots[NW * SLOT];
+  constexpr int UNITS = NW * TM * TN;  // 32 x 32 blocks of a tile
+  static_assert(UNITS % 4 == 0, "the wavefronts of a workgroup share a tile");
+  constexpr int SLOT = 32 * (2 * 32 + 16);
+  __shared__ __attribute__((aligned(1024))) unsigned char slots[4 * SLOT];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tile_id = (int)(blockIdx.x / (UNITS / 4)), unit = (int)(blockIdx.x % (UNITS / 4)) * 4 + w;
   int batch, tile_m, tile_n;
-  map_tile(map, batch, tile_m, tile_n);
+  map_tile(map, batch, tile_m, tile_n, tile_id);
   const int m0 = tile_m * BM, n0 = tile_n * BN;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / WN, wn = wave % WN;
+  const int wave = unit / (TM * TN), i = unit / TN % TM, j = unit % TN;
+  const int y0 = m0 + wave / WN * WTM + i * 32, x0 = n0 + wave % WN * WTN + j * 32;
   half_t* const out = a.output + (int64_t)batch * a.stride_oz;
   if (a.mask == ADR_MASK_CAUSAL && n0 > m0 + BM - 1) {
-    fill_masked_tile<BM, BN, NT>(a, out, m0, n0, tid);
+    fill_masked_tile<32, 32, 64>(a, out, y0, x0, lane);
     return;
   }
-  float16_t acc[TM][TN];
+  if (y0 >= a.m || x0 >= a.n) return;
+  const int64_t step = (int64_t)map.total * (TM * TN * 4) * NT;  // float4 between two pieces
+  const float4_t* ws = (const float4_t*)a.workspace + ((int64_t)tile_id * (TM * TN * 4) + (i * TN + j) * 4) * NT +
+                       wave * 64 + lane;
+  float4_t sum[4] = {};
+  int piece = 0;
+  for (; piece + 4 <= map.splits; piece += 4, ws += 4 * step) {
+    float4_t v[4][4];
 #pragma unroll
-  for (int i = 0; i < TM; i++)
+    for (int p = 0; p < 4; p++)
 #pragma unroll
-    for (int j = 0; j < TN; j++)
+      for (int c = 0; c < 4; c++) v[p][c] = ws[p * step + c * NT];
 #pragma unroll
-      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-  for (int piece = 0; piece < map.splits; piece++) {
-    const float4_t* const ws = (const float4_t*)a.workspace +
-                               ((int64_t)piece * map.total + blockIdx.x) * (TM * TN * 4) * NT + tid;
+    for (int p = 0; p < 4; p++)
 #pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-      for (int j = 0; j < TN; j++)
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-          const float4_t v = ws[(int64_t)((i * TN + j) * 4 + c) * NT];
-#pragma unroll
-          for (int e = 0; e < 4; e++) acc[i][j][4 * c + e] += v[e];
-        }
+      for (int c = 0; c < 4; c++) sum[c] += v[p][c];
   }
-  wave_epilogue<TM, 2 * TN>(a, out, acc, m0 + wm * WTM, n0 + wn * WTN, slots + wave * SLOT,
-                        (half_t)a.scale, lane);
+  for (; piece < map.splits; piece++, ws += step) {
+    float4_t v[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) v[c] = ws[c * NT];
+#pragma unroll
+    for (int c = 0; c < 4; c++) sum[c] += v[c];
+  }
+  unsigned char* const slot = slots + w * SLOT;
+  if constexpr (MI16) {
+    float4_t acc[2][2] = {{sum[0], sum[1]}, {sum[2], sum[3]}};
+    wave_epilogue<1, 2>(a, out, acc, y0, x0, slot, (half_t)a.scale, lane);
+  } else {
+    float16_t acc[1][1];
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[0][0][r] = sum[r / 4][r % 4];
+    wave_epilogue<1, 2>(a, out, acc, y0, x0, slot, (half_t)a.scale, lane);
+  }
 }
 
 // =============================================================================================
@@ -2214,18 +2235,20 @@ int64_t split_workspace_bytes(const MatmulArgs& a, int bm, int bn, int splits) {
   return tiles * splits * bm * bn * 4;
 }
 
-template <int BM, int BN, int WM, int WN, int NSTAGE, int MINB>
+template <int BM, int BN, int WM, int WN, int NSTAGE, int MINB, int BK = 64, bool MI16 = false>
 hipError_t launch_dma_split(hipStream_t stream, const MatmulArgs& a, int splits) {
   TileMap map = make_map(a, BM, BN);
   if (map.total < 0 || (int64_t)map.total * splits > 0x7fffffffLL) return hipErrorInvalidConfiguration;
   if (!a.workspace || a.workspace_bytes < split_workspace_bytes(a, BM, BN, splits)) return hipErrorInvalidValue;
   map.splits = splits;
-  hipLaunchKernelGGL((gemm_nt_dma_kernel<BM, BN, WM, WN, NSTAGE, MINB, false, 64, true>),
+  hipLaunchKernelGGL((gemm_nt_dma_kernel<BM, BN, WM, WN, NSTAGE, MINB, false, BK, true, MI16>),
                      dim3((unsigned)(map.total * splits)), dim3(WM * WN * 64), 0, stream, a, map);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((splitk_reduce_kernel<BM, BN, WM, WN>), dim3((unsigned)map.total),
-                     dim3(WM * WN * 64), 0, stream, a, map);
+  constexpr int WGS = BM * BN / (32 * 32) / 4;  // of the second launch per tile
+  if ((int64_t)map.total * WGS > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL((splitk_reduce_kernel<BM, BN, WM, WN, MI16>), dim3((unsigned)(map.total * WGS)), dim3(256), 0,
+                     stream, a, map);
   return hipGetLastError();
 }
 
@@ -2484,38 +2507,28 @@ GemmChoice choose(const MatmulArgs& a) {
 
 // Splitting K over workgroups (needs a workspace): a product with few tiles and a long K keeps
 // most compute units idle while a few walk all of K.  With `splits` workgroups per tile every
-// one of them walks K / splits; a second launch sums the pieces.  The estimate is pick()'s cost
-// (tile area on the busiest compute unit over the tile's efficiency) times K, 2.9e6 units per
-// microsecond, plus the second launch and the fp32 pieces written and read again.
+// one of them walks K / splits; a second launch sums the pieces.
 struct SplitChoice {
   GemmChoice tile;
   int splits;
   int bm, bn;
 };
 
-SplitChoice choose_split(const MatmulArgs& a, int64_t avail_bytes) {
+// Slices of 64 in all of these (K no multiple of 128): the estimate is pick()'s cost (tile area on the
+// busiest compute unit over the tile's efficiency) times K, 2.9e6 units per microsecond, plus the second
+// launch and the fp32 pieces written and read again.
+SplitChoice choose_split_k64(const MatmulArgs& a, int64_t avail_bytes, GemmChoice whole) {
   const SplitChoice none = {GEMM_NONE, 1, 0, 0};
-#ifdef ADR_PHASE_STAMPS
-  return none;  // (the diagnostic build: the workspace argument receives the stamps)
-#endif
-  if (avail_bytes <= 0 || a.rhs_q || a.load != ADR_LOAD_IDENTITY || a.k % 64 != 0 || a.k < 1024)
-    return none;
-  const GemmChoice whole = choose(a);
-  if (whole != DMA_128x128 && whole != DMA_128x64 && whole != DMA_64x64 && whole != DMA_64x64_K128 &&
-      whole != DMA_128x64_K128 && whole != DMA_256x128)
-    return none;
   const int NUM_CU = num_cu();
   double whole_cost;
   pick(a, DMA_TILES, N_DMA_TILES, &whole_cost);
   whole_cost *= a.k;
   // With about one small tile per compute unit the time is set by the latency of the K slices,
-  // not by the tile's arithmetic: 0.38 us per slice of 64 (measured: K4160 N4096 m=130 25.7 us),
-  // 0.25 us where the tile walks K in slices of 128.
+  // not by the tile's arithmetic: 0.38 us per slice of 64 (measured: K4160 N4096 m=130 25.7 us).
   const double US = 2.9e6;
   auto latency_floor = [&](int k, double us_per_slice) { return ((k / 64) * us_per_slice + 2.0) * US; };
   if (whole != DMA_256x128 && whole != DMA_128x128) {
-    const bool k128 = whole == DMA_64x64_K128 || whole == DMA_128x64_K128;
-    const double f = latency_floor(a.k, k128 ? 0.25 : 0.38);
+    const double f = latency_floor(a.k, 0.38);
     if (f > whole_cost) whole_cost = f;
   }
   static const Candidate tiles[] = {{DMA_128x128, 128, 128, 2, 0.80f}, {DMA_128x64, 128, 64, 2, 0.60f},
@@ -2537,6 +2550,70 @@ SplitChoice choose_split(const MatmulArgs& a, int64_t avail_bytes) {
       const double extra = (4.0 + 2.0 * (double)bytes / 4.0e6) * US;
       if (mm + extra < best_cost) {
         best_cost = mm + extra;
+        best = {t.id, sp, t.bm, t.bn};
+      }
+    }
+  }
+  return best;
+}
+
+// K a multiple of 128.  Both times are estimated in microseconds, from 700 (tile, pieces) forced on 60
+// products (K 1024 .. 13824, N 768 .. 12288, m 64 .. 2056, weights from HBM):
+//   split: 5.3 + 1.4 per round + a slice's time on the busiest compute unit + 0.28 per MB of partial
+//          sums (written and read) + 0.067 per MB of weights
+//   whole: 4.5 + a slice's time, which falls with the tiles in flight and with weights that a cache holds
+// The pieces it picks are the fastest forced ones or within 2 % on 50 of the 60 and 7 % behind at worst; against
+// the unsplit launch it takes a split where that is 5 % ahead by the estimates.  (K11008 N4096, us, before the
+// second launch was spread over the chip and the 256-row tiles could split -> now: m=128 37 -> 30, 256 45 -> 39,
+// 512 67 -> 54, 640 101 -> 71, 768 101 -> 79, 1024 104 -> 88; K13824 N5120 m=512 124 -> 74; K4096 N4096 m=96
+// 18.7 -> 16.0; K5120 N1280 m=100 23.3 -> 11.5.)
+SplitChoice choose_split(const MatmulArgs& a, int64_t avail_bytes) {
+  const SplitChoice none = {GEMM_NONE, 1, 0, 0};
+#ifdef ADR_PHASE_STAMPS
+  return none;  // (the diagnostic build: the workspace argument receives the stamps)
+#endif
+  if (avail_bytes <= 0 || a.rhs_q || a.load != ADR_LOAD_IDENTITY || a.k % 64 != 0 || a.k < 1024)
+    return none;
+  const GemmChoice whole = choose(a);
+  const int NUM_CU = num_cu();
+  if (a.k % 128 != 0)
+    return whole == DMA_128x128 || whole == DMA_128x64 || whole == DMA_64x64 || whole == DMA_256x128
+               ? choose_split_k64(a, avail_bytes, whole) : none;
+  // us per slice of 64 with every compute unit busy and weights from HBM; the share of it that is left when
+  // few tiles are in flight (`alone`); the rest goes with the tiles (three quarters on the large tiles)
+  // and, a quarter of the whole, with the weights that must come from HBM
+  struct Whole { GemmChoice id; int bm, bn; double us, alone; };
+  static const Whole wholes[] = {{DMA_64x64, 64, 64, 0.26, 0.40}, {DMA_64x64_K128, 64, 64, 0.26, 0.40},
+                                 {DMA_128x64, 128, 64, 0.35, 0.40}, {DMA_128x64_K128, 128, 64, 0.35, 0.40},
+                                 {DMA_128x128, 128, 128, 0.565, 0.23}, {DMA_128x192, 128, 192, 0.75, 0.23},
+                                 {DMA_256x128, 256, 128, 0.84, 0.23}};
+  auto tiles_of = [&](int bm, int bn) { return (int64_t)((a.m + bm - 1) / bm) * ((a.n + bn - 1) / bn) * a.batches; };
+  const double weights_mb = 2e-6 * a.k * a.n * a.batches, slices = a.k / 64;
+  double limit = 0;
+  for (const Whole& w : wholes)
+    if (w.id == whole) {
+      const int64_t nt = tiles_of(w.bm, w.bn), rounds = (nt + NUM_CU - 1) / NUM_CU;
+      const double busy = nt < NUM_CU ? (double)nt / NUM_CU : 1.0, cold = weights_mb < 32 ? weights_mb / 32 : 1.0;
+      limit = 0.95 * (4.5 + rounds * slices * w.us * (w.alone + (0.75 - w.alone) * busy + 0.25 * cold));
+    }
+  const double least = 6.7 + 0.067 * weights_mb;
+  if (least >= limit) return none;  // (as for most products: no host time for the search)
+  struct Piece { GemmChoice id; int bm, bn; double us; };
+  static const Piece pieces[] = {{DMA_64x64_K128, 64, 64, 0.19}, {DMA_128x64_K128, 128, 64, 0.296},
+                                 {DMA_128x128, 128, 128, 0.439}, {DMA_128x256, 128, 256, 0.766},
+                                 {DMA_256x128, 256, 128, 0.659}};
+  SplitChoice best = none;
+  for (const Piece& t : pieces) {
+    const int64_t nt = tiles_of(t.bm, t.bn);
+    for (int sp = 2; sp <= 16; sp++) {
+      if (a.k / sp < 256) break;  // at least four slices per piece
+      if (nt * sp > 4 * (int64_t)NUM_CU) break;
+      const int64_t bytes = nt * sp * t.bm * t.bn * 4;
+      if (bytes > avail_bytes) break;
+      const int64_t rounds = (nt * sp + NUM_CU - 1) / NUM_CU;
+      const double us = least - 1.4 + rounds * (1.4 + (a.k / 64 + sp - 1) / sp * t.us) + 0.28e-6 * bytes;
+      if (us < limit) {
+        limit = us;
         best = {t.id, sp, t.bm, t.bn};
       }
     }
@@ -2660,26 +2737,24 @@ static bool split_m_tail(const MatmulArgs& a, MatmulArgs& head, MatmulArgs& tail
   return (first + rest) * a.k + 8.7e6 < whole * a.k;
 }
 
+// "gemm_nt_mfma_dma_128x128x64_splitk4": the tile, then the number of pieces
 static const char* split_name(const SplitChoice& sc) {
-  // "gemm_nt_mfma_dma_128x128x64_splitk4": the tile, then the number of pieces
-  static const char* const names[3][15] = {
-      {"gemm_nt_mfma_dma_128x128x64_splitk2", "gemm_nt_mfma_dma_128x128x64_splitk3", "gemm_nt_mfma_dma_128x128x64_splitk4",
-       "gemm_nt_mfma_dma_128x128x64_splitk5", "gemm_nt_mfma_dma_128x128x64_splitk6", "gemm_nt_mfma_dma_128x128x64_splitk7",
-       "gemm_nt_mfma_dma_128x128x64_splitk8", "gemm_nt_mfma_dma_128x128x64_splitk9", "gemm_nt_mfma_dma_128x128x64_splitk10",
-       "gemm_nt_mfma_dma_128x128x64_splitk11", "gemm_nt_mfma_dma_128x128x64_splitk12", "gemm_nt_mfma_dma_128x128x64_splitk13",
-       "gemm_nt_mfma_dma_128x128x64_splitk14", "gemm_nt_mfma_dma_128x128x64_splitk15", "gemm_nt_mfma_dma_128x128x64_splitk16"},
-      {"gemm_nt_mfma_dma_128x64x64_splitk2", "gemm_nt_mfma_dma_128x64x64_splitk3", "gemm_nt_mfma_dma_128x64x64_splitk4",
-       "gemm_nt_mfma_dma_128x64x64_splitk5", "gemm_nt_mfma_dma_128x64x64_splitk6", "gemm_nt_mfma_dma_128x64x64_splitk7",
-       "gemm_nt_mfma_dma_128x64x64_splitk8", "gemm_nt_mfma_dma_128x64x64_splitk9", "gemm_nt_mfma_dma_128x64x64_splitk10",
-       "gemm_nt_mfma_dma_128x64x64_splitk11", "gemm_nt_mfma_dma_128x64x64_splitk12", "gemm_nt_mfma_dma_128x64x64_splitk13",
-       "gemm_nt_mfma_dma_128x64x64_splitk14", "gemm_nt_mfma_dma_128x64x64_splitk15", "gemm_nt_mfma_dma_128x64x64_splitk16"},
-      {"gemm_nt_mfma_dma_64x64x64_splitk2", "gemm_nt_mfma_dma_64x64x64_splitk3", "gemm_nt_mfma_dma_64x64x64_splitk4",
-       "gemm_nt_mfma_dma_64x64x64_splitk5", "gemm_nt_mfma_dma_64x64x64_splitk6", "gemm_nt_mfma_dma_64x64x64_splitk7",
-       "gemm_nt_mfma_dma_64x64x64_splitk8", "gemm_nt_mfma_dma_64x64x64_splitk9", "gemm_nt_mfma_dma_64x64x64_splitk10",
-       "gemm_nt_mfma_dma_64x64x64_splitk11", "gemm_nt_mfma_dma_64x64x64_splitk12", "gemm_nt_mfma_dma_64x64x64_splitk13",
-       "gemm_nt_mfma_dma_64x64x64_splitk14", "gemm_nt_mfma_dma_64x64x64_splitk15", "gemm_nt_mfma_dma_64x64x64_splitk16"}};
-  const int t = sc.tile == DMA_128x128 ? 0 : sc.tile == DMA_128x64 ? 1 : 2;
-  return names[t][sc.splits - 2];
+  static const GemmChoice tiles[] = {DMA_64x64, DMA_64x64_K128, DMA_128x64, DMA_128x64_K128, DMA_128x128, DMA_128x256, DMA_256x128};
+  constexpr int N = sizeof(tiles) / sizeof(tiles[0]);
+  struct Names { char of[N][17][48]; };
+  static const Names names = [] {
+    Names t;
+    for (int i = 0; i < N; i++)
+      for (int sp = 0; sp <= 16; sp++) {
+        const char* tile = "";
+        choice_name(tiles[i], &tile);
+        snprintf(t.of[i][sp], sizeof(t.of[i][sp]), "%s_splitk%d", tile, sp);
+      }
+    return t;
+  }();
+  int i = 0;
+  while (i + 1 < N && tiles[i] != sc.tile) i++;
+  return names.of[i][sc.splits];
 }
 
 int64_t mfma_gemm_workspace_bytes(const MatmulArgs& a, int64_t avail) {
@@ -2700,9 +2775,16 @@ bool mfma_gemm_supported(const MatmulArgs& a, const char** name) {
 
 hipError_t launch_mfma_gemm(hipStream_t stream, const MatmulArgs& a) {
   const SplitChoice sc = choose_split(a, a.workspace ? a.workspace_bytes : 0);
-  if (sc.tile == DMA_128x128) return launch_dma_split<128, 128, 2, 2, 3, 1>(stream, a, sc.splits);
-  if (sc.tile == DMA_128x64) return launch_dma_split<128, 64, 2, 2, 3, 2>(stream, a, sc.splits);
-  if (sc.tile == DMA_64x64) return launch_dma_split<64, 64, 2, 2, 3, 3>(stream, a, sc.splits);
+  switch (sc.tile) {
+    case DMA_256x128: return launch_dma_split<256, 128, 4, 2, 7, 1, 64, true>(stream, a, sc.splits);
+    case DMA_128x256: return launch_dma_split<128, 256, 2, 4, 3, 1, 64, true>(stream, a, sc.splits);
+    case DMA_128x128: return launch_dma_split<128, 128, 4, 2, 7, 1, 64, true>(stream, a, sc.splits);
+    case DMA_128x64_K128: return launch_dma_split<128, 64, 2, 2, 3, 1, 128>(stream, a, sc.splits);
+    case DMA_64x64_K128: return launch_dma_split<64, 64, 2, 2, 3, 1, 128>(stream, a, sc.splits);
+    case DMA_128x64: return launch_dma_split<128, 64, 2, 2, 3, 2>(stream, a, sc.splits);
+    case DMA_64x64: return launch_dma_split<64, 64, 2, 2, 3, 3>(stream, a, sc.splits);
+    default: break;
+  }
   MatmulArgs head, tail;
   if (split_m_tail(a, head, tail)) {
     const hipError_t e = launch_choice(stream, head, choose(head));

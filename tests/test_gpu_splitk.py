@@ -189,3 +189,47 @@ def test_workspace_contract(ws):
     ws2 = torch.zeros(ws.numel(), dtype=torch.uint8, device="cuda")
     assert call_ws(fresh, a[:m2], w, 1, m2, K, N, so2, sl2, sr2, ws2) == 0
     assert torch.equal(second, fresh)
+
+
+@pytest.mark.parametrize("store", [(0, "identity"), (5, "add"), (3, "beta_bias")], ids=lambda s: s[1])
+@pytest.mark.parametrize("case", [(500, 11008, 4100, "256x128x64"), (330, 11008, 4100, "128x256x64"),
+                                  (100, 11008, 4097, "128x128x64"), (100, 4096, 4104, "128x64x128"),
+                                  (70, 4096, 1001, "64x64x128")], ids=lambda c: c[3])
+def test_split_k_tiles_of_k_multiples_of_128(ws, case, store):
+    """The tiles that products with K % 128 == 0 split on, and the second launch's 32 x 32 blocks in both
+    accumulator layouts: a last tile row and column that the matrix only begins to fill, pieces of unequal
+    length, result rows aligned to 16, 8 and 2 bytes.  Dyadic inputs: every sum and every store is one
+    rounding of the float64 value."""
+    M, K, N, tile = case
+    op, _ = store
+    so, sl, sr = nt(M, K, N)
+    assert ("_dma_" + tile + "_splitk") in ws_plan(1, M, K, N, so, sl, sr, store=op, ws_bytes=ws.numel())
+    gen = torch.Generator(device="cuda").manual_seed(4500 + M + op)
+    a = (torch.randint(-4, 5, (M, K), generator=gen, device="cuda") / 8.0).half()
+    w = (torch.randint(-4, 5, (N, K), generator=gen, device="cuda") / 8.0).half()
+    prev = (torch.randint(-8, 9, (M, N), generator=gen, device="cuda") / 4.0).half()
+    bias = (torch.randint(-8, 9, (N,), generator=gen, device="cuda") / 4.0).half()
+    out = prev.clone()
+    assert call_ws(out, a, w, 1, M, K, N, so, sl, sr, ws, bias_t=bias, beta=0.5, store=op) == 0
+    got = (a.double() @ w.double().t()).half()
+    # (the operators work on the narrowed sum, in fp16 steps: identity, sum + prev, sum + 0.5 * prev + bias)
+    want = got if op == 0 else got + prev if op == 5 else (got.float() + bias.float() + 0.5 * prev.float()).half()
+    bad = (out != want).nonzero()
+    assert bad.numel() == 0, (bad[:5].tolist(), out[tuple(bad[0])].item(), want[tuple(bad[0])].item())
+
+
+def test_split_k_causal_mask_on_16x16_accumulators(ws):
+    """Batches and the causal mask through the second launch of a tile on 16x16x32 MFMAs: blocks above the
+    diagonal of a tile nothing was written for, of one that was, and on the diagonal."""
+    B, M, K, N = 4, 300, 8192, 700
+    so, sl, sr = (1, N, M * N), (1, K, M * K), (K, 1, N * K)
+    assert "_dma_128x128x64_splitk" in ws_plan(B, M, K, N, so, sl, sr, store=4, mask=1, ws_bytes=ws.numel())
+    gen = torch.Generator(device="cuda").manual_seed(4600)
+    a = (torch.randint(-4, 5, (B, M, K), generator=gen, device="cuda") / 8.0).half()
+    w = (torch.randint(-4, 5, (B, N, K), generator=gen, device="cuda") / 8.0).half()
+    out = torch.full((B, M, N), 7.0, dtype=torch.float16, device="cuda")
+    assert call_ws(out, a, w, B, M, K, N, so, sl, sr, ws, scale=0.125, store=4, mask=1) == 0
+    want = torch.stack([(a[b].double() @ w[b].double().t()).half() * 0.125 for b in range(B)])
+    above = torch.arange(N, device="cuda")[None, :] > torch.arange(M, device="cuda")[:, None]
+    want.masked_fill_(above[None], float("-inf"))
+    assert torch.equal(out, want)
