@@ -38,6 +38,7 @@ struct MatmulArgs {
   // partial tiles, fully rewritten by every launch that uses them; null / 0: no such kernel
   float* workspace;
   int64_t workspace_bytes;
+  int split;  // the choice mfma_gemm_workspace_bytes made for this call (0: none made yet), so that it is made once
 };
 
 // Internal store operator of the contiguous NT entry points (matmul_nt_wmma_16x128x256.cu:63-66):
@@ -310,7 +311,7 @@ hipError_t launch_mfma_gemm(hipStream_t stream, const MatmulArgs& a);
 // Scratch bytes the split-K form of these arguments would use when at most `avail` bytes can be
 // had (0: no split pays here, or none fits); the kernel family splits that way when a.workspace
 // holds at least this much.
-int64_t mfma_gemm_workspace_bytes(const MatmulArgs& a, int64_t avail = INT64_MAX);
+int64_t mfma_gemm_workspace_bytes(MatmulArgs& a, int64_t avail = INT64_MAX);
 // fp16 skinny matmul (m <= 32, K-contiguous operands): true when a streaming kernel covers it.
 bool gemv_f16_supported(const MatmulArgs& a, const char** name);
 hipError_t launch_gemv_f16(hipStream_t stream, const MatmulArgs& a);

@@ -40,6 +40,8 @@
 // the way.
 #include <stdint.h>
 #include <stdio.h>
+
+#include <algorithm>
 #include <type_traits>
 
 #include "adr_common.hpp"
@@ -2562,18 +2564,18 @@ SplitChoice choose_split_k64(const MatmulArgs& a, int64_t avail_bytes, GemmChoic
 //   split: 5.3 + 1.4 per round + a slice's time on the busiest compute unit + 0.28 per MB of partial
 //          sums (written and read) + 0.067 per MB of weights
 //   whole: 4.5 + a slice's time, which falls with the tiles in flight and with weights that a cache holds
-// The pieces it picks are the fastest forced ones or within 2 % on 50 of the 60 and 7 % behind at worst; against
-// the unsplit launch it takes a split where that is 5 % ahead by the estimates.  (K11008 N4096, us, before the
-// second launch was spread over the chip and the 256-row tiles could split -> now: m=128 37 -> 30, 256 45 -> 39,
-// 512 67 -> 54, 640 101 -> 71, 768 101 -> 79, 1024 104 -> 88; K13824 N5120 m=512 124 -> 74; K4096 N4096 m=96
-// 18.7 -> 16.0; K5120 N1280 m=100 23.3 -> 11.5.)
-SplitChoice choose_split(const MatmulArgs& a, int64_t avail_bytes) {
+// The pieces it picks are the fastest forced ones or within 2 % on 50 of the 60 and 7 % behind at worst.  A split is
+// taken where it is 5 % ahead by the estimates on weights that no cache holds (32 MB and more), 17 % on small
+// ones, which a caller may find in a cache: there the unsplit launch gains more (M2056 K4096 N1024, a model's
+// MLP behind its other product: 56 us unsplit and 64 split with 165 MB in use in all, 62 and 68 with 900).
+// us, before the second launch was spread over the chip and the large tiles could split -> now, weights from
+// HBM: K11008 N4096 m=128 37 -> 31, 256 45 -> 41, 512 67 -> 55, 640 101 -> 71, 768 101 -> 81, 1024 105 -> 89;
+// K13824 N5120 m=512 124 -> 77; K4096 N4096 m=96 18.7 -> 16.0; K5120 N1280 m=100 23.3 -> 11.5.
+SplitChoice search_split(const MatmulArgs& a, int64_t avail_bytes) {
   const SplitChoice none = {GEMM_NONE, 1, 0, 0};
 #ifdef ADR_PHASE_STAMPS
   return none;  // (the diagnostic build: the workspace argument receives the stamps)
 #endif
-  if (avail_bytes <= 0 || a.rhs_q || a.load != ADR_LOAD_IDENTITY || a.k % 64 != 0 || a.k < 1024)
-    return none;
   const GemmChoice whole = choose(a);
   const int NUM_CU = num_cu();
   if (a.k % 128 != 0)
@@ -2583,7 +2585,7 @@ SplitChoice choose_split(const MatmulArgs& a, int64_t avail_bytes) {
   // few tiles are in flight (`alone`); the rest goes with the tiles (three quarters on the large tiles)
   // and, a quarter of the whole, with the weights that must come from HBM
   struct Whole { GemmChoice id; int bm, bn; double us, alone; };
-  static const Whole wholes[] = {{DMA_64x64, 64, 64, 0.26, 0.40}, {DMA_64x64_K128, 64, 64, 0.26, 0.40},
+  static const Whole wholes[] = {{DMA_64x64, 64, 64, 0.26, 0.55}, {DMA_64x64_K128, 64, 64, 0.26, 0.55},
                                  {DMA_128x64, 128, 64, 0.35, 0.40}, {DMA_128x64_K128, 128, 64, 0.35, 0.40},
                                  {DMA_128x128, 128, 128, 0.565, 0.23}, {DMA_128x192, 128, 192, 0.75, 0.23},
                                  {DMA_256x128, 256, 128, 0.84, 0.23}};
@@ -2594,7 +2596,7 @@ SplitChoice choose_split(const MatmulArgs& a, int64_t avail_bytes) {
     if (w.id == whole) {
       const int64_t nt = tiles_of(w.bm, w.bn), rounds = (nt + NUM_CU - 1) / NUM_CU;
       const double busy = nt < NUM_CU ? (double)nt / NUM_CU : 1.0, cold = weights_mb < 32 ? weights_mb / 32 : 1.0;
-      limit = 0.95 * (4.5 + rounds * slices * w.us * (w.alone + (0.75 - w.alone) * busy + 0.25 * cold));
+      limit = (0.83 + 0.12 * cold) * (4.5 + rounds * slices * w.us * (w.alone + (0.75 - w.alone) * busy + 0.25 * cold));
     }
   const double least = 6.7 + 0.067 * weights_mb;
   if (least >= limit) return none;  // (as for most products: no host time for the search)
@@ -2605,12 +2607,12 @@ SplitChoice choose_split(const MatmulArgs& a, int64_t avail_bytes) {
   SplitChoice best = none;
   for (const Piece& t : pieces) {
     const int64_t nt = tiles_of(t.bm, t.bn);
-    for (int sp = 2; sp <= 16; sp++) {
-      if (a.k / sp < 256) break;  // at least four slices per piece
-      if (nt * sp > 4 * (int64_t)NUM_CU) break;
+    if (2 * nt > 4 * (int64_t)NUM_CU) continue;
+    const int most = std::min(std::min(16, a.k / 256), (int)(4 * NUM_CU / nt));  // at least four slices per piece
+    for (int sp = 2; sp <= most; sp++) {
       const int64_t bytes = nt * sp * t.bm * t.bn * 4;
       if (bytes > avail_bytes) break;
-      const int64_t rounds = (nt * sp + NUM_CU - 1) / NUM_CU;
+      const int rounds = ((int)nt * sp + NUM_CU - 1) / NUM_CU;
       const double us = least - 1.4 + rounds * (1.4 + (a.k / 64 + sp - 1) / sp * t.us) + 0.28e-6 * bytes;
       if (us < limit) {
         limit = us;
@@ -2619,6 +2621,15 @@ SplitChoice choose_split(const MatmulArgs& a, int64_t avail_bytes) {
     }
   }
   return best;
+}
+
+SplitChoice choose_split(const MatmulArgs& a, int64_t avail_bytes) {
+  const SplitChoice none = {GEMM_NONE, 1, 0, 0};
+  if (avail_bytes <= 0 || a.rhs_q || a.load != ADR_LOAD_IDENTITY || a.k % 64 != 0 || a.k < 1024)
+    return none;
+  if (a.split == 0) return search_split(a, avail_bytes);
+  const SplitChoice made = {(GemmChoice)(a.split >> 24), a.split & 0xff, (a.split >> 16 & 0xff) * 32, (a.split >> 8 & 0xff) * 32};
+  return made.tile == GEMM_NONE || split_workspace_bytes(a, made.bm, made.bn, made.splits) > avail_bytes ? none : made;
 }
 
 }  // namespace
@@ -2757,8 +2768,9 @@ static const char* split_name(const SplitChoice& sc) {
   return names.of[i][sc.splits];
 }
 
-int64_t mfma_gemm_workspace_bytes(const MatmulArgs& a, int64_t avail) {
+int64_t mfma_gemm_workspace_bytes(MatmulArgs& a, int64_t avail) {
   const SplitChoice sc = choose_split(a, avail);
+  a.split = (int)sc.tile << 24 | sc.bm / 32 << 16 | sc.bn / 32 << 8 | sc.splits;
   return sc.tile == GEMM_NONE ? 0 : split_workspace_bytes(a, sc.bm, sc.bn, sc.splits);
 }
 
