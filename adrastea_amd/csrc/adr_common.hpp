@@ -346,6 +346,7 @@ struct AttentionPlan {
   bool tile;   // attention_tile_kernel
   bool wide;   // 64-bit addresses (attention_fwd_kernel)
   int groups;  // of four wavefronts (attention_fwd_kernel)
+  bool two_rounds;  // two groups and more workgroups than compute units: heavy blocks first
   int splits;
   int cus;
   int64_t workspace_bytes;

@@ -1032,6 +1032,13 @@ AttentionPlan attention_plan(const AttentionShape& t, int cus, int64_t avail) {
   // which pays from six tiles on (20 heads of 64, 1500 x 1500: 25.3 -> 21.2 us, 12 x 1000 causal
   // 15.3 -> 12.7; 12 x 256 6.2 -> 6.3).
   p.groups = !p.rows && !p.wide && blocks <= cus && n > 5 * BN ? 2 : 1;
+  // Under the mask also with up to half as many blocks again, from 1024 keys on: the heavy blocks start first and
+  // the light ones fill in behind them, and none is left to a single group alone on its unit (us, one
+  // group / two: 32 heads of 128, 1100 24.9 / 22.1, 1280 26.6 / 23.4, 1500 29.8 / 28.1; 20 of 64, 1700 22.1 / 17.6,
+  // 2048 25.1 / 21.1).  With more blocks the second round is as long as what it saves (32 heads, 2048 43.8 / 42.9, 40
+  // heads, 1300 28.0 / 29.5, 1600 36.9 / 40.8), with fewer keys the merges are (64 heads, 513 13.6 / 16.6).
+  p.two_rounds = !p.rows && !p.wide && t.mask == ADR_MASK_CAUSAL && blocks > cus && 2 * blocks <= 3 * (int64_t)cus && n >= 1024;
+  if (p.two_rounds) p.groups = 2;
   p.splits = 1;
   // Times beyond what every launch takes, in us, fitted to 40 shapes of 12-40 heads, 1-448 query rows
   // and 64-8192 keys with every number of parts: the rows kernel reads 69 GB/s per compute unit; parts
@@ -1043,7 +1050,7 @@ AttentionPlan attention_plan(const AttentionShape& t, int cus, int64_t avail) {
     if (p.rows) {
       us = ceil((double)t.heads * s / cus) * keys * t.d * (4.0 / 69e3);
       if (s > 1) us += 4.0;
-    } else if (s == 1 && p.groups == 2) {
+    } else if (s == 1 && p.groups == 2 && !p.two_rounds) {
       us = keys * 0.0095 + 0.5;
     } else {
       us = ceil((double)blocks * s / cus) * keys * 0.014;
@@ -1057,7 +1064,7 @@ AttentionPlan attention_plan(const AttentionShape& t, int cus, int64_t avail) {
     // 10.0; 500 9.9, 10.0; 640 10.9, 9.9).
     if (!p.rows && s == 1 && us < 5.5) break;
   }
-  if (p.splits > 1) p.groups = 1;
+  if (p.splits > 1) p.groups = 1, p.two_rounds = false;
   p.workspace_bytes = p.splits > 1 ? p.splits * part : 0;
   return p;
 }
@@ -1091,7 +1098,7 @@ hipError_t launch_attention(hipStream_t stream, half_t* out, const half_t* q, co
   a.part_o = (float*)workspace;
   a.part_ml = (float2*)((float*)workspace + (a.splits > 1 ? a.splits * rows * t.d : 0));
   a.qblocks = (t.m + BM - 1) / BM;
-  a.upper = (int64_t)t.heads * a.qblocks * a.splits <= 2 * p.cus ? (a.qblocks + 1) / 2 : a.qblocks;
+  a.upper = !p.two_rounds && (int64_t)t.heads * a.qblocks * a.splits <= 2 * p.cus ? (a.qblocks + 1) / 2 : a.qblocks;
   // (parts are shared only where their rows can be counted: no product here runs over)
   if ((int64_t)t.heads * a.qblocks * a.splits > 0x7fffffffLL) return hipErrorInvalidConfiguration;
   if (t.d == 128) attention_launches<128>(stream, a, p);

@@ -87,6 +87,14 @@ def test_two_groups_of_wavefronts(d, n):
     run(2, 130, n, d, False)
 
 
+@pytest.mark.parametrize("heads,m,n,d", [(29, 1025, 1025, 128), (33, 1024, 1024, 64), (26, 1410, 1410, 64), (32, 1100, 1030, 64),
+                                         (40, 1101, 1300, 128)])
+def test_two_groups_of_wavefronts_in_a_second_round(heads, m, n, d):
+    """Under the mask with up to half as many query blocks again as compute units (261 ... 384 of 256 here), from
+    1024 keys that some row sees on; heads that do and do not divide by the dies, and a few rows past a block."""
+    run(heads, m, n, d, True)
+
+
 @pytest.mark.parametrize("heads,m,n,d", [(4, 1, 2048, 128), (4, 1, 2047, 128), (3, 16, 3001, 64), (5, 9, 4100, 64),
                                          (1, 40, 2000, 128), (2, 130, 1500, 64), (1, 17, 8192, 128)])
 def test_keys_shared_by_workgroups(heads, m, n, d):
