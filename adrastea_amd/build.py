@@ -12,6 +12,7 @@ import concurrent.futures
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -144,7 +145,28 @@ def build_host_test(force: bool = False) -> str:
     return HOST_TEST_BIN
 
 
+NATIVE_SRC = os.path.join(HERE, "host", "native.cpp")
+NATIVE_MODULE = os.path.join(HERE, "_native" + sysconfig.get_config_var("EXT_SUFFIX"))
+
+
+def build_native_module(force: bool = False) -> str:
+    """Compiles the native host path (host/native.cpp) with g++ as the CPython module adrastea_amd._native.
+    It calls the library through addresses handed to it, and links nothing of HIP."""
+    deps = [NATIVE_SRC, os.path.join(os.path.dirname(HERE), "include", "adrastea_kernels.h")]
+    if (not force and os.path.exists(NATIVE_MODULE)
+            and all(os.path.getmtime(d) <= os.path.getmtime(NATIVE_MODULE) for d in deps)):
+        return NATIVE_MODULE
+    cmd = ["g++", "-std=c++17", "-O2", "-Wall", "-Wno-missing-field-initializers", "-fPIC", "-shared", "-fvisibility=hidden",
+           "-I" + sysconfig.get_paths()["include"], "-o", NATIVE_MODULE + ".new", NATIVE_SRC]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for {NATIVE_SRC}:\n{r.stdout}\n{r.stderr}")
+    os.replace(NATIVE_MODULE + ".new", NATIVE_MODULE)  # (this process may have the old one mapped)
+    return NATIVE_MODULE
+
+
 if __name__ == "__main__":
+    print(build_native_module(force="--force" in sys.argv))
     print(build_library(force="--force" in sys.argv))
     print(build_stamps_library(force="--force" in sys.argv))
     print(build_legacy_modules(force="--force" in sys.argv))

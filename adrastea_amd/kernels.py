@@ -17,7 +17,7 @@ from dataclasses import dataclass, field
 from typing import Optional, Tuple
 
 from . import _ffi
-from .tensor import TensorLayout, TensorView
+from .tensor import TensorLayout, TensorView, _native
 
 
 class AdrasteaError(RuntimeError):
@@ -183,8 +183,15 @@ def _current_stream() -> int:
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
+_NATIVE_CALLS = ("adr_matmul_f16", "adr_attention_f16", "adr_softmax_rows", "adr_matmul_nt_fp16u8",
+                 "adr_quantize_absmax_u8", "adr_dequantize_absmax_u8", "adr_error_stats_f16", "adr_error_stats_f32")
+
+
 class GpuKernels(CommonKernels):
     """Launches through the C ABI on torch's current HIP stream.
+
+    Where host/native.cpp is built, the calls below are lowered by it; what it does not take (it
+    returns None) goes the way written out here, which is also the definition of what it does.
 
     `workspace_bytes` > 0 gives the instance a scratch buffer of that size, owned like any other
     tensor of the host (in the reference: one more GpuBuffer held by GpuKernels); matmul_f16 then
@@ -201,6 +208,19 @@ class GpuKernels(CommonKernels):
             raise RuntimeError("adrastea_amd.GpuKernels needs a GPU; there is no CPU fallback")
         self._workspace = (torch.empty(workspace_bytes, dtype=torch.uint8, device="cuda")
                            if workspace_bytes > 0 else None)
+        if _native is not None:
+            _native.bind(*(C.cast(getattr(self._lib, name), C.c_void_p).value for name in _NATIVE_CALLS),
+                         torch.cuda.current_device, torch._C._cuda_getCurrentRawStream)
+
+    @staticmethod
+    def _lowered(name, *args) -> bool:
+        """The call as native code; False: it has to go the general way."""
+        if _native is None:
+            return False
+        rc = getattr(_native, name)(*args)
+        if rc:
+            raise AdrasteaError(rc, name)
+        return rc == 0
 
     def _matmul(self, fn, what, output, left, right, options):
         scalars, tail = _lower(output.layout, left.layout, right.layout, options)
@@ -212,6 +232,8 @@ class GpuKernels(CommonKernels):
 
     def matmul_f16(self, output, left, right, options=MatmulOptions()):
         if self._workspace is None:
+            if self._lowered("matmul_f16", output, left, right, options):
+                return
             return self._matmul(self._lib.adr_matmul_f16, "matmul_f16", output, left, right, options)
         ws = self._workspace
 
@@ -226,6 +248,8 @@ class GpuKernels(CommonKernels):
     def softmax_rows_inplace(self, output, temperature: float = 1.0):
         """kernels.rs:892-915: rows = size(-2), heads = size(-3) (1 for rank 2), width size(-1);
         like the reference's kernel, the tensor is taken to be contiguous."""
+        if self._lowered("softmax_rows_inplace", output, temperature):
+            return
         lay = output.layout
         assert lay == TensorLayout.row_major(list(lay.dims)), "softmax_rows needs a contiguous view"
         heads = lay.size(-3) if len(lay.dims) > 2 else 1
@@ -241,6 +265,8 @@ class GpuKernels(CommonKernels):
         [heads, m, d] views, `key`/`value` [heads, n, d] views (rank 2 = one head).  Raises
         AdrasteaError with code ADR_EUNSUPPORTED_LAYOUT for head dimensions or strides the fused
         kernel does not cover; the three-call sequence remains available for those."""
+        if self._workspace is None and self._lowered("attention_f16", output, query, key, value, scale, temperature, mask):
+            return
         lo, lq, lk, lv = output.layout, query.layout, key.layout, value.layout
         do, dq, dk, dv = lo.dims, lq.dims, lk.dims, lv.dims
         so, sq, sk, sv = lo.strides, lq.strides, lk.strides, lv.strides
@@ -263,6 +289,12 @@ class GpuKernels(CommonKernels):
             raise AdrasteaError(rc, "attention_f16")
 
     def _error_stats(self, fn, what, output, lhs, rhs):
+        if _native is not None:
+            rc = _native.error_stats(output, lhs, rhs, int(what == "error_stats_f32"))
+            if rc:
+                raise AdrasteaError(rc, what)
+            if rc == 0:
+                return
         # kernels.rs:717-751: both operands flattened with shape_cast(&[-1]); equal lengths
         lhs, rhs = lhs.shape_cast([-1]), rhs.shape_cast([-1])
         assert lhs.size(-1) == rhs.size(-1)
@@ -288,6 +320,8 @@ class GpuKernels(CommonKernels):
             raise AdrasteaError(rc, "matmul_nt_f16")
 
     def matmul_nt_fp16u8(self, output, lhs, rhs_q, scales, block_size: int, beta: float = 0.0):
+        if self._workspace is None and self._lowered("matmul_nt_fp16u8", output, lhs, rhs_q, scales, block_size, beta):
+            return
         m, p = lhs.shape
         n = rhs_q.shape[0]
         assert rhs_q.shape[1] == p and tuple(output.shape) == (m, n)
@@ -308,6 +342,8 @@ class GpuKernels(CommonKernels):
             raise AdrasteaError(rc, "matmul_nt_fp16u8")
 
     def dequantize_absmax_uint8(self, output, scales, q):
+        if self._lowered("dequantize_absmax_uint8", output, scales, q):
+            return
         rows, cols = q.shape
         block_size = cols // scales.shape[1]
         rc = self._lib.adr_dequantize_absmax_u8(_current_stream(), output.data_ptr(),
@@ -317,6 +353,8 @@ class GpuKernels(CommonKernels):
             raise AdrasteaError(rc, "dequantize_absmax_uint8")
 
     def quantize_absmax_uint8(self, q, scales, x):
+        if self._lowered("quantize_absmax_uint8", q, scales, x):
+            return
         rows, cols = x.shape
         block_size = cols // scales.shape[1]
         rc = self._lib.adr_quantize_absmax_u8(_current_stream(), q.data_ptr(), scales.data_ptr(),

@@ -142,3 +142,11 @@ class TensorView:
 
     def take(self, sizes) -> "TensorView":
         return TensorView(self.storage, self.layout.take(sizes), self.offset)
+
+
+try:  # the same three methods as native code (host/native.cpp), where it is built
+    from . import _native
+except ImportError:
+    _native = None
+if _native is not None:
+    _native.install(TensorLayout, TensorView)
