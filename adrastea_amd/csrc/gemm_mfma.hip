@@ -1089,33 +1089,7 @@ struct ShortKMap {
   int tiles_m, tiles_n, rows;   // rows = batches * tiles_m
   int seg, segs_per_row, units; // a unit is `seg` consecutive tiles of one tile row
   int xcds;                     // dies of the device
-  int prefilled;                // the tiles above the diagonal of a causal product are written
 };
-
-// The 128-column tiles that lie entirely above the diagonal of a causal product, as whole runs
-// of a row (one wavefront per row): -inf without any arithmetic (matmul.cu:182-184).  Runs of up
-// to a whole row are what the memory likes best; the same bytes written tile by tile from inside
-// the persistent kernel hold up its barriers.
-__global__ __launch_bounds__(256) void fill_causal_rows_kernel(MatmulArgs a) {
-  const int lane = threadIdx.x & 63;
-  const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);  // row, over all batches
-  if (r >= (int64_t)a.batches * a.m) return;
-  const int batch = (int)(r / a.m), y = (int)(r - (int64_t)batch * a.m);
-  const int x0 = (y / 128 + 1) * 128;  // first column right of the tile that holds the diagonal
-  half_t* const out = a.output + (int64_t)batch * a.stride_oz;
-  half_t* const row = out + (int64_t)y * a.stride_oy;
-  const half_t ninf = neg_inf_half();
-  const half8_t v = {ninf, ninf, ninf, ninf, ninf, ninf, ninf, ninf};
-  const bool aligned = out_vectorizable(a, out);
-  for (int x = x0 + lane * 8; x < a.n; x += 512) {
-    if (x + 8 <= a.n) {
-      if (aligned) __builtin_nontemporal_store(v, (half8_t*)(row + x));
-      else store8_any(row + x, v);
-    } else {
-      for (int q = 0; x + q < a.n; q++) row[x + q] = ninf;
-    }
-  }
-}
 
 // (four writers instead of two leave the multiplying wavefronts 128 registers, nine short, and
 // measure the same: the stores wait for the memory, not for wavefronts to issue them)
@@ -1148,13 +1122,18 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
   // Workgroup g runs on die g % 8: the workgroups of a die take neighbouring units (they share
   // right panels in the die's L2).  Odd rounds walk the workgroups backwards, which pairs long
   // and short rows of a causal product.
+  // Tiles above the diagonal of a causal product take their turn like the others, less the MFMAs: -inf
+  // goes through the staging tile.  The launch is bound by its writes, and those of a unit follow each other this
+  // way; the hidden tiles as whole rows by the writers, behind or before the others of a unit, or in a launch of
+  // their own took longer (us: a launch of its own / rows by the writers / this; 32 heads of 128, 1024 keys 31.4 /
+  // 34.5 / 15.9, 513 52.7 / 39.2 / 19.9, 2048 75.7 / 72.3 / 67.5; 20 heads of 64, 1500 50.9 / 74.3 / 45.0).
   const int XCDS = map.xcds;
   const int gl = G % XCDS == 0 ? (blockIdx.x % XCDS) * (G / XCDS) + blockIdx.x / XCDS : blockIdx.x;
 
   // Cursor over this workgroup's units and the tiles in them, in processing order.
   struct Cursor {
-    int t, unit, batch, m0, n, n_end, n_vis_end;  // tiles [n, n_vis_end) computed, [.., n_end) filled
-    bool valid, first;                            // first: no earlier computed tile in this unit
+    int t, unit, batch, m0, n, n_end;
+    bool valid, first;  // first: no earlier tile in this unit
   };
   auto load_unit = [&](Cursor& c) {
     c.unit = c.t * G + ((c.t & 1) ? G - 1 - gl : gl);
@@ -1164,23 +1143,25 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
     c.m0 = (row - c.batch * map.tiles_m) * BM;
     c.n = sg * map.seg;
     c.n_end = min(c.n + map.seg, map.tiles_n);
-    // tiles with n0 > m0 + BM - 1 of a causal product are all -inf
-    const int vis = a.mask == ADR_MASK_CAUSAL ? (c.m0 + BM - 1) / BN + 1 : map.tiles_n;
-    c.n_vis_end = min(c.n_end, vis);
     c.valid = true;
   };
-  // first / next tile that is computed (units without one are skipped)
   auto first_item = [&](Cursor& c) {
     c.t = 0;
     load_unit(c);
-    while (c.valid && c.n >= c.n_vis_end) { c.t++; load_unit(c); }
     c.first = true;
   };
   auto next_item = [&](Cursor& c) {
     c.n++;
     c.first = false;
-    while (c.valid && c.n >= c.n_vis_end) { c.t++; load_unit(c); c.first = true; }
+    if (c.valid && c.n >= c.n_end) { c.t++; load_unit(c); c.first = true; }
   };
+  const bool causal = a.mask == ADR_MASK_CAUSAL;
+  // Identity and Scale need neither the previous output nor the bias (the fp16 product x * 1 is exact: one
+  // multiply serves both).  With a positive factor the mask is applied where the results are staged, by eight
+  // wavefronts instead of the two that write: -inf stays -inf.
+  const bool plain = a.store == ADR_STORE_IDENTITY || a.store == ADR_STORE_SCALE;
+  const half_t mul = a.store == ADR_STORE_SCALE ? (half_t)a.scale : (half_t)1.0f;
+  const bool staged_mask = causal && plain && mul > (half_t)0.0f;
 
   if (wave >= 8 + NWW) {
     // ---------------------------------------------------------------- loader wavefronts
@@ -1268,9 +1249,6 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
     Epilogue ep{a.bias, a.beta, hscale, a.store, true};
     const int walign = out_chunk_alignment(a, a.output);
     const bool vec = walign >= 2;
-    // (Identity and Scale need neither the previous output nor the bias: any alignment)
-    const bool plain = a.store == ADR_STORE_IDENTITY || a.store == ADR_STORE_SCALE;
-    const half_t mul = a.store == ADR_STORE_SCALE ? hscale : (half_t)1.0f;
     auto write_half = [&](int batch, int m0, int n0, int half) {
       const int r0 = half * 64 + sw * WROWS;  // first of this wavefront's rows in the tile
       auto staged = [&](int it) {
@@ -1280,12 +1258,11 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
       half_t* const out = a.output + (int64_t)batch * a.stride_oz;
       const int y0 = m0 + r0 + rrow, x = n0 + rc * 8;
       const bool inside = m0 + r0 + WROWS <= a.m && n0 + BN <= a.n;
-      const bool unmasked = a.mask != ADR_MASK_CAUSAL || n0 + BN - 1 <= m0 + r0;
+      const bool unmasked = !causal || staged_mask || n0 + BN - 1 <= m0 + r0;
       if (plain && unmasked) {
         half8_t v[WIT];
 #pragma unroll
         for (int it = 0; it < WIT; it++) v[it] = staged(it);
-        // x * 1 is exact: one multiply serves Identity and Scale (fp16 product, matmul.cu)
         half_t* const p = out + (int64_t)y0 * a.stride_oy + x;
         if (inside && walign == 8) {
 #pragma unroll
@@ -1352,8 +1329,7 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
     load_unit(c);
     bool started = false;
     while (c.valid) {
-      const int first = c.n;
-      for (; c.n < c.n_vis_end; c.n++) {
+      for (; c.n < c.n_end; c.n++) {
         if (!started) {
           __builtin_amdgcn_s_barrier();  // barrier 0
           __builtin_amdgcn_s_barrier();  // barrier 1
@@ -1364,11 +1340,6 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
         __builtin_amdgcn_s_barrier();  // barrier 2j+3: the lower half
         write_half(c.batch, c.m0, c.n * BN, 1);
       }
-      // fully masked tiles of this unit, unless fill_causal_rows_kernel wrote them already
-      if (!map.prefilled)
-        for (int n = max(first, c.n_vis_end); n < c.n_end; n++)
-          fill_masked_tile<BM, BN, NWW * 64>(a, a.output + (int64_t)c.batch * a.stride_oz, c.m0, n * BN,
-                                        tid - 512);
       c.t++;
       load_unit(c);
     }
@@ -1387,7 +1358,7 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
   const int offQ = lds_chunk_off<CPR>(grp * 64 + frow, fkg);
   const int offB = lds_chunk_off<CPR>(wn * 32 + frow, fkg);
   half8_t qa[KS][4];   // this wavefront's rows of the left panel
-  float4_t acc[4][2];
+  float4_t acc[4][2] = {};  // (of a hidden first tile nothing is computed)
   // Load Scale (matmul.cu:439-443): both operands are multiplied by the scale, in fp16, before the
   // product -- the left panel once per segment, the right fragments as they are read
   const bool load_scale = a.load == ADR_LOAD_SCALE;
@@ -1437,9 +1408,11 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
     __builtin_amdgcn_sched_barrier(0);
   };
   // narrow and write the wavefront's 64 x 32 block: lane l of block (i, jj) holds row l % 16,
-  // columns 4 * (l / 16) .. +3 of the block
-  auto narrow = [&]() {
+  // columns 4 * (l / 16) .. +3 of the block.  below: how far the block's first row is below its first column
+  // (under the mask; a hidden element lies above the diagonal)
+  auto narrow = [&](int below) {
     const int lrow = lane & 15, cg = lane >> 4;
+    const bool edge = staged_mask && below < 31;  // (the block's last column against its first row)
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int row = grp * 64 + i * 16 + lrow;
@@ -1448,6 +1421,11 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
         half4_t h;
 #pragma unroll
         for (int e = 0; e < 4; e++) h[e] = (half_t)acc[i][jj][e];
+        if (edge) {
+          const int seen = below + i * 16 + lrow - (jj * 16 + cg * 4);  // columns of the lane's four up to the row's own
+#pragma unroll
+          for (int e = 0; e < 4; e++) h[e] = e > seen ? neg_inf_half() : h[e];
+        }
         const int cc = wn * 4 + jj * 2 + (cg >> 1);
         *(half4_t*)(sC + row * 256 + ((cc ^ (row & 15)) << 4) + (cg & 1) * 8) = h;
       }
@@ -1457,14 +1435,17 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
   Cursor c;
   first_item(c);
   if (!c.valid) return;
+  // first row of the wavefront's block less its first column
+  auto below = [&]() { return c.m0 + grp * 64 - c.n * BN - wn * 32; };
+  auto visible = [&]() { return !causal || below() > -64; };  // (the block's last row sees its first column)
   if (grp == 0) {
     for (int j = 0; c.valid; j++) {
       __builtin_amdgcn_s_barrier();  // barrier 2j: the panels of tile j have landed
       if (c.first) copy_left();
-      multiply(sB + (j % RING) * PANEL);
+      if (visible()) multiply(sB + (j % RING) * PANEL);
       __builtin_amdgcn_s_waitcnt(0xC07F);  // the panel has been read (lgkmcnt 0)
       __builtin_amdgcn_s_barrier();  // barrier 2j+1: this half of the staging tile is free
-      narrow();
+      narrow(below());
       __builtin_amdgcn_s_waitcnt(0xC07F);  // staged
       next_item(c);
     }
@@ -1476,11 +1457,12 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
     for (int j = 0; c.valid; j++) {
       __builtin_amdgcn_s_waitcnt(0xC07F);
       __builtin_amdgcn_s_barrier();  // barrier 2j+1
-      multiply(sB + (j % RING) * PANEL);
+      if (visible()) multiply(sB + (j % RING) * PANEL);
       __builtin_amdgcn_s_waitcnt(0xC07F);
       __builtin_amdgcn_s_barrier();  // barrier 2j+2: the ring buffer of tile j is free
+      const int tile_below = below();
       next_item(c);
-      narrow();
+      narrow(tile_below);
       if (c.valid && c.first) copy_left();  // tile j+1 opens a unit: its left panel has landed
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);
@@ -2311,15 +2293,6 @@ hipError_t launch_shortk(hipStream_t stream, const MatmulArgs& a) {
   map.segs_per_row = (map.tiles_n + map.seg - 1) / map.seg;
   map.units = map.rows * map.segs_per_row;
   const unsigned grid = map.units < NUM_CU ? (unsigned)map.units : NUM_CU;
-  map.prefilled = 0;
-  const int64_t all_rows = (int64_t)a.m * a.batches;
-  if (a.mask == ADR_MASK_CAUSAL && map.tiles_n > 1 && all_rows <= 0x7fffffffLL) {
-    hipLaunchKernelGGL(fill_causal_rows_kernel, dim3((unsigned)((all_rows + 3) / 4)), dim3(256), 0,
-                       stream, a);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    map.prefilled = 1;
-  }
   hipLaunchKernelGGL((gemm_nt_shortk_kernel<CPR>), dim3(grid), dim3(SHORTK_THREADS), 0, stream, a, map);
   return hipGetLastError();
 }
