@@ -1480,11 +1480,17 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
 // of two fp16 LDS stages in the same swizzled layout the DMA produces, so that every weight is
 // dequantised once per workgroup and the MFMA loop is the one of the fp16 kernel.
 // MI16: 16x16x32 MFMAs, two k-steps per slice, all chunks dequantised in the first (the 256 x 128
-// tile: 5-6 % faster; the 256 x 192 tile has no registers for the second set of fragments)
+// tile: 5-6 % faster; the 256 x 192 tile, which got the registers for the second set of fragments when its
+// addresses left them: 1-4 %, K4096 N11008 M2048 192.7 -> 186.6 us)
 // G: groups of WM x WN wavefronts that split K between them (1: none).  A tile that has its compute
 // unit to itself is bound by the chain of one slice -- barrier, fragment reads, MFMAs, the wait for
 // the next slice: 0.3-0.4 us per slice of a 64 x 64 tile whatever its loads -- so with at most one
 // tile per compute unit the small tiles run G such chains side by side.
+// A slice's requests: the left operand's first and behind the fence, the weights' wherever the scheduler finds room
+// among the MFMAs.  All of them ahead of the slice's MFMAs held every wavefront up for as long as the requests took to
+// leave (weights from HBM, us: K11008 N4096 m=160 55.0 -> 47.1, 384 81.5 -> 70.3, K13824 N5120 m=96 66.8 -> 57.7,
+// K4096 N12288 m=64 29.0 -> 27.1, 1536 179 -> 172); without the fence the left operand's moved back as well, and the
+// large tiles lost 10-15 %.
 template <int BM, int BN, int WM, int WN, bool MI16, int BK = 64, int G = 1, int SA = 3>
 __global__ __launch_bounds__(WM* WN* G * 64, 1) void gemm_nt_u8_kernel(MatmulArgs a, TileMap map,
                                                                       int block_shift) {
@@ -1527,25 +1533,34 @@ __global__ __launch_bounds__(WM* WN* G * 64, 1) void gemm_nt_u8_kernel(MatmulArg
   const int wm = wave / WN, wn = wave % WN;
   half_t* const out = a.output;
 
-  const half_t* gA[IA];
+  // Addresses: buffer descriptors of the tile's rows, the lane's byte offset of its rows (clamped to the last one) in
+  // 32 bits (choose() sends rows of more than 2^22 weights elsewhere) and the place in K as the scalar offset, so that
+  // no address is computed in the vector ALU and none takes a register pair.
+  const uint32_t rows_a = min(BM, a.m - m0), rows_b = min(BN, a.n - n0);
+  auto rA = __builtin_amdgcn_make_buffer_rsrc((void*)(a.lhs + (int64_t)m0 * a.stride_ly), 0,
+                                              (int)(rows_a * (uint32_t)a.k * 2), 0x00020000);
+  auto rQ = __builtin_amdgcn_make_buffer_rsrc((void*)(a.rhs_q + (int64_t)n0 * a.k), 0,
+                                              (int)(rows_b * (uint32_t)a.k), 0x00020000);
+  auto rS = __builtin_amdgcn_make_buffer_rsrc((void*)(a.scales + (int64_t)n0 * (a.k >> block_shift)), 0,
+                                              (int)(rows_b * (uint32_t)(a.k >> block_shift) * 2), 0x00020000);
+  uint32_t gA[IA];
 #pragma unroll
   for (int i = 0; i < IA; i++) {
     int row, kc;
     lds_chunk_inv<CPR>((i * NW + wave) * 64 + lane, row, kc);
-    gA[i] = a.lhs + (int64_t)min(m0 + row, a.m - 1) * a.stride_ly + kc * 8;
+    gA[i] = (min((uint32_t)row, rows_a - 1) * (uint32_t)a.k + kc * 8) * 2;
   }
   // weight chunk c = tid + i*NT -> (row, 8-weight group kc); rows beyond N are clamped
-  const uint8_t* gQ[LB];
-  const half_t* gS[LB];
+  uint32_t gQ[LB], gS[LB];
   int offB[LB];
 #pragma unroll
   for (int i = 0; i < LB; i++) {
     const int c = tid + i * NT, row = c / CPR, kc = c % CPR;
-    const int brow = min(n0 + row, a.n - 1);
-    gQ[i] = a.rhs_q + (int64_t)brow * a.k + kc * 8;
+    const uint32_t brow = min((uint32_t)row, rows_b - 1);
+    gQ[i] = brow * (uint32_t)a.k + kc * 8;
     // block of weight k0 + 8*kc: k0 is a multiple of BK and 8*kc < BK, so the two parts of the
     // index add up exactly for any power-of-two block size
-    gS[i] = a.scales + (int64_t)brow * (a.k >> block_shift) + ((kc * 8) >> block_shift);
+    gS[i] = (brow * (uint32_t)(a.k >> block_shift) + ((kc * 8) >> block_shift)) * 2;
     offB[i] = lds_chunk_off<CPR>(row, kc);
   }
   const int KT = a.k / (BK * G);
@@ -1555,8 +1570,7 @@ __global__ __launch_bounds__(WM* WN* G * 64, 1) void gemm_nt_u8_kernel(MatmulArg
     kloadA++;
 #pragma unroll
     for (int i = 0; i < IA; i++)
-      __builtin_amdgcn_global_load_lds(ADR_GLB_PTR(gA[i] + k0),
-                                       ADR_LDS_PTR(dA + goA + (i * NW + wave) * 1024), 16, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, ADR_LDS_PTR(dA + goA + (i * NW + wave) * 1024), 16, (int)gA[i], k0 * 2, 0, 0);
   };
   // three register sets: the weights consumed in slice kt+1 were requested at the head of slice
   // kt-1, so the wait at the end of slice kt-1 (everything but that slice's own requests)
@@ -1564,12 +1578,12 @@ __global__ __launch_bounds__(WM* WN* G * 64, 1) void gemm_nt_u8_kernel(MatmulArg
   u32x2_t rq[3][LB];
   half_t rs[3][LB];
   auto fetchQ = [&](int set) {
-    const int ks = min(kloadQ, KT - 1) * G + grp;
+    const int k0 = (min(kloadQ, KT - 1) * G + grp) * BK;
     kloadQ++;
 #pragma unroll
     for (int i = 0; i < LB; i++) {
-      rq[set][i] = *(const u32x2_t*)(gQ[i] + ks * BK);
-      rs[set][i] = gS[i][(ks * BK) >> block_shift];
+      rq[set][i] = __builtin_amdgcn_raw_buffer_load_b64(rQ, (int)gQ[i], k0, 0);
+      rs[set][i] = __builtin_bit_cast(half_t, __builtin_amdgcn_raw_buffer_load_b16(rS, (int)gS[i], (k0 >> block_shift) * 2, 0));
     }
   };
   auto dequant_store1 = [&](int set, unsigned char* dB, int i) {
@@ -1623,9 +1637,9 @@ __global__ __launch_bounds__(WM* WN* G * 64, 1) void gemm_nt_u8_kernel(MatmulArg
   // that receives the weights of slice kt+3 (the one slice kt was dequantised from).
   auto slice = [&](const unsigned char* cA, const unsigned char* cB, const unsigned char* nA,
                    unsigned char* nB, unsigned char* dA, int fset, int nset) {
-    fetchQ(fset);
     dmaA(dA);
     __builtin_amdgcn_sched_barrier(0);
+    fetchQ(fset);
     // first k-step: the fragments of the second are read and the slice's LB 8-weight chunks are
     // dequantised, their VALU work and LDS writes filling the gaps between its MFMAs
 #pragma unroll
@@ -1655,6 +1669,7 @@ __global__ __launch_bounds__(WM* WN* G * 64, 1) void gemm_nt_u8_kernel(MatmulArg
     // in flight; the dequantised weights of slice kt+1 are in LDS
     // (four A stages: the transfer issued in the slice before, which is younger than that slice's
     // weight requests, may stay in flight too)
+    __builtin_amdgcn_sched_barrier(0x38F);
     constexpr int n = 2 * LB + (SA - 2) * IA;
     __builtin_amdgcn_s_waitcnt(0x0070 | (n & 0xF) | ((n >> 4) << 14));
     __builtin_amdgcn_s_barrier();
@@ -2465,7 +2480,8 @@ GemmChoice choose(const MatmulArgs& a) {
     // instead of 128 x 128 is within +-4 % up to K 512 and 4-12 % behind above.)
     return c;
   }
-  if (a.rhs_q && a.k % 64 == 0 && a.block_size >= 8 && (a.block_size & (a.block_size - 1)) == 0) {
+  // (the u8 kernel addresses the rows of a tile in 32 bits: 256 rows of 2^22 halves are 2^31 bytes)
+  if (a.rhs_q && a.k % 64 == 0 && a.k <= 1 << 22 && a.block_size >= 8 && (a.block_size & (a.block_size - 1)) == 0) {
     // (tests and benchmarks can force a tile: adr_debug_knob; 1 + N_U8_TILES: 128 x 64 with two K
     // groups, 2 + N_U8_TILES: 64 x 64 with four, 3 + N_U8_TILES: the staged kernels below)
     const int forced = knob(KNOB_U8_TILE);
@@ -2653,7 +2669,7 @@ static hipError_t launch_choice(hipStream_t stream, const MatmulArgs& a, GemmCho
   switch (c) {
     case SHORTK_64: return launch_shortk<8>(stream, a);
     case SHORTK_128: return launch_shortk<16>(stream, a);
-    case U8_256x192: return launch_u8<256, 192, 4, 2, false>(stream, a);
+    case U8_256x192: return launch_u8<256, 192, 4, 2, true>(stream, a);
     // (four stages of the left operand, three slices ahead, fill the 160 KB: K11008 N4096 M2048 with
     // weights from HBM 202 -> 191 us, K4096 unchanged; the smaller tiles gain nothing from a fourth stage)
     case U8_256x128: return launch_u8<256, 128, 4, 2, true, 64, 1, 4>(stream, a);
@@ -2808,9 +2824,10 @@ const char* gemm_u8_mfma_plan(int m, int p, int n, int block_size) {
 }
 
 // Estimated time of the u8 product on the tiled u8 kernel, in us (negative: that kernel does not
-// cover it): pick()'s cost of the chosen tile times K.  4 us + 4.3e-7 us per unit fits one tile per
-// CU of 64 x 64 (K11008 53-59 us, K4096 23-26) and of 128 x 64 (71-85, 30-35) on weights that come
-// from HBM (3.5e-7 where the Infinity Cache holds them: 47 / 21 and 68 / 30).
+// cover it): pick()'s cost of the chosen tile times K.  4 us + 4.3e-7 us per unit is 10-15 % above what one
+// tile per CU of 64 x 64 (K11008 43-50 us, K4096 20-23) and of 128 x 64 (67-73, 28-30) takes on weights that
+// come from HBM: where this is compared with the passes of 64 rows the two are that close (K11008 m=72 42.5 us
+// tiled and 41.4 in passes, 96 46.4 and 44.5, 128 49.8 and 52.5), and the passes keep the tie.
 double gemm_u8_mfma_estimate_us(int m, int p, int n, int block_size) {
   const MatmulArgs a = u8_args(nullptr, nullptr, (const uint8_t*)16, nullptr, m, p, n, block_size, 0.0f);
   if (!(p % 64 == 0 && block_size >= 8 && (block_size & (block_size - 1)) == 0)) return -1.0;
