@@ -334,7 +334,7 @@ def main():
                          "gbs": round(byts / t / 1e9, 1),
                          "frac_hbm_peak": round(byts / t / 1e9 / PEAK_HBM_GBS, 4)}}
         # the same product under the causal mask (llama.rs:534-545): the same bytes are written,
-        # half of them -inf by a fill launch of their own, and half the arithmetic is done
+        # half of them -inf, and half the arithmetic is done
         t = timed(lambda: f_qk(1), 50, 5)
         attn["qk_t_causal"] = {"us": round(t * 1e6, 1), "gbs": round(byts / t / 1e9, 1),
                                "frac_hbm_peak": round(byts / t / 1e9 / PEAK_HBM_GBS, 4),
