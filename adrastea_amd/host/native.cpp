@@ -46,11 +46,24 @@ struct Ref {
   }
 };
 
+// Clears what an Exception reports (the general path raises it again, if it is one of the call's own); false: an
+// interrupt or an exit came by on its way through torch's functions, which is the caller's to see.
+bool cleared() {
+  if (!PyErr_Occurred()) return true;
+  if (!PyErr_ExceptionMatches(PyExc_Exception)) return false;
+  PyErr_Clear();
+  return true;
+}
+
 // None to the caller: "take the general path" (which raises if there is something to raise).
 PyObject* general() {
-  PyErr_Clear();
+  if (!cleared()) return nullptr;
   Py_RETURN_NONE;
 }
+
+// An attribute, unless the object is missing or an exception is on its way already.
+PyObject* attr(PyObject* o, PyObject* name) { return o && !PyErr_Occurred() ? PyObject_GetAttr(o, name) : nullptr; }
+PyObject* call(PyObject* o, PyObject* method) { return o && !PyErr_Occurred() ? PyObject_CallMethodNoArgs(o, method) : nullptr; }
 
 // A plain int that fits 64 bits.
 bool as_int(PyObject* o, int64_t& v) {
@@ -77,15 +90,15 @@ bool read_ints(PyObject* t, int64_t* out, int& rank) {
 }
 
 bool read_layout(PyObject* view, Layout& l) {
-  const Ref lay(PyObject_GetAttr(view, s_layout));
+  const Ref lay(attr(view, s_layout));
   if (!lay.p || (PyObject*)Py_TYPE(lay.p) != layout_type) return false;
-  const Ref dims(PyObject_GetAttr(lay, s_dims)), strides(PyObject_GetAttr(lay, s_strides));
+  const Ref dims(attr(lay, s_dims)), strides(attr(lay, s_strides));
   l.rank = -1;
   return read_ints(dims, l.dims, l.rank) && read_ints(strides, l.strides, l.rank);
 }
 
 bool call_int(PyObject* o, PyObject* method, int64_t& v) {
-  const Ref r(PyObject_CallMethodNoArgs(o, method));
+  const Ref r(call(o, method));
   return as_int(r, v);
 }
 
@@ -93,11 +106,11 @@ bool call_int(PyObject* o, PyObject* method, int64_t& v) {
 bool read_ptr(PyObject* o, void*& p) {
   int64_t v;
   if ((PyObject*)Py_TYPE(o) == view_type) {
-    const Ref offset(PyObject_GetAttr(o, s_offset));
+    const Ref offset(attr(o, s_offset));
     int64_t at;
     if (!as_int(offset, at)) return false;
     if (at == 0) {
-      const Ref storage(PyObject_GetAttr(o, s_storage));
+      const Ref storage(attr(o, s_storage));
       if (!storage.p || !call_int(storage, s_data_ptr, v)) return false;
       p = (void*)(uintptr_t)v;
       return true;
@@ -152,7 +165,7 @@ PyObject* make_view(PyObject* storage, PyObject* dims, PyObject* strides, PyObje
 PyObject* view_of(PyObject*, PyObject* const* a, Py_ssize_t n, PyObject* names) {
   if (n == 1 && !names) {
     PyObject* const t = a[0];
-    const Ref shape(PyObject_GetAttr(t, s_shape)), stride(PyObject_CallMethodNoArgs(t, s_stride));
+    const Ref shape(attr(t, s_shape)), stride(call(t, s_stride));
     int64_t d[MAX_RANK], s[MAX_RANK];
     int rank = -1;
     if (shape.p && stride.p && PyTuple_Check(shape) && PyTuple_CheckExact(stride) && read_ints(shape, d, rank) &&
@@ -166,13 +179,12 @@ PyObject* view_of(PyObject*, PyObject* const* a, Py_ssize_t n, PyObject* names) 
       }
     }
   }
-  PyErr_Clear();
-  return PyObject_Vectorcall(of_general, a, n, names);
+  return cleared() ? PyObject_Vectorcall(of_general, a, n, names) : nullptr;
 }
 
 // A method's general definition, with `self` in front of its arguments.
 PyObject* call_general(PyObject* method, PyObject* self, PyObject* const* a, Py_ssize_t n, PyObject* names) {
-  PyErr_Clear();
+  if (!cleared()) return nullptr;
   const Ref bound(PyMethod_New(method, self));
   return bound.p ? PyObject_Vectorcall(bound, a, n, names) : nullptr;
 }
@@ -187,7 +199,7 @@ PyObject* view_permute(PyObject* self, PyObject* const* a, Py_ssize_t n, PyObjec
       inside = inside && o[i] >= 0 && o[i] < l.rank;
       if (inside) d[i] = l.dims[o[i]], s[i] = l.strides[o[i]];
     }
-    const Ref storage(PyObject_GetAttr(self, s_storage)), offset(PyObject_GetAttr(self, s_offset));
+    const Ref storage(attr(self, s_storage)), offset(attr(self, s_offset));
     if (inside && storage.p && offset.p && PyLong_CheckExact(offset))
       return make_view(storage, ints(d, l.rank), ints(s, l.rank), offset);
   }
@@ -209,7 +221,7 @@ PyObject* view_shape_cast(PyObject* self, PyObject* const* a, Py_ssize_t nargs, 
   if (ok) {
     int64_t step = 1;
     for (int i = n - 1; i >= 0; i--) s[i] = step, step *= d[i];
-    const Ref storage(PyObject_GetAttr(self, s_storage)), offset(PyObject_GetAttr(self, s_offset));
+    const Ref storage(attr(self, s_storage)), offset(attr(self, s_offset));
     if (storage.p && offset.p && PyLong_CheckExact(offset)) return make_view(storage, ints(d, n), ints(s, n), offset);
   }
   return call_general(cast_general, self, a, nargs, names);
@@ -229,23 +241,23 @@ PyObject* matmul_f16(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return general();
   const int64_t M = last(l.dims, l, 2), K = last(l.dims, l, 1), N = last(r.dims, r, 1);
   if (K != last(r.dims, r, 2) || last(o.dims, o, 2) != M || last(o.dims, o, 1) != N) return general();
-  const Ref load(PyObject_GetAttr(a[3], s_load)), store(PyObject_GetAttr(a[3], s_store)), mask(PyObject_GetAttr(a[3], s_mask));
+  const Ref load(attr(a[3], s_load)), store(attr(a[3], s_store)), mask(attr(a[3], s_mask));
   if (!load.p || !store.p) return general();
-  const Ref load_op(PyObject_GetAttr(load, s_op)), store_op(PyObject_GetAttr(store, s_op)), bias(PyObject_GetAttr(store, s_bias));
+  const Ref load_op(attr(load, s_op)), store_op(attr(store, s_op)), bias(attr(store, s_bias));
   int64_t lop, sop, msk;
   if (!as_int(load_op, lop) || !as_int(store_op, sop) || !as_int(mask, msk) || !bias.p) return general();
   double scale = 1.0, beta = 0.0, v;
   if (lop == 1) {
-    const Ref f(PyObject_GetAttr(load, s_scale));
+    const Ref f(attr(load, s_scale));
     if (!read_double(f, scale)) return general();
   }
   if (sop == 4) {
-    const Ref f(PyObject_GetAttr(store, s_scale));
+    const Ref f(attr(store, s_scale));
     if (!read_double(f, v)) return general();
     scale *= v;
   }
   if (sop == 2 || sop == 3) {
-    const Ref f(PyObject_GetAttr(store, s_beta));
+    const Ref f(attr(store, s_beta));
     if (!read_double(f, beta)) return general();
   }
   adr_stream_t stream;
@@ -316,12 +328,12 @@ PyObject* softmax_rows_inplace(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 bool read_shape(PyObject* t, int64_t (&d)[MAX_RANK], int rank) {
-  const Ref shape(PyObject_GetAttr(t, s_shape));
+  const Ref shape(attr(t, s_shape));
   return shape.p && PyTuple_Check(shape) && read_ints(shape, d, rank);
 }
 
 bool is_contiguous(PyObject* t) {
-  const Ref r(PyObject_CallMethodNoArgs(t, s_is_contiguous));
+  const Ref r(call(t, s_is_contiguous));
   return r == Py_True;
 }
 

@@ -165,3 +165,62 @@ def test_error_stats_descriptors():
     _native.bind(*([0] * len(_NATIVE_CALLS)), lambda: 0, lambda dev: 0)
     assert _native.error_stats(out, a, a, 0) is None
     assert _native.error_stats(out, a, a, 2) is None
+
+
+class Interrupted:
+    """A tensor whose attributes and methods report what they are given."""
+    def __init__(self, what):
+        self.what = what
+
+    def raised(self, *_):
+        raise self.what
+    shape = property(raised)
+    stride = data_ptr = is_contiguous = raised
+
+
+@pytest.mark.parametrize("what", [KeyboardInterrupt, SystemExit])
+def test_an_interrupt_is_not_taken_for_an_unusual_argument(calls, what):
+    """A signal's handler runs inside the functions that the native path calls: an interrupt goes on to the caller,
+    and nothing is launched; an Exception goes back to the definitions, which raise it themselves."""
+    x = TensorView.of(torch.zeros(4, 4, dtype=torch.float16))
+    for error in (what, RuntimeError):
+        inside = Interrupted(error)
+        with pytest.raises(error):
+            TensorView.of(inside)
+        view = TensorView(inside, x.layout, 0)
+        attempts = [lambda: _native.matmul_f16(x, view, x, MatmulOptions()), lambda: _native.matmul_f16(x, x, x, inside),
+                    lambda: _native.softmax_rows_inplace(view, 1.0),
+                    lambda: _native.quantize_absmax_uint8(inside, x.storage, x.storage),
+                    lambda: _native.matmul_nt_fp16u8(inside, inside, inside, inside, 32, 0.0)]
+        Interrupted.load_ = Interrupted.shape
+        try:
+            for attempt in attempts:
+                if error is RuntimeError:
+                    assert attempt() is None
+                else:
+                    with pytest.raises(what):
+                        attempt()
+        finally:
+            del Interrupted.load_
+
+        def device():
+            raise error
+        _native.bind(*([0x1000] * len(_NATIVE_CALLS)), device, lambda dev: 0)   # (never called: the stream comes first)
+        if error is RuntimeError:
+            assert _native.softmax_rows_inplace(x, 1.0) is None
+        else:
+            with pytest.raises(what):
+                _native.softmax_rows_inplace(x, 1.0)
+    assert calls == []
+
+
+def test_a_tensor_without_a_shape_is_asked_no_further():
+    class Strange:
+        asked = 0
+
+        def stride(self):
+            Strange.asked += 1
+            return (1,)
+    with pytest.raises(AttributeError, match="shape"):
+        TensorView.of(Strange())
+    assert Strange.asked == 0   # (the definition reads the shape first as well)
