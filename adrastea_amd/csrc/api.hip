@@ -15,7 +15,6 @@ int set_knob(int id, int value);  // device.hip
 
 namespace {
 
-constexpr int ABI_VERSION = 1;
 
 int validate_matmul(const MatmulArgs& a, bool check_ptrs) {
   if (a.store > ADR_STORE_QUICK_GELU_BIAS || a.load > ADR_LOAD_SCALE || a.mask > ADR_MASK_CAUSAL)
@@ -348,7 +347,7 @@ int run_matmul_held(hipStream_t stream, MatmulArgs& a) {
 
 extern "C" {
 
-int adr_abi_version(void) { return ABI_VERSION; }
+int adr_abi_version(void) { return ADR_ABI_VERSION; }
 
 const char* adr_strerror(int code) {
   switch (code) {

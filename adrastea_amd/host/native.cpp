@@ -450,11 +450,17 @@ PyObject* install(PyObject*, PyObject* args) {
   Py_RETURN_NONE;
 }
 
-// bind(addresses of the library's functions ..., torch.cuda.current_device, torch's raw stream of a device)
+// bind(the library's ABI version, addresses of its functions ..., torch.cuda.current_device, torch's raw stream of a
+// device).  The signatures above are those of the header at this module's own build.
 PyObject* bind(PyObject*, PyObject* args) {
+  int abi;
   unsigned long long p[8];
   PyObject *dev, *raw;
-  if (!PyArg_ParseTuple(args, "KKKKKKKKOO", p, p + 1, p + 2, p + 3, p + 4, p + 5, p + 6, p + 7, &dev, &raw)) return nullptr;
+  if (!PyArg_ParseTuple(args, "iKKKKKKKKOO", &abi, p, p + 1, p + 2, p + 3, p + 4, p + 5, p + 6, p + 7, &dev, &raw)) return nullptr;
+  if (abi != ADR_ABI_VERSION)
+    return PyErr_Format(PyExc_RuntimeError,
+                        "adrastea_amd._native was built for ABI version %d, the library has %d: build both "
+                        "with `python -m adrastea_amd.build`", ADR_ABI_VERSION, abi);
   matmul_fn = (decltype(matmul_fn))p[0];
   attention_fn = (decltype(attention_fn))p[1];
   softmax_fn = (decltype(softmax_fn))p[2];

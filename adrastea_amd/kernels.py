@@ -209,7 +209,8 @@ class GpuKernels(CommonKernels):
         self._workspace = (torch.empty(workspace_bytes, dtype=torch.uint8, device="cuda")
                            if workspace_bytes > 0 else None)
         if _native is not None:
-            _native.bind(*(C.cast(getattr(self._lib, name), C.c_void_p).value for name in _NATIVE_CALLS),
+            _native.bind(self._lib.adr_abi_version(),
+                         *(C.cast(getattr(self._lib, name), C.c_void_p).value for name in _NATIVE_CALLS),
                          torch.cuda.current_device, torch._C._cuda_getCurrentRawStream)
 
     @staticmethod

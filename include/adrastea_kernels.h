@@ -27,6 +27,10 @@
 extern "C" {
 #endif
 
+/* The version of the signatures declared here (bumped on any change of one): what adr_abi_version() of a library
+ * built from them returns. */
+#define ADR_ABI_VERSION 1
+
 /* A hipStream_t, declared opaquely so that this header needs no HIP include. */
 typedef void* adr_stream_t;
 
@@ -450,7 +454,7 @@ int adr_microbench_stream_read(adr_stream_t stream, const void* src, int64_t byt
 
 /* Human-readable text for an ADR_E* code or hipError_t. */
 const char* adr_strerror(int code);
-/* ABI version of this library (bumped on any signature change). */
+/* ADR_ABI_VERSION of the header that this library was built from. */
 int adr_abi_version(void);
 
 #ifdef __cplusplus

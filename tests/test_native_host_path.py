@@ -11,6 +11,7 @@ from adrastea_amd import MatmulLoad, MatmulMask, MatmulOptions, MatmulStore, Ten
 from adrastea_amd.kernels import _NATIVE_CALLS, descriptor, _lower
 from adrastea_amd.tensor import _native
 
+ABI = _ffi.lib().adr_abi_version()
 pytestmark = pytest.mark.skipif(_native is None, reason="the native module is not built")
 
 
@@ -76,9 +77,9 @@ def calls():
             keep.append(None)
             continue
         keep.append(C.CFUNCTYPE(C.c_int, *types)(lambda *a, name=name: seen.append((name, a)) or 7))
-    _native.bind(*(C.cast(f, C.c_void_p).value if f else 0 for f in keep), lambda: 3, lambda dev: 0x1000 + dev)
+    _native.bind(ABI, *(C.cast(f, C.c_void_p).value if f else 0 for f in keep), lambda: 3, lambda dev: 0x1000 + dev)
     yield seen
-    _native.bind(*([0] * len(_NATIVE_CALLS)), lambda: 0, lambda dev: 0)
+    _native.bind(ABI, *([0] * len(_NATIVE_CALLS)), lambda: 0, lambda dev: 0)
 
 
 def as_ctypes(name, args):
@@ -162,7 +163,7 @@ def test_error_stats_descriptors():
     (test_gpu_error_stats.py); here, what the native path hands back."""
     out, a = TensorView.of(torch.zeros(3)), TensorView.of(torch.zeros(4, 6, dtype=torch.float16))
     assert descriptor(a.shape_cast([-1])).shape[0] == 24
-    _native.bind(*([0] * len(_NATIVE_CALLS)), lambda: 0, lambda dev: 0)
+    _native.bind(ABI, *([0] * len(_NATIVE_CALLS)), lambda: 0, lambda dev: 0)
     assert _native.error_stats(out, a, a, 0) is None
     assert _native.error_stats(out, a, a, 2) is None
 
@@ -205,7 +206,7 @@ def test_an_interrupt_is_not_taken_for_an_unusual_argument(calls, what):
 
         def device():
             raise error
-        _native.bind(*([0x1000] * len(_NATIVE_CALLS)), device, lambda dev: 0)   # (never called: the stream comes first)
+        _native.bind(ABI, *([0x1000] * len(_NATIVE_CALLS)), device, lambda dev: 0)   # (never called: the stream comes first)
         if error is RuntimeError:
             assert _native.softmax_rows_inplace(x, 1.0) is None
         else:
@@ -224,3 +225,9 @@ def test_a_tensor_without_a_shape_is_asked_no_further():
     with pytest.raises(AttributeError, match="shape"):
         TensorView.of(Strange())
     assert Strange.asked == 0   # (the definition reads the shape first as well)
+
+
+def test_a_library_of_another_abi_is_refused():
+    for abi in (ABI - 1, ABI + 1):
+        with pytest.raises(RuntimeError, match="ABI version"):
+            _native.bind(abi, *([0] * len(_NATIVE_CALLS)), lambda: 0, lambda dev: 0)
