@@ -165,9 +165,16 @@ def build_native_module(force: bool = False) -> str:
     return NATIVE_MODULE
 
 
+def main(force: bool = False) -> None:
+    print(build_library(force=force))
+    print(build_stamps_library(force=force))
+    print(build_legacy_modules(force=force))
+    print(build_host_test(force=force))
+    try:  # (the calls work without it, through the interpreter: no reason to go without the library)
+        print(build_native_module(force=force))
+    except (RuntimeError, OSError) as e:
+        sys.stderr.write(f"warning: the native host path is not built: {e}\n")
+
+
 if __name__ == "__main__":
-    print(build_native_module(force="--force" in sys.argv))
-    print(build_library(force="--force" in sys.argv))
-    print(build_stamps_library(force="--force" in sys.argv))
-    print(build_legacy_modules(force="--force" in sys.argv))
-    print(build_host_test(force="--force" in sys.argv))
+    main(force="--force" in sys.argv)

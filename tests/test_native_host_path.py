@@ -231,3 +231,17 @@ def test_a_library_of_another_abi_is_refused():
     for abi in (ABI - 1, ABI + 1):
         with pytest.raises(RuntimeError, match="ABI version"):
             _native.bind(abi, *([0] * len(_NATIVE_CALLS)), lambda: 0, lambda dev: 0)
+
+
+def test_the_library_is_built_without_a_compiler_for_the_native_module(monkeypatch, capsys):
+    from adrastea_amd import build
+    done = []
+    for name in ("build_library", "build_stamps_library", "build_legacy_modules", "build_host_test"):
+        monkeypatch.setattr(build, name, lambda force, name=name: done.append(name))
+    for error in (RuntimeError("no Python.h"), FileNotFoundError("g++")):
+        def native(force):
+            raise error
+        monkeypatch.setattr(build, "build_native_module", native)
+        build.main()
+        assert str(error) in capsys.readouterr().err
+    assert done == 2 * ["build_library", "build_stamps_library", "build_legacy_modules", "build_host_test"]
