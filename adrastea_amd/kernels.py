@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import ctypes as C
 import threading
+import warnings
 from dataclasses import dataclass, field
 from typing import Optional, Tuple
 
@@ -187,11 +188,20 @@ _NATIVE_CALLS = ("adr_matmul_f16", "adr_attention_f16", "adr_softmax_rows", "adr
                  "adr_quantize_absmax_u8", "adr_dequantize_absmax_u8", "adr_error_stats_f16", "adr_error_stats_f32")
 
 
+def _bind_native() -> None:
+    """Hands the library's functions and torch's to the native host path (the same ones every time)."""
+    import torch
+    lib = _ffi.lib()
+    _native.bind(lib.adr_abi_version(), *(C.cast(getattr(lib, name), C.c_void_p).value for name in _NATIVE_CALLS),
+                 torch.cuda.current_device, torch._C._cuda_getCurrentRawStream)
+
+
 class GpuKernels(CommonKernels):
     """Launches through the C ABI on torch's current HIP stream.
 
     Where host/native.cpp is built, the calls below are lowered by it; what it does not take (it
     returns None) goes the way written out here, which is also the definition of what it does.
+    Without it every call goes that way, and the constructor warns.
 
     `workspace_bytes` > 0 gives the instance a scratch buffer of that size, owned like any other
     tensor of the host (in the reference: one more GpuBuffer held by GpuKernels); matmul_f16 then
@@ -209,9 +219,10 @@ class GpuKernels(CommonKernels):
         self._workspace = (torch.empty(workspace_bytes, dtype=torch.uint8, device="cuda")
                            if workspace_bytes > 0 else None)
         if _native is not None:
-            _native.bind(self._lib.adr_abi_version(),
-                         *(C.cast(getattr(self._lib, name), C.c_void_p).value for name in _NATIVE_CALLS),
-                         torch.cuda.current_device, torch._C._cuda_getCurrentRawStream)
+            _bind_native()
+        else:
+            warnings.warn("adrastea_amd._native is not built for this interpreter: the calls take 2-10 us more of the host "
+                          "each (`python -m adrastea_amd.build`)", RuntimeWarning, stacklevel=2)
 
     @staticmethod
     def _lowered(name, *args) -> bool:

@@ -2,6 +2,7 @@
 view type over device memory.  Strides are in elements; dims are outermost first."""
 from __future__ import annotations
 
+import importlib.util
 import math
 from dataclasses import dataclass
 from typing import Sequence, Tuple
@@ -144,9 +145,12 @@ class TensorView:
         return TensorView(self.storage, self.layout.take(sizes), self.offset)
 
 
-try:  # the same three methods as native code (host/native.cpp), where it is built
-    from . import _native
-except ImportError:
-    _native = None
+def _load_native(name: str = __package__ + "._native"):
+    """The native host path (host/native.cpp): None where it is not built for this interpreter.  A module that is
+    there and does not load raises, as a broken library does."""
+    return importlib.import_module(name) if importlib.util.find_spec(name) else None
+
+
+_native = _load_native()  # the three methods of a view that make views, and the calls of kernels.py
 if _native is not None:
     _native.install(TensorLayout, TensorView)

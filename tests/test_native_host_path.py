@@ -3,6 +3,7 @@ over ranks, orders and casts, what those refuse, and the argument tuples that re
 in the place of the library's functions."""
 import ctypes as C
 import itertools
+import warnings
 
 import pytest
 import torch
@@ -245,3 +246,21 @@ def test_the_library_is_built_without_a_compiler_for_the_native_module(monkeypat
         build.main()
         assert str(error) in capsys.readouterr().err
     assert done == 2 * ["build_library", "build_stamps_library", "build_legacy_modules", "build_host_test"]
+
+
+def test_a_module_that_does_not_load_is_reported(tmp_path, monkeypatch):
+    from importlib.machinery import EXTENSION_SUFFIXES
+    from adrastea_amd import GpuKernels, kernels, tensor
+    assert tensor._load_native("adrastea_amd.no_such_module") is None
+    (tmp_path / ("broken_native" + EXTENSION_SUFFIXES[0])).write_bytes(b"no shared object")
+    monkeypatch.syspath_prepend(tmp_path)
+    with pytest.raises(ImportError):
+        tensor._load_native("broken_native")
+    # without the module the kernels say so; with it they say nothing
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        GpuKernels()
+        monkeypatch.setattr(kernels, "_native", None)
+        with pytest.raises(RuntimeWarning, match="_native"):
+            GpuKernels()
