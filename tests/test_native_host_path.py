@@ -3,23 +3,35 @@ over ranks, orders and casts, what those refuse, and the argument tuples that re
 in the place of the library's functions."""
 import ctypes as C
 import itertools
+import os
+import shutil
+import sysconfig
 import warnings
 
 import pytest
 import torch
 
-from adrastea_amd import MatmulLoad, MatmulMask, MatmulOptions, MatmulStore, TensorLayout, TensorView, _ffi
-from adrastea_amd.kernels import _NATIVE_CALLS, descriptor, _lower
+from adrastea_amd import GpuKernels, MatmulLoad, MatmulMask, MatmulOptions, MatmulStore, TensorLayout, TensorView, _ffi
+from adrastea_amd import kernels
+from adrastea_amd.kernels import _NATIVE_CALLS, _bind_native, descriptor, _lower
 from adrastea_amd.tensor import _native
 
 ABI = _ffi.lib().adr_abi_version()
-pytestmark = pytest.mark.skipif(_native is None, reason="the native module is not built")
+built = pytest.mark.skipif(_native is None, reason="the native module is not built (test_the_module_is_built)")
+
+
+def test_the_module_is_built():
+    """Where it can be: the tests below say nothing of a module that is not there."""
+    if shutil.which("g++") is None or not os.path.exists(os.path.join(sysconfig.get_paths()["include"], "Python.h")):
+        pytest.skip("no C++ compiler or no headers of the interpreter")
+    assert _native is not None
 
 
 class Heads(TensorView):
     pass
 
 
+@built
 @pytest.mark.parametrize("dims", [(1,), (6,), (3, 4), (1, 5, 1), (2, 3, 4), (2, 1, 3, 2, 2, 1, 2)])
 def test_views(dims):
     t = torch.zeros(dims, dtype=torch.float16)
@@ -42,6 +54,7 @@ def test_views(dims):
     assert eight.permute(list(range(8))).layout == eight.layout
 
 
+@built
 @pytest.mark.parametrize("method,args", [
     ("permute", ([0],)), ("permute", ([0, 2],)), ("permute", ([0, 1, 1],)), ("permute", ("01",)), ("permute", (None,)),
     ("permute", ()), ("permute", ([0, 1], 2)), ("permute", ([0.0, 1],)), ("permute", ([True, False],)),
@@ -60,6 +73,7 @@ def test_unusual_arguments_do_what_the_definition_does(method, args):
     assert outcome(getattr(view, method)) == want
 
 
+@built
 def test_tensors_without_a_layout():
     for t in (torch.zeros(0, 4), torch.zeros(()), torch.zeros(1, 4).expand(3, 4)):
         with pytest.raises(ValueError):
@@ -80,7 +94,7 @@ def calls():
         keep.append(C.CFUNCTYPE(C.c_int, *types)(lambda *a, name=name: seen.append((name, a)) or 7))
     _native.bind(ABI, *(C.cast(f, C.c_void_p).value if f else 0 for f in keep), lambda: 3, lambda dev: 0x1000 + dev)
     yield seen
-    _native.bind(ABI, *([0] * len(_NATIVE_CALLS)), lambda: 0, lambda dev: 0)
+    _bind_native()   # (what every GpuKernels of this process is bound to)
 
 
 def as_ctypes(name, args):
@@ -97,6 +111,7 @@ STORES = [MatmulStore.Identity(), MatmulStore.Add(), MatmulStore.Scale(0.3),
           MatmulStore.BetaGeluBias(1, TensorView.of(torch.zeros(5, dtype=torch.float16)))]
 
 
+@built
 @pytest.mark.parametrize("store", STORES, ids=lambda s: str(s.op))
 @pytest.mark.parametrize("rank_o,rank_l,rank_r", [(2, 2, 2), (3, 3, 3), (3, 3, 2), (3, 2, 3), (4, 4, 2)])
 def test_matmul_arguments(calls, store, rank_o, rank_l, rank_r):
@@ -117,6 +132,7 @@ def test_matmul_arguments(calls, store, rank_o, rank_l, rank_r):
     assert len(calls) == 1
 
 
+@built
 @pytest.mark.parametrize("rank", [2, 3])
 def test_attention_and_softmax_arguments(calls, rank):
     def view(rows, d=64, heads=3):
@@ -140,6 +156,7 @@ def test_attention_and_softmax_arguments(calls, rank):
     assert _native.softmax_rows_inplace(TensorView.of(torch.zeros(7)), 0.5) is None
 
 
+@built
 def test_u8_and_quantisation_arguments(calls):
     m, p, n, bs = 3, 64, 5, 32
     out, x = torch.zeros(m, n, dtype=torch.float16), torch.zeros(m, p, dtype=torch.float16)
@@ -159,14 +176,18 @@ def test_u8_and_quantisation_arguments(calls):
     assert len(calls) == 3
 
 
+@built
 def test_error_stats_descriptors():
     """Callbacks take no structures by value that large: the descriptors are compared through the results
     (test_gpu_error_stats.py); here, what the native path hands back."""
     out, a = TensorView.of(torch.zeros(3)), TensorView.of(torch.zeros(4, 6, dtype=torch.float16))
     assert descriptor(a.shape_cast([-1])).shape[0] == 24
     _native.bind(ABI, *([0] * len(_NATIVE_CALLS)), lambda: 0, lambda dev: 0)
-    assert _native.error_stats(out, a, a, 0) is None
-    assert _native.error_stats(out, a, a, 2) is None
+    try:
+        assert _native.error_stats(out, a, a, 0) is None
+        assert _native.error_stats(out, a, a, 2) is None
+    finally:
+        _bind_native()
 
 
 class Interrupted:
@@ -180,6 +201,7 @@ class Interrupted:
     stride = data_ptr = is_contiguous = raised
 
 
+@built
 @pytest.mark.parametrize("what", [KeyboardInterrupt, SystemExit])
 def test_an_interrupt_is_not_taken_for_an_unusual_argument(calls, what):
     """A signal's handler runs inside the functions that the native path calls: an interrupt goes on to the caller,
@@ -216,6 +238,7 @@ def test_an_interrupt_is_not_taken_for_an_unusual_argument(calls, what):
     assert calls == []
 
 
+@built
 def test_a_tensor_without_a_shape_is_asked_no_further():
     class Strange:
         asked = 0
@@ -228,6 +251,7 @@ def test_a_tensor_without_a_shape_is_asked_no_further():
     assert Strange.asked == 0   # (the definition reads the shape first as well)
 
 
+@built
 def test_a_library_of_another_abi_is_refused():
     for abi in (ABI - 1, ABI + 1):
         with pytest.raises(RuntimeError, match="ABI version"):
@@ -250,7 +274,7 @@ def test_the_library_is_built_without_a_compiler_for_the_native_module(monkeypat
 
 def test_a_module_that_does_not_load_is_reported(tmp_path, monkeypatch):
     from importlib.machinery import EXTENSION_SUFFIXES
-    from adrastea_amd import GpuKernels, kernels, tensor
+    from adrastea_amd import tensor
     assert tensor._load_native("adrastea_amd.no_such_module") is None
     (tmp_path / ("broken_native" + EXTENSION_SUFFIXES[0])).write_bytes(b"no shared object")
     monkeypatch.syspath_prepend(tmp_path)
@@ -264,3 +288,44 @@ def test_a_module_that_does_not_load_is_reported(tmp_path, monkeypatch):
         monkeypatch.setattr(kernels, "_native", None)
         with pytest.raises(RuntimeWarning, match="_native"):
             GpuKernels()
+
+
+@built
+@pytest.mark.gpu
+def test_both_paths_give_the_same_results(monkeypatch):
+    """Every call the native path lowers, against the definitions in kernels.py, end to end."""
+    gen = torch.Generator(device="cuda").manual_seed(12)
+
+    def normal(*shape):
+        return torch.randn(*shape, dtype=torch.float16, device="cuda", generator=gen)
+
+    def heads(t):
+        return TensorView.of(t).shape_cast([t.shape[0], 3, 64]).permute([1, 0, 2])
+    x, w, bias, q, kv = normal(70, 192), normal(80, 192), normal(80), normal(33, 192), normal(50, 192)
+    options = MatmulOptions.new().store(MatmulStore.BetaBias(0.5, TensorView.of(bias)))
+    masked = MatmulOptions.new().store(MatmulStore.Scale(0.125)).load(MatmulLoad.Scale(0.5)).mask(MatmulMask.CAUSAL)
+
+    def results():
+        k, view = GpuKernels(), TensorView.of
+        product, scores, fused = torch.ones_like(normal(70, 80)), torch.ones_like(normal(3, 33, 50)), torch.ones_like(q)
+        k.matmul_f16(view(product), view(x), view(w).permute([1, 0]), options)
+        k.matmul_f16(view(scores), heads(q), heads(kv).permute([0, 2, 1]), masked)
+        k.softmax_rows_inplace(view(scores), 0.7)
+        k.attention_f16(heads(fused), heads(q), heads(kv), heads(kv), 0.125, 0.9, MatmulMask.CAUSAL)
+        u8, scales = torch.zeros(80, 192, dtype=torch.uint8, device="cuda"), torch.zeros_like(w[:, :6]).contiguous()
+        k.quantize_absmax_uint8(u8, scales, w)
+        back, by_u8 = torch.zeros_like(w), torch.ones_like(product)
+        k.dequantize_absmax_uint8(back, scales, u8)
+        k.matmul_nt_fp16u8(by_u8, x, u8, scales, 32, 0.25)
+        stats, stats32 = torch.zeros(3, device="cuda"), torch.zeros(3, device="cuda")
+        k.error_stats_f16(view(stats), view(back), view(w))
+        k.error_stats_f32(view(stats32), view(back.float()), view(w.float()))
+        return product, scores, fused, u8, scales, back, by_u8, stats, stats32
+    native = results()
+    monkeypatch.setattr(kernels, "_native", None)
+    with pytest.warns(RuntimeWarning):
+        general = results()
+    for got, want in zip(native[:-2], general[:-2]):
+        assert torch.equal(got, want)
+    for got, want in zip(native[-2:], general[-2:]):   # (sums of atomics: the order is not fixed)
+        assert torch.allclose(got, want, rtol=1e-5, atol=0)
