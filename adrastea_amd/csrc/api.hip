@@ -71,11 +71,13 @@ bool empty(const MatmulArgs& a) { return a.batches == 0 || a.m == 0 || a.n == 0;
 // a gfx950 (the kernels are built for nothing else), or the error of the failed device query.
 int check_device() { return device_info().status; }
 
-int run_matmul(hipStream_t stream, const MatmulArgs& a, bool allow_fast) {
+int run_matmul(hipStream_t stream, MatmulArgs& a, bool allow_fast) {
   if (empty(a)) return ADR_OK;
   if (int rc = check_device()) return rc;
   const char* name;
   if (allow_fast && gemv_f16_supported(a, &name)) return (int)launch_gemv_f16(stream, a);
+  // (a caller's own workspace: the choice is made here, once for both calls below; a search takes the host 2 us)
+  if (allow_fast && a.split == 0 && a.workspace_bytes > 0) (void)mfma_gemm_workspace_bytes(a, a.workspace_bytes);
   if (allow_fast && mfma_gemm_supported(a, &name)) return (int)launch_mfma_gemm(stream, a);
   return (int)launch_matmul_general(stream, a);  // also the k == 0 case: store(0)
 }
