@@ -12,6 +12,7 @@ follow the device kernels' argument lists (matmul_nt_fp16u8.cu:4-12, quantize.cu
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import threading
 import warnings
 from dataclasses import dataclass, field
@@ -188,12 +189,17 @@ _NATIVE_CALLS = ("adr_matmul_f16", "adr_attention_f16", "adr_softmax_rows", "adr
                  "adr_quantize_absmax_u8", "adr_dequantize_absmax_u8", "adr_error_stats_f16", "adr_error_stats_f32")
 
 
-def _bind_native() -> None:
-    """Hands the library's functions and torch's to the native host path (the same ones every time)."""
+@functools.lru_cache(maxsize=None)
+def _native_binding() -> tuple:
+    """The library's functions and torch's for the native host path (ctypes takes 20 us to find the addresses)."""
     import torch
     lib = _ffi.lib()
-    _native.bind(lib.adr_abi_version(), *(C.cast(getattr(lib, name), C.c_void_p).value for name in _NATIVE_CALLS),
-                 torch.cuda.current_device, torch._C._cuda_getCurrentRawStream)
+    return (lib.adr_abi_version(), *(C.cast(getattr(lib, name), C.c_void_p).value for name in _NATIVE_CALLS),
+            torch.cuda.current_device, torch._C._cuda_getCurrentRawStream)
+
+
+def _bind_native() -> None:
+    _native.bind(*_native_binding())
 
 
 class GpuKernels(CommonKernels):

@@ -329,3 +329,13 @@ def test_both_paths_give_the_same_results(monkeypatch):
         assert torch.equal(got, want)
     for got, want in zip(native[-2:], general[-2:]):   # (sums of atomics: the order is not fixed)
         assert torch.allclose(got, want, rtol=1e-5, atol=0)
+
+
+@built
+def test_the_binding_is_looked_up_once(monkeypatch):
+    """A program that makes its kernels for each state pays for the addresses once."""
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
+    kernels._native_binding.cache_clear()
+    for _ in range(3):
+        GpuKernels()
+    assert kernels._native_binding.cache_info().misses == 1
