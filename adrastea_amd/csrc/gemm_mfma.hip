@@ -1474,8 +1474,8 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
 // u8-weight kernel: left operand by DMA, weights dequantised on their way into LDS
 // =============================================================================================
 // K % 64 == 0, block size a power of two >= 8.  The fp16 left operand goes global -> LDS by DMA
-// through three stages (two slices ahead; SA = 4: four stages, three ahead).  The u8 weights of slice kt+2 are fetched into
-// registers (8 weights + their scale per chunk, three chunks per lane) while slice kt runs; the
+// through three stages, two slices ahead.  The u8 weights of slice kt+3 are fetched into registers (8 weights
+// + their scale per chunk) while slice kt runs; the
 // chunks of slice kt+1 are dequantised (bit-identical to quantize.cu:53-54) and written to one
 // of two fp16 LDS stages in the same swizzled layout the DMA produces, so that every weight is
 // dequantised once per workgroup and the MFMA loop is the one of the fp16 kernel.
@@ -1491,7 +1491,7 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
 // leave (weights from HBM, us: K11008 N4096 m=160 55.0 -> 47.1, 384 81.5 -> 70.3, K13824 N5120 m=96 66.8 -> 57.7,
 // K4096 N12288 m=64 29.0 -> 27.1, 1536 179 -> 172); without the fence the left operand's moved back as well, and the
 // large tiles lost 10-15 %.
-template <int BM, int BN, int WM, int WN, bool MI16, int BK = 64, int G = 1, int SA = 3>
+template <int BM, int BN, int WM, int WN, bool MI16, int BK = 64, int G = 1>
 __global__ __launch_bounds__(WM* WN* G * 64, 1) void gemm_nt_u8_kernel(MatmulArgs a, TileMap map,
                                                                       int block_shift) {
   constexpr int CPR = BK / 8, MI = MI16 ? 16 : 32, KG = 64 / MI, KK = CPR / KG;
@@ -1514,8 +1514,6 @@ __global__ __launch_bounds__(WM* WN* G * 64, 1) void gemm_nt_u8_kernel(MatmulArg
   __shared__ __attribute__((aligned(1024))) unsigned char sA0[G * BM * BK * 2];
   __shared__ __attribute__((aligned(1024))) unsigned char sA1[G * BM * BK * 2];
   __shared__ __attribute__((aligned(1024))) unsigned char sA2[G * BM * BK * 2];
-  __shared__ __attribute__((aligned(1024))) unsigned char sA3[SA == 4 ? G * BM * BK * 2 : 1024];
-  static_assert(SA == 3 || SA == 4, "three stages of the left operand (two slices ahead) or four (three ahead)");
   __shared__ __attribute__((aligned(1024))) unsigned char sB0[G * BN * BK * 2];
   __shared__ __attribute__((aligned(1024))) unsigned char sB1[G * BN * BK * 2];
 
@@ -1572,9 +1570,9 @@ __global__ __launch_bounds__(WM* WN* G * 64, 1) void gemm_nt_u8_kernel(MatmulArg
     for (int i = 0; i < IA; i++)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, ADR_LDS_PTR(dA + goA + (i * NW + wave) * 1024), 16, (int)gA[i], k0 * 2, 0, 0);
   };
-  // three register sets: the weights consumed in slice kt+1 were requested at the head of slice
-  // kt-1, so the wait at the end of slice kt-1 (everything but that slice's own requests)
-  // already covers them and nothing in slice kt waits for a load issued a moment ago
+  // three register sets: the weights dequantised in slice kt were requested in slice kt-2, so the wait at the end
+  // of slice kt-1 (everything but that slice's own requests) already covers them and nothing in slice kt waits
+  // for a load issued a moment ago
   u32x2_t rq[3][LB];
   half_t rs[3][LB];
   auto fetchQ = [&](int set) {
@@ -1667,34 +1665,38 @@ __global__ __launch_bounds__(WM* WN* G * 64, 1) void gemm_nt_u8_kernel(MatmulArg
     }
     // A(kt+1) has landed: only the weight fetch and the DMA issued in this slice may still be
     // in flight; the dequantised weights of slice kt+1 are in LDS
-    // (four A stages: the transfer issued in the slice before, which is younger than that slice's
-    // weight requests, may stay in flight too)
+    // (The weights that the last two slices behind the loop request are used by none, and the compiler drops
+    // them: the count then covers a transfer of this slice and the weight requests of the slice before, which are
+    // younger than that slice's transfer.  Neither weights nor transfers move past the fences of their slice.)
+    // (A fourth stage of A, its transfers three slices ahead, had gained 5 % on 256 x 128 while the weights
+    // were requested first; behind the transfers it gains nothing with three register sets of weights, as the wait
+    // for a slice's weights covers the older transfer, nor with four, as its shorter period of 4 slices was
+    // measured to: K11008 N4096 m=2048 174.2 us with three stages, 173.7 with four, 175.7 with four of either; K4096
+    // N4096 70.5, 71.8, 71.6; K4096 N11008 m=512 58.5, 60.5, 60.4; K5120 N5120 m=1280 76.6, 78.3, 79.5.)
     __builtin_amdgcn_sched_barrier(0x38F);
-    constexpr int n = 2 * LB + (SA - 2) * IA;
+    constexpr int n = 2 * LB + IA;
     __builtin_amdgcn_s_waitcnt(0x0070 | (n & 0xF) | ((n >> 4) << 14));
     __builtin_amdgcn_s_barrier();
     load_frags(0, nA, nB, 0);
   };
 
-  // slice kt (kt % P == p) reads A stage p % SA and B stage p % 2, dequantises register set
+  // slice kt (kt % 6 == p) reads A stage p % 3 and B stage p % 2, dequantises register set
   // (p + 1) % 3 into the other B stage, refills the A stage read one slice earlier with slice
-  // kt + SA - 1 and register set p % 3 with the weights of slice kt + 3
-  auto stA = [&](int i) -> unsigned char* { return i == 0 ? sA0 : i == 1 ? sA1 : i == 2 ? sA2 : sA3; };
+  // kt + 2 and register set p % 3 with the weights of slice kt + 3
+  auto stA = [&](int i) -> unsigned char* { return i == 0 ? sA0 : i == 1 ? sA1 : sA2; };
   auto stB = [&](int i) -> unsigned char* { return i == 0 ? sB0 : sB1; };
-  constexpr int P = SA == 3 ? 6 : 12;  // the common period of the stages and the register sets
+  constexpr int P = 6;  // the common period of the stages and the register sets
   auto slice_p = [&](int p) {
-    slice(stA(p % SA), stB(p % 2), stA((p + 1) % SA), stB((p + 1) % 2), stA((p + SA - 1) % SA), p % 3,
-          (p + 1) % 3);
+    slice(stA(p % 3), stB(p % 2), stA((p + 1) % 3), stB((p + 1) % 2), stA((p + 2) % 3), p % 3, (p + 1) % 3);
   };
   fetchQ(0);
   fetchQ(1);
   dmaA(sA0);
   fetchQ(2);
   dmaA(sA1);
-  if (SA == 4) dmaA(sA2);
   dequant_store(0, sB0);
   {
-    constexpr int n = (SA - 2) * IA;
+    constexpr int n = IA;
     __builtin_amdgcn_s_waitcnt(0x0070 | (n & 0xF) | ((n >> 4) << 14));
     __builtin_amdgcn_s_barrier();
   }
@@ -2270,11 +2272,11 @@ hipError_t launch_stage(hipStream_t stream, const MatmulArgs& a) {
   return hipGetLastError();
 }
 
-template <int BM, int BN, int WM, int WN, bool MI16, int BK = 64, int G = 1, int SA = 3>
+template <int BM, int BN, int WM, int WN, bool MI16, int BK = 64, int G = 1>
 hipError_t launch_u8(hipStream_t stream, const MatmulArgs& a) {
   TileMap map = make_map(a, BM, BN);
   if (map.total < 0 || a.k % (BK * G) != 0) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((gemm_nt_u8_kernel<BM, BN, WM, WN, MI16, BK, G, SA>), dim3((unsigned)map.total),
+  hipLaunchKernelGGL((gemm_nt_u8_kernel<BM, BN, WM, WN, MI16, BK, G>), dim3((unsigned)map.total),
                      dim3(WM * WN * G * 64), 0, stream, a, map, __builtin_ctz(a.block_size));
   return hipGetLastError();
 }
@@ -2670,9 +2672,7 @@ static hipError_t launch_choice(hipStream_t stream, const MatmulArgs& a, GemmCho
     case SHORTK_64: return launch_shortk<8>(stream, a);
     case SHORTK_128: return launch_shortk<16>(stream, a);
     case U8_256x192: return launch_u8<256, 192, 4, 2, true>(stream, a);
-    // (four stages of the left operand, three slices ahead, fill the 160 KB: K11008 N4096 M2048 with
-    // weights from HBM 202 -> 191 us, K4096 unchanged; the smaller tiles gain nothing from a fourth stage)
-    case U8_256x128: return launch_u8<256, 128, 4, 2, true, 64, 1, 4>(stream, a);
+    case U8_256x128: return launch_u8<256, 128, 4, 2, true>(stream, a);
     case U8_128x128: return launch_u8<128, 128, 4, 2, true>(stream, a);
     case U8_128x64: return launch_u8<128, 64, 2, 2, true>(stream, a);
     case U8_64x64: return launch_u8<64, 64, 2, 2, true>(stream, a);
