@@ -1084,7 +1084,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(MatmulArgs a, TileMa
 // A workgroup with T tiles passes 2T + 2 barriers in every role.  The right panel of tile j is read
 // in phases 2j and 2j+1 and its buffer refilled (tile j+3) in phase 2j+2.  Both groups copy the
 // left panel of a new segment in the even phase of its first tile (the lower group's registers
-// are free by then), and the loader refills that buffer for the next segment one phase later.
+// are free by then; of a segment that is all hidden under the mask, whatever the buffer holds, for nobody), and the loader refills that buffer for the next segment one phase later.
 struct ShortKMap {
   int tiles_m, tiles_n, rows;   // rows = batches * tiles_m
   int seg, segs_per_row, units; // a unit is `seg` consecutive tiles of one tile row
@@ -1102,7 +1102,9 @@ __device__ __forceinline__ void wait_vmcnt_at_most() {
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 0xF) | ((N >> 4) << 14));
 }
 
-template <int CPR>  // 16-byte chunks per row: 8 (K = 64) or 16 (K = 128)
+// CPR: 16-byte chunks per row: 8 (K = 64) or 16 (K = 128).  DIRECT: the writers store the -inf of hidden tiles by
+// themselves (launch_shortk; a template parameter because a flag that they look at takes 10 % of a small result's time)
+template <int CPR, bool DIRECT>
 __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(MatmulArgs a,
                                                                            ShortKMap map) {
   constexpr int BM = 128, BN = 128, NWL = SHORTK_LOADERS, NWW = SHORTK_WRITERS;
@@ -1122,11 +1124,13 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
   // Workgroup g runs on die g % 8: the workgroups of a die take neighbouring units (they share
   // right panels in the die's L2).  Odd rounds walk the workgroups backwards, which pairs long
   // and short rows of a causal product.
-  // Tiles above the diagonal of a causal product take their turn like the others, less the MFMAs: -inf
-  // goes through the staging tile.  The launch is bound by its writes, and those of a unit follow each other this
-  // way; the hidden tiles as whole rows by the writers, behind or before the others of a unit, or in a launch of
-  // their own took longer (us: a launch of its own / rows by the writers / this; 32 heads of 128, 1024 keys 31.4 /
-  // 34.5 / 15.9, 513 52.7 / 39.2 / 19.9, 2048 75.7 / 72.3 / 67.5; 20 heads of 64, 1500 50.9 / 74.3 / 45.0).
+  // Tiles above the diagonal of a causal product (hidden()) take their turn like the others, but nothing is read or
+  // multiplied for them: -inf goes through the staging tile, or straight to memory (DIRECT).  The
+  // launch is bound by its writes, and those of a unit follow each other this way; in a model the cache it writes into
+  // is full of the softmax of the layer before, and the panels that were read for hidden tiles took their part of the
+  // memory's time (us of the three calls of attention in a row, with the hidden rows written by a launch of their
+  // own ahead of this one / hidden tiles with their panels / without: 32 heads of 128, 2048 keys 255 / 258 / 246, 1984 222 /
+  // 227 / 216, 1536 152 / 144 / 136, 1024 80.5 / 70.0 / 69.2; 40 of 128, 1600 234 / 230 / 218).
   const int XCDS = map.xcds;
   const int gl = G % XCDS == 0 ? (blockIdx.x % XCDS) * (G / XCDS) + blockIdx.x / XCDS : blockIdx.x;
 
@@ -1156,6 +1160,7 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
     if (c.valid && c.n >= c.n_end) { c.t++; load_unit(c); c.first = true; }
   };
   const bool causal = a.mask == ADR_MASK_CAUSAL;
+  auto hidden = [&](const Cursor& c) { return causal && c.n * BN > c.m0 + BM - 1; };  // (and then the rest of its unit)
   // Identity and Scale need neither the previous output nor the bias (the fp16 product x * 1 is exact: one
   // multiply serves both).  With a positive factor the mask is applied where the results are staged, by eight
   // wavefronts instead of the two that write: -inf stays -inf.
@@ -1194,16 +1199,23 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
     Cursor is = cur;  // next right panel to issue
     auto issued_into = [&](int byte) { age = (age + 0x01010101u) & ~(0xFFu << (8 * byte)); };
     auto younger_than = [&](int byte) { return (int)((age >> (8 * byte)) & 0xFFu); };
+    // a buffer that nothing is transferred to: older than any count of groups in flight
+    auto nothing_into = [&](int byte) { age = (age & ~(0xFFu << (8 * byte))) | 0x40u << (8 * byte); };
     auto issue_left = [&](const Cursor& c) {
+      if (hidden(c)) return nothing_into(3);  // (the unit's first tile)
       panel(a.lhs + (int64_t)c.batch * a.stride_lz, a.stride_ly, c.m0, a.m - 1, sA);
       issued_into(3);
     };
     auto issue_right = [&]() {
       if (!is.valid) return;
       const int slot = right_issued % RING;
-      panel(a.rhs + (int64_t)is.batch * a.stride_rz, a.stride_rx, is.n * BN, a.n - 1,
-            sB + slot * PANEL);
-      issued_into(slot);
+      if (hidden(is)) {
+        nothing_into(slot);
+      } else {
+        panel(a.rhs + (int64_t)is.batch * a.stride_rz, a.stride_rx, is.n * BN, a.n - 1,
+              sB + slot * PANEL);
+        issued_into(slot);
+      }
       right_issued++;
       next_item(is);
     };
@@ -1249,6 +1261,35 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
     Epilogue ep{a.bias, a.beta, hscale, a.store, true};
     const int walign = out_chunk_alignment(a, a.output);
     const bool vec = walign >= 2;
+    // Half of a hidden tile, straight to memory.  Chunks of eight from the first 16-byte boundary of the tile in each
+    // row: the last one may reach into the next tile, which is hidden too and leaves that much to this one; what lies
+    // before the boundary is this tile's only if the tile on its left is not hidden, what is left of a row behind its
+    // last whole chunk is the tile's that chunk would begin in.  Either is one more store, of an element a lane.
+    // (no nontemporal stores: the lines that two chunks share are put together in the L2)
+    auto write_hidden = [&](int batch, int m0, int n0, int half) {
+      const int y0 = m0 + half * 64 + sw * WROWS + rrow;
+      const int64_t step = 4 * (int64_t)a.stride_oy;
+      half_t* const p = a.output + (int64_t)batch * a.stride_oz + (int64_t)y0 * a.stride_oy + n0;
+      auto head = [&](int it) { return (int)(-(uintptr_t)(p + it * step) >> 1) & 7; };  // halves before the boundary
+      const half_t ninf = neg_inf_half();
+      const half8_t v = {ninf, ninf, ninf, ninf, ninf, ninf, ninf, ninf};
+      if (n0 - BN <= m0 + BM - 1) {
+#pragma unroll
+        for (int it = 0; it < WIT; it++)
+          if (rc < head(it) && n0 + rc < a.n && y0 + it * 4 < a.m) p[it * step + rc] = ninf;
+      }
+      if (y0 - rrow + WROWS <= a.m && n0 + BN + 7 <= a.n) {
+#pragma unroll
+        for (int it = 0; it < WIT; it++) *(half8_t*)(p + it * step + head(it) + rc * 8) = v;
+        return;
+      }
+#pragma unroll
+      for (int it = 0; it < WIT; it++) {
+        const int h = head(it), left = y0 + it * 4 < a.m ? a.n - n0 - h : 0;  // elements of the row from the boundary on
+        if (rc * 8 + 8 <= left) *(half8_t*)(p + it * step + h + rc * 8) = v;
+        if (left > 0 && left < BN && rc < (left & 7)) p[it * step + h + (left & ~7) + rc] = ninf;
+      }
+    };
     auto write_half = [&](int batch, int m0, int n0, int half) {
       const int r0 = half * 64 + sw * WROWS;  // first of this wavefront's rows in the tile
       auto staged = [&](int it) {
@@ -1335,10 +1376,13 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
           __builtin_amdgcn_s_barrier();  // barrier 1
           started = true;
         }
+        const bool nothing_staged = DIRECT && hidden(c);
         __builtin_amdgcn_s_barrier();  // barrier 2j+2: the upper half of tile j is staged
-        write_half(c.batch, c.m0, c.n * BN, 0);
+        if (nothing_staged) write_hidden(c.batch, c.m0, c.n * BN, 0);
+        else write_half(c.batch, c.m0, c.n * BN, 0);
         __builtin_amdgcn_s_barrier();  // barrier 2j+3: the lower half
-        write_half(c.batch, c.m0, c.n * BN, 1);
+        if (nothing_staged) write_hidden(c.batch, c.m0, c.n * BN, 1);
+        else write_half(c.batch, c.m0, c.n * BN, 1);
       }
       c.t++;
       load_unit(c);
@@ -1445,7 +1489,7 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
       if (visible()) multiply(sB + (j % RING) * PANEL);
       __builtin_amdgcn_s_waitcnt(0xC07F);  // the panel has been read (lgkmcnt 0)
       __builtin_amdgcn_s_barrier();  // barrier 2j+1: this half of the staging tile is free
-      narrow(below());
+      if (!DIRECT || !hidden(c)) narrow(below());
       __builtin_amdgcn_s_waitcnt(0xC07F);  // staged
       next_item(c);
     }
@@ -1461,8 +1505,9 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
       __builtin_amdgcn_s_waitcnt(0xC07F);
       __builtin_amdgcn_s_barrier();  // barrier 2j+2: the ring buffer of tile j is free
       const int tile_below = below();
+      const bool staged = !DIRECT || !hidden(c);
       next_item(c);
-      narrow(tile_below);
+      if (staged) narrow(tile_below);
       if (c.valid && c.first) copy_left();  // tile j+1 opens a unit: its left panel has landed
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);
@@ -2310,7 +2355,19 @@ hipError_t launch_shortk(hipStream_t stream, const MatmulArgs& a) {
   map.segs_per_row = (map.tiles_n + map.seg - 1) / map.seg;
   map.units = map.rows * map.segs_per_row;
   const unsigned grid = map.units < NUM_CU ? (unsigned)map.units : NUM_CU;
-  hipLaunchKernelGGL((gemm_nt_shortk_kernel<CPR>), dim3(grid), dim3(SHORTK_THREADS), 0, stream, a, map);
+  // Rows that are no whole 128-byte lines share lines between tiles; large results of such rows are bound by writing
+  // parts of lines, and get their hidden tiles in aligned 16-byte pieces that the L2 puts together.
+  // us of the three calls of attention in a row under the mask, hidden tiles staged / direct: 32 heads of 128, 1025
+  // keys 127.2 / 121.6, 1100 131.7 / 130.2, 1501 213 / 196, 1800 240 / 212, 1900 293 / 260, 2047 444 / 377; 40 heads of 128,
+  // 1590 297 / 273; 20 heads of 64, 1500 110.3 / 106.2; 16 of 64, 1999 182 / 147.  Below 64 MB the caches do that by
+  // themselves and staging is as good or better (32 heads of 128, 400 26.3 / 28.5, 513 50.1 / 51.4, 900 71.2 / 72.5; 40 of
+  // 128, 800 69.9 / 73.7; 16 of 64, 1250 74.0 / 76.9; 12 of 64, 1100 56.8 / 55.3), and so it is for whole lines (32 of 128,
+  // 2048 245.5 / 243.1, alone 72 / 94; 1600 of 40 heads 217 / 223; 1024 69.1 / 71.2).
+  const bool lines = ((uintptr_t)a.output | 2 * (uintptr_t)a.stride_oy | (a.batches > 1 ? 2 * (uintptr_t)a.stride_oz : 0)) % 128 == 0;
+  if (a.mask == ADR_MASK_CAUSAL && !lines && (int64_t)a.batches * a.m * a.n >= 32 << 20)
+    hipLaunchKernelGGL((gemm_nt_shortk_kernel<CPR, true>), dim3(grid), dim3(SHORTK_THREADS), 0, stream, a, map);
+  else
+    hipLaunchKernelGGL((gemm_nt_shortk_kernel<CPR, false>), dim3(grid), dim3(SHORTK_THREADS), 0, stream, a, map);
   return hipGetLastError();
 }
 

@@ -1,5 +1,5 @@
-"""Causal score products on the persistent kernel (K = 64, 128): hidden tiles take their turn with the others, and the
-mask is applied where results are staged (Identity, and Scale with a positive factor) or where they are written (every
+"""Causal score products on the persistent kernel (K = 64, 128): hidden tiles take their turn with the others, staged or (large
+results whose rows are no whole 128-byte lines) in aligned pieces whatever the rows' alignment, and the mask is applied where results are staged (Identity, and Scale with a positive factor) or where they are written (every
 other operator and factor).  Against the step-for-step kernel on the same device, bit for bit: the inputs are
 dyadic and the sums exact."""
 import pytest
@@ -48,3 +48,38 @@ def test_causal_scores_match_the_step_for_step_kernel(shape, k):
         assert bad.numel() == 0, (store, scale, load, bad[:4].tolist())
         rows, cols = torch.arange(m, device="cuda")[:, None], torch.arange(n, device="cuda")[None, :]
         assert bool((got[:, :, :n][:, cols > rows] == float("-inf")).all())
+
+
+# 2^25 results and more (direct): rows of every remainder of 8, several hidden tiles in a row, keys that end in the last
+# piece of a tile, one behind it and inside a tile, a last tile row of one row; and smaller ones (staged)
+HIDDEN = [(109, 300, 1031 + i, i) for i in range(8)] + [(376, 140, 640, 3), (502, 129, 519, 1), (502, 129, 520, 1),
+          (64, 128, 4097, 2), (64, 129, 4096, 64), (63, 128, 4097, 2), (65, 128, 4080, 3)]
+
+
+@pytest.mark.parametrize("k", [64, 128])
+@pytest.mark.parametrize("shape", HIDDEN, ids=lambda s: "h%d_m%d_n%d_pad%d" % s)
+def test_hidden_tiles_are_written_to_the_last_element_and_no_further(shape, k):
+    """Results at every offset from a 16-byte boundary: the whole buffer against the step-for-step kernel's, and what
+    is no element of the result (the pad of the rows, the space before and behind it) as it was."""
+    heads, m, n, pad = shape
+    width = n + pad
+    size = heads * m * width
+    args = (heads, m, k, n, 1, width, m * width, 1, heads * k, k, heads * k, 1, k)
+    gen = torch.Generator(device="cuda").manual_seed(n + k)
+
+    def dyadic(*shape_):
+        return (torch.randint(-8, 9, shape_, generator=gen, device="cuda") / 8.0).half()
+    q, keys, bias = dyadic(m, heads * k), dyadic(n, heads * k), dyadic(n)
+    for offset in range(8):   # (of the buffer; with whole lines in a row the first one is staged)
+        prev = torch.full((size + 80,), 5.0, dtype=torch.float16, device="cuda")
+        assert prev.data_ptr() % 128 == 0
+        got, want = prev.clone(), prev.clone()
+        store, scale, beta = [(0, 1.0, 0.0), (4, 0.125, 0.0), (4, -0.5, 0.0), (3, 1.0, 0.5)][offset % 4]
+        call("adr_matmul_f16", got[64 + offset:], q, keys, args, bias, beta, scale, store, 0)
+        call("adr_matmul_f16_slow", want[64 + offset:], q, keys, args, bias, beta, scale, store, 0)
+        same = (got.view(torch.int16) == want.view(torch.int16)) | ((got == 0) & (want == 0))
+        bad = (~same).nonzero()
+        assert bad.numel() == 0, (offset, bad[:4].tolist())
+        inside = got[64 + offset:64 + offset + size].view(heads, m, width)
+        assert bool((inside[:, :, n:] == 5.0).all()) and bool((got[:64 + offset] == 5.0).all())
+        assert bool((got[64 + offset + size:] == 5.0).all())
