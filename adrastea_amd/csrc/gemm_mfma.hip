@@ -2421,13 +2421,12 @@ const Candidate DMA_TILES[] = {
     {DMA_64x64, 64, 64, 4, 0.40f}, {DMA_256x160, 256, 160, 1, 1.19f}};
 constexpr int N_DMA_TILES = sizeof(DMA_TILES) / sizeof(DMA_TILES[0]);
 
-// The tiles of the u8-weight kernel.  One tile per CU, time per tile at K 11008 / K 4096 in us:
-// 256x192 195 / 78, 256x128 140 / 56, 128x128 97 / 41, 128x64 68 / 30 (two K groups; one: 73 / 32),
-// 64x64 47 / 22 (four K groups; one: 58 / 25).  The two smallest tiles are bound by what the L2s
-// deliver to all CUs together (M256 K11008 N4096 on 64x64: 540 MB in 47 us), the larger ones by
-// the path into one CU.  Over M 70..1536 x (K, N) of the LLaMA-7B and 13B layers the choice by
-// these constants is the fastest forced tile or within 5 % of it, with the weights resident in
-// the Infinity Cache and with weights that come from HBM (rotated through 600 MB) alike.
+// The tiles of the u8-weight kernel.  One tile on every CU, weights from HBM, us at K 11008 / K 4096: 256x192 210 / 93
+// (176 and 232 tiles), 256x128 179 / 72, 128x128 114 / 47, 128x64 77 / 31 (two K groups; one: 87 / 35), 64x64
+// 50 / 23 (four K groups; one: 71 / 30).  The two smallest tiles are bound by what the L2s deliver to all CUs
+// together (M256 K11008 N4096 on 64x64: 540 MB in 50 us), the larger ones by the path into one CU.  Over M 65 .. 1536
+// x (K, N) of the LLaMA-7B and 13B layers (181 products that are tiled) the choice by these constants is the fastest
+// forced tile or within 3 % of it.
 const Candidate U8_TILES[] = {{U8_256x192, 256, 192, 1, 1.10f}, {U8_256x128, 256, 128, 1, 1.05f},
                               {U8_128x128, 128, 128, 1, 0.72f}, {U8_128x64, 128, 64, 2, 0.52f},
                               {U8_64x64, 64, 64, 4, 0.37f}};
@@ -2881,16 +2880,18 @@ const char* gemm_u8_mfma_plan(int m, int p, int n, int block_size) {
 }
 
 // Estimated time of the u8 product on the tiled u8 kernel, in us (negative: that kernel does not
-// cover it): pick()'s cost of the chosen tile times K.  4 us + 4.3e-7 us per unit is 10-15 % above what one
-// tile per CU of 64 x 64 (K11008 43-50 us, K4096 20-23) and of 128 x 64 (67-73, 28-30) takes on weights that
-// come from HBM: where this is compared with the passes of 64 rows the two are that close (K11008 m=72 42.5 us
-// tiled and 41.4 in passes, 96 46.4 and 44.5, 128 49.8 and 52.5), and the passes keep the tie.
+// cover it): pick()'s cost of the chosen tile times K, 4 us + 4.3e-7 us per unit, weights from HBM.  One row of
+// tiles, or tiles on less than half of the compute units, take a tenth more (K5120 N5120 m=64 32.0 us, K5120 N1280
+// m=128 29.4, K1024 N4096 m=64 10.5), more tiles some 6 % less (K4096 N4096 m=96 22.0, K11008 N4096 m=128 50.9).
 double gemm_u8_mfma_estimate_us(int m, int p, int n, int block_size) {
   const MatmulArgs a = u8_args(nullptr, nullptr, (const uint8_t*)16, nullptr, m, p, n, block_size, 0.0f);
   if (!(p % 64 == 0 && block_size >= 8 && (block_size & (block_size - 1)) == 0)) return -1.0;
   double cost;
-  pick(a, U8_TILES, N_U8_TILES, &cost);
-  return 4.0 + cost * p * 4.3e-7;
+  const GemmChoice c = pick(a, U8_TILES, N_U8_TILES, &cost);
+  int64_t tiles = 0;
+  for (const Candidate& t : U8_TILES)
+    if (t.id == c) tiles = (int64_t)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
+  return (4.0 + cost * p * 4.3e-7) * (m > 64 && 2 * tiles >= num_cu() ? 0.94 : 1.1);
 }
 
 bool gemm_u8_mfma_supported(const half_t* lhs, const uint8_t* rhs, const half_t* scales, int m, int p,

@@ -728,14 +728,16 @@ U8Choice choose_u8(const void* lhs, const void* rhs, const void* scales, int m, 
 
 // 17 activation rows and more against at least 4 MiB of weights: passes of up to 64 rows on the
 // matrix-core streaming kernels, each pass reading the weights once.  A pass of 64 rows is one
-// workgroup per sixteen weight rows, 2 + 0.0023 K us per round of them over the CUs (K4096 N4096
-// 13.1 us, N8192 23.5, N12288 33.9, K11008 N4096 26.4, K5120 N5120 25.7); a last pass of r rows
-// costs 0.55 + 0.45 r / 64 of that.  Up to 32 rows the passes always win (K4096 N12288 m=32 18 us
-// against 25 on 64 x 64 tiles); above, where this estimate is below the tiled kernel's own.
-// Measured with weights that come from HBM, us in passes and tiled: K11008 N4096 m=64 26 and 53, m=96 44.5 and
-// 46.4, m=128 52.5 and 49.8, m=160 71 and 47; K4096 N4096 m=96 22.5 and 21.4, m=128 25.3 and 22.7, m=160 36 and 22;
-// wide matrices are tiled from 33 rows (K4096 N12288 m=64 34 and 27, m=70 47 and 30), 13B-sized narrow ones from 65
-// (K13824 N5120 m=64 57 and 66, m=70 78 and 52).
+// workgroup per sixteen weight rows, 2.7 us + 2.5 + 0.00192 K us per round of them over the CUs, 5 % less where the
+// last round is half empty or more (K4096 N4096 13.1 us, N8192 23.8, N12288 33.7, K11008 N4096 26.4, K5120 N5120 25.8,
+// K13824 N5120 57.8, K1024 N4096 6.2); a last pass of r rows costs 0.55 + 0.45 r / 64 of that.  Up to 32 rows the
+// passes always win (K4096 N12288 m=32 18 us against 25 on 64 x 64 tiles); above, where this estimate is below the
+// tiled kernel's own.  Of 392 products (24 matrices of K 1024 .. 14336, N 1024 .. 22016, 33 .. 256 rows, weights from
+// HBM) the choice costs 7 % on two (K1280 N5120, 56 and 64 rows) and 4 % or less on the others.
+// us in passes and tiled: K11008 N4096 m=64 26 and 42, m=96 44.5 and 47.8, m=112 48.9 and 49.7, m=128 52.8 and 50.9, m=160
+// 71 and 48; K4096 N4096 m=72 21.7 and 20.9, m=96 22.9 and 22.0, m=128 26.1 and 23.3; K1024 N4096 m=64 6.2 and 10.5;
+// wide matrices are tiled from 33 rows (K4096 N12288 m=64 34 and 26, m=72 47 and 30), 13B-sized narrow ones from 65
+// (K13824 N5120 m=64 58 and 67, m=72 78 and 52).
 bool rows_in_passes(int m, int p, int n, int block_size) {
   if (m <= 16 || m > 256 || (int64_t)n * p < (1 << 22) ||
       choose_u8(nullptr, nullptr, nullptr, 16, p, n, block_size) != U8_GEMV)
@@ -748,8 +750,8 @@ bool rows_in_passes(int m, int p, int n, int block_size) {
   // second round: K6656 N17920 m=40 57.5 us against 73.6, K8192 N22016 m=48 74 against 89 (weights
   // from HBM; with four blocks the pass loses: m=64 104 against 92)
   if (m <= 48 && (n + 63) / 64 > cus) return true;
-  const int rounds = ((n + ROWS - 1) / ROWS + cus - 1) / cus;
-  const double t64 = fmax(12.0, rounds * (2.0 + 0.0023 * p));
+  const int groups = (n + ROWS - 1) / ROWS, rounds = (groups + cus - 1) / cus, last = groups % cus;
+  const double t64 = (2.7 + rounds * (2.5 + 0.00192 * p)) * (last && 2 * last <= cus ? 0.95 : 1.0);
   const int rem = m % 64;
   const double passes = (m / 64) * t64 + (rem ? t64 * (0.55 + 0.45 * rem / 64.0) : 0.0);
   const double tiled = gemm_u8_mfma_estimate_us(m, p, n, block_size);

@@ -252,3 +252,20 @@ def test_held_workspace_controls():
         assert A.held_workspace_declined() == lib.adr_held_workspace_declined() >= 0
     finally:
         lib.adr_set_held_workspace_limit(before)
+
+
+def test_u8_passes_and_tiles():
+    """Where the passes of 64 rows give way to the tiled kernel, on both sides of the line: a second pass against 128
+    tiles or more, one row of tiles against a short K, tiles that are few."""
+    lib = _ffi.lib()
+
+    def passes(m, p, n):
+        buf = C.create_string_buffer(96)
+        assert lib.adr_matmul_nt_fp16u8_plan(buf, 96, m, p, n, 32) == 0
+        return buf.value.startswith(b"gemv_u8_mfma16")
+    assert passes(72, 4096, 4096) and not passes(96, 4096, 4096) and not passes(112, 4096, 4096)
+    assert passes(112, 8192, 4096) and not passes(144, 8192, 4096)
+    assert passes(33, 1024, 4096) and passes(64, 1024, 4096) and not passes(72, 1024, 4096)
+    assert passes(48, 1280, 5120) and not passes(72, 1280, 5120)
+    assert passes(64, 5120, 5120) and not passes(72, 5120, 5120)
+    assert passes(128, 5120, 1280) and passes(128, 4096, 1024)
