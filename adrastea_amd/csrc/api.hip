@@ -574,12 +574,13 @@ int adr_matmul_nt_f16(adr_stream_t stream, uint16_t* output, const uint16_t* lhs
   return nt_f16(stream, output, lhs, rhs, m, p, n, beta, true);
 }
 
-// Where dequantising the matrix once and running the fp16 kernels beats the fused kernels
-// (measured over M 64 .. 4096 on (K, N) of the LLaMA-7B and 13B layers): from 768 rows on.  Below,
-// the fused kernel's small tiles are 5-80 % ahead (K11008 N4096 M512 73 against 84 us, M256 46
-// against 63; K4096 N12288 M128 31 against 50); at 768 and 1024 rows the two are within 5 % of each
-// other either way; from 1536 rows on the fused kernel dequantises every weight six times and more
-// and is 6-25 % behind (K4096 N12288 M2048 218 against 185 us).
+// From how many rows on the matrix is dequantised once and the fp16 kernels run on it, where a workspace or
+// adr_set_u8_dequantise_first allows it.  Measured over M 384 .. 4096 on the eight (K, N) of the LLaMA-7B and 13B layers,
+// weights from HBM, this route's time over the fused kernels': 0.89-1.44 at 384 and 512 rows, 0.92-1.21 at 768, 0.97-1.14 at
+// 1024, 0.87-1.05 at 1152 and 1280, 0.86-1.05 at 1536, 0.92-1.02 at 1792, 0.90-1.02 at 2048, 0.86-0.95 from 3072 on; wide
+// matrices (N 11008 and more) are the upper ends to 1280 rows (K4096 N12288 M1024 110 against 101 us, M2048 190 against
+// 196).  The line dates from fused tiles that took 10-25 % longer, when the two were level at 768 rows and this route 6-25
+// % ahead from 1536; it stays because callers size their buffers by it.
 static bool u8_dequantise_first(int m, int p, int n) {
   (void)n;
   return m >= 768 && p > 0;

@@ -350,8 +350,8 @@ class GpuKernels(CommonKernels):
                                                 rhs_q.data_ptr(), scales.data_ptr(), m, p, n,
                                                 block_size, beta)
         else:
-            # with a workspace of n * p * 2 bytes or more, products of 129 rows and more may
-            # dequantise the matrix once and run the fp16 kernels (same bits, less time)
+            # with a workspace of n * p * 2 bytes or more, products of 768 rows and more dequantise
+            # the matrix once and run the fp16 kernels (same bits)
             rc = self._lib.adr_matmul_nt_fp16u8_ws(_current_stream(), output.data_ptr(), lhs.data_ptr(),
                                                    rhs_q.data_ptr(), scales.data_ptr(), m, p, n,
                                                    block_size, beta, self._workspace.data_ptr(),
