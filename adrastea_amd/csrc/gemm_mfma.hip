@@ -599,10 +599,11 @@ __global__ __launch_bounds__(WM* WN * 64, MINB) void gemm_nt_dma_kernel(MatmulAr
   constexpr int CPR = BK / 8, KK = CPR / KG;   // k-steps per slice: of 16 k (32x32x16) or 32 k
   static_assert(BK == 64 || (BK == 128 && !NN && NSTAGE == 3), "slices of 64, or 128 with three stages");
   constexpr int NW = WM * WN, NT = NW * 64;
-  // DMA instructions per thread and slice.  NSTAGE == 6 (two left + four right stages) and
-  // NSTAGE == 7 (three left + four right): the first half of the wavefronts issues all transfers
-  // of the left operand, the second half all of the right one (NWD each)
-  constexpr int NWD = NSTAGE >= 6 ? NW / 2 : NW;
+  // DMA instructions per thread and slice.  NSTAGE == 4 (two left + three right stages), 5 (five of
+  // each), 6 (two left + four right) and 7 (three left + four right): the first half of the wavefronts
+  // issues all transfers of the left operand, the second half all of the right one (NWD each)
+  constexpr bool ROLES = NSTAGE >= 4;
+  constexpr int NWD = ROLES ? NW / 2 : NW;
   constexpr int IA = BM * CPR / (NWD * 64), IB = BN * CPR / (NWD * 64);
   constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
   constexpr int FM = WTM / MI, FN = WTN / MI;  // MFMA blocks of the wavefront's sub-tile
@@ -614,25 +615,27 @@ __global__ __launch_bounds__(WM* WN * 64, MINB) void gemm_nt_dma_kernel(MatmulAr
   static_assert(WTM % 32 == 0 && WTN % (MI16 ? 16 : 32) == 0,
                 "whole MFMA blocks (with 16x16x32 the sub-tile may be an odd number of them wide)");
   // epilogue slots: half of the wavefronts in each of the first two stages of the larger operand
-  constexpr bool SLOTS_IN_B = BN > BM;
+  constexpr bool SLOTS_IN_B = BN > BM || NSTAGE == 4;
   // (per stage: half the wavefronts where they fit, else as many as fit, over three stages)
   constexpr int SLOT_STAGE = (SLOTS_IN_B ? BN : BM) * BK * 2;
   constexpr int SLOTS = (NW / 2) * SLOT <= SLOT_STAGE ? NW / 2 : SLOT_STAGE / SLOT;
-  static_assert(SLOTS >= 1 && (NW + SLOTS - 1) / SLOTS <= (NSTAGE == 3 || (NSTAGE == 7 && !SLOTS_IN_B) ? 3 : 2),
+  static_assert(SLOTS >= 1 && (NW + SLOTS - 1) / SLOTS <= (NSTAGE == 3 || NSTAGE == 4 || NSTAGE == 5 || (NSTAGE == 7 && !SLOTS_IN_B) ? 3 : 2),
                 "epilogue slots must fit in the stage buffers");
-  static_assert(NSTAGE == 2 || NSTAGE == 3 || NSTAGE == 6 || NSTAGE == 7,
-                "2 or 3 LDS stages, or 6: two stages of the left and four of the right operand");
-  static_assert(NSTAGE < 6 || (!NN && NW % 2 == 0), "role split: NT products");
+  static_assert(NSTAGE >= 2 && NSTAGE <= 7, "2 or 3 LDS stages of both operands, or one of the role splits");
+  static_assert(!ROLES || (!NN && NW % 2 == 0), "role split: NT products");
   static_assert(!NN || BN == 128, "the N-contiguous right operand is staged as [64][128] tiles");
   // Separate objects per stage: the compiler's alias analysis then knows that the asynchronous
   // LDS writes of one stage cannot touch the stage being read, and does not serialise them.
   __shared__ __attribute__((aligned(1024))) unsigned char sA0[BM * BK * 2];
   __shared__ __attribute__((aligned(1024))) unsigned char sA1[BM * BK * 2];
-  __shared__ __attribute__((aligned(1024))) unsigned char sA2[NSTAGE == 3 || NSTAGE == 7 ? BM * BK * 2 : 1024];
+  __shared__ __attribute__((aligned(1024))) unsigned char sA2[NSTAGE == 3 || NSTAGE == 5 || NSTAGE == 7 ? BM * BK * 2 : 1024];
+  __shared__ __attribute__((aligned(1024))) unsigned char sA3[NSTAGE == 5 ? BM * BK * 2 : 1024];
+  __shared__ __attribute__((aligned(1024))) unsigned char sA4[NSTAGE == 5 ? BM * BK * 2 : 1024];
   __shared__ __attribute__((aligned(1024))) unsigned char sB0[BN * BK * 2];
   __shared__ __attribute__((aligned(1024))) unsigned char sB1[BN * BK * 2];
   __shared__ __attribute__((aligned(1024))) unsigned char sB2[NSTAGE >= 3 ? BN * BK * 2 : 1024];
-  __shared__ __attribute__((aligned(1024))) unsigned char sB3[NSTAGE >= 6 ? BN * BK * 2 : 1024];
+  __shared__ __attribute__((aligned(1024))) unsigned char sB3[NSTAGE >= 5 ? BN * BK * 2 : 1024];
+  __shared__ __attribute__((aligned(1024))) unsigned char sB4[NSTAGE == 5 ? BN * BK * 2 : 1024];
 
   // Diagnostic build only (-DADR_PHASE_STAMPS, adrastea_amd.build.build_stamps_library, read by
   // bench.py --phase-stamps): every wavefront leaves the shader-clock and 100 MHz real-time
@@ -669,15 +672,28 @@ __global__ __launch_bounds__(WM* WN * 64, MINB) void gemm_nt_dma_kernel(MatmulAr
 
   // DMA instruction i of this wavefront fills LDS chunks [(i*NW + wave)*64, +64) of a stage,
   // lane l the l-th of them; the lane fetches whatever (row, k-chunk) the swizzle puts there.
-  // Rows beyond the matrix are clamped to the last row (their results are never stored).
-  const int dwave = NSTAGE >= 6 ? wave % NWD : wave;  // index among the wavefronts issuing an operand
-  const half_t* gA[IA];
-  const half_t* gB[IB];
+  // Rows beyond the matrix (their results are never stored) are clamped to the last row by the 256-row and
+  // 256-column tiles.  The smaller ones address their rows through buffer descriptors, a lane's byte offset and the place
+  // in K as the scalar offset: rows beyond the matrix lie past the descriptor's end and are no transfer, and no address
+  // is computed per slice (us, clamped -> this: K1024 N2048 m=512 on 64x64 7.2 -> 7.05, K4096 N2048 m=1024 on 128x64
+  // 29.5 -> 29.0, K1024 N4096 m=1400 on 192x128 14.2 -> 14.0; the large ones lost 1 % with it, 128x256 8 %).  Row pitches
+  // that 32 bits do not hold stay off those tiles: buffer_rows() below.
+  constexpr bool BUFFER = !NN && BM <= 192 && BN <= 192;  // (the host's side of it: buffer_rows())
+  const int dwave = ROLES ? wave % NWD : wave;  // index among the wavefronts issuing an operand
+  const half_t* gA[BUFFER ? 1 : IA];
+  const half_t* gB[BUFFER ? 1 : IB];
+  uint32_t oA[BUFFER ? IA : 1], oB[BUFFER ? IB : 1];
+  const uint32_t rows_a = min(BM, a.m - m0), rows_b = min(BN, a.n - n0);
+  auto rA = __builtin_amdgcn_make_buffer_rsrc((void*)(A + (int64_t)m0 * a.stride_ly), 0,
+                                              (int)(((rows_a - 1) * (uint32_t)a.stride_ly + (uint32_t)(a.k - kt_begin * BK)) * 2), 0x00020000);
+  auto rB = __builtin_amdgcn_make_buffer_rsrc((void*)(B + (int64_t)n0 * a.stride_rx), 0,
+                                              (int)(((rows_b - 1) * (uint32_t)a.stride_rx + (uint32_t)(a.k - kt_begin * BK)) * 2), 0x00020000);
 #pragma unroll
   for (int i = 0; i < IA; i++) {
     int row, kc;
     lds_chunk_inv<CPR>((i * NWD + dwave) * 64 + lane, row, kc);
-    gA[i] = A + (int64_t)min(m0 + row, a.m - 1) * a.stride_ly + kc * 8;
+    if constexpr (BUFFER) oA[i] = ((uint32_t)row * (uint32_t)a.stride_ly + kc * 8) * 2;
+    else gA[i] = A + (int64_t)min(m0 + row, a.m - 1) * a.stride_ly + kc * 8;
   }
 #pragma unroll
   for (int i = 0; i < IB; i++) {
@@ -691,7 +707,8 @@ __global__ __launch_bounds__(WM* WN * 64, MINB) void gemm_nt_dma_kernel(MatmulAr
     } else {
       int row, kc;
       lds_chunk_inv<CPR>((i * NWD + dwave) * 64 + lane, row, kc);
-      gB[i] = B + (int64_t)min(n0 + row, a.n - 1) * a.stride_rx + kc * 8;
+      if constexpr (BUFFER) oB[i] = ((uint32_t)row * (uint32_t)a.stride_rx + kc * 8) * 2;
+      else gB[i] = B + (int64_t)min(n0 + row, a.n - 1) * a.stride_rx + kc * 8;
     }
   }
   const int64_t b_slice = NN ? (int64_t)BK * a.stride_ry : BK;  // elements per K slice
@@ -700,14 +717,22 @@ __global__ __launch_bounds__(WM* WN * 64, MINB) void gemm_nt_dma_kernel(MatmulAr
   auto dmaA = [&](int ks, unsigned char* dA) {
 #pragma unroll
     for (int i = 0; i < IA; i++)
-      __builtin_amdgcn_global_load_lds(ADR_GLB_PTR(gA[i] + ks * BK),
-                                       ADR_LDS_PTR(dA + (i * NWD + dwave) * 1024), 16, 0, 0);
+      if constexpr (BUFFER)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, ADR_LDS_PTR(dA + (i * NWD + dwave) * 1024), 16, (int)oA[i],
+                                                 ks * (BK * 2), 0, 0);
+      else
+        __builtin_amdgcn_global_load_lds(ADR_GLB_PTR(gA[i] + ks * BK),
+                                         ADR_LDS_PTR(dA + (i * NWD + dwave) * 1024), 16, 0, 0);
   };
   auto dmaB = [&](int ks, unsigned char* dB) {
 #pragma unroll
     for (int i = 0; i < IB; i++)
-      __builtin_amdgcn_global_load_lds(ADR_GLB_PTR(gB[i] + ks * b_slice),
-                                       ADR_LDS_PTR(dB + (i * NWD + dwave) * 1024), 16, 0, 0);
+      if constexpr (BUFFER)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rB, ADR_LDS_PTR(dB + (i * NWD + dwave) * 1024), 16, (int)oB[i],
+                                                 ks * (BK * 2), 0, 0);
+      else
+        __builtin_amdgcn_global_load_lds(ADR_GLB_PTR(gB[i] + ks * b_slice),
+                                         ADR_LDS_PTR(dB + (i * NWD + dwave) * 1024), 16, 0, 0);
   };
   auto dma = [&](unsigned char* dA, unsigned char* dB) {
     const int ks = min(kload, KT - 1);
@@ -841,8 +866,9 @@ __global__ __launch_bounds__(WM* WN * 64, MINB) void gemm_nt_dma_kernel(MatmulAr
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  if constexpr (NSTAGE >= 6) {
-    // Two (NSTAGE 6) or three (NSTAGE 7) stages of the left and four of the right operand, and two roles.  A wavefront's
+  if constexpr (ROLES) {
+    // Two (NSTAGE 6) or three (NSTAGE 7) stages of the left and four of the right operand -- or two and three,
+    // where the tile leaves no more room (NSTAGE 4), or five of each (NSTAGE 5) -- and two roles.  A wavefront's
     // transfers complete in the order it issued them, so a wavefront that issues both operands
     // cannot leave a right-operand slice in flight across the wait for the next left-operand
     // slice.  Here wavefronts 0 .. NW/2-1 issue every transfer of the left operand (slice kt+1 at
@@ -850,9 +876,10 @@ __global__ __launch_bounds__(WM* WN * 64, MINB) void gemm_nt_dma_kernel(MatmulAr
     // (slice kt+3 at the head of slice kt; at its end slices kt+2 and kt+3 may still be in
     // flight): weights that no cache holds get three slices to arrive.  Each role has its own
     // instruction stream; both pass the same barriers.
-    constexpr int SA = NSTAGE == 6 ? 2 : 3, SB = 4, P = NSTAGE == 6 ? 4 : 12;  // P: the stages' common period
-    auto stA = [&](int i) -> unsigned char* { return i == 0 ? sA0 : i == 1 ? sA1 : sA2; };
-    auto stB = [&](int i) -> unsigned char* { return i == 0 ? sB0 : i == 1 ? sB1 : i == 2 ? sB2 : sB3; };
+    constexpr int SA = NSTAGE == 4 || NSTAGE == 6 ? 2 : NSTAGE == 5 ? 5 : 3, SB = NSTAGE == 4 ? 3 : NSTAGE == 5 ? 5 : 4;
+    constexpr int P = NSTAGE == 4 ? 6 : NSTAGE == 5 ? 5 : NSTAGE == 6 ? 4 : 12;  // the stages' common period
+    auto stA = [&](int i) -> unsigned char* { return i == 0 ? sA0 : i == 1 ? sA1 : i == 2 ? sA2 : i == 3 ? sA3 : sA4; };
+    auto stB = [&](int i) -> unsigned char* { return i == 0 ? sB0 : i == 1 ? sB1 : i == 2 ? sB2 : i == 3 ? sB3 : sB4; };
     auto run = [&](auto role_tag) {
       constexpr bool LEFT = decltype(role_tag)::value;
       // (measured on the qkv product, same box, us with the weights rewritten by other launches in
@@ -2376,6 +2403,7 @@ enum GemmChoice {
   SHORTK_64, SHORTK_128,
   U8_256x192, U8_256x128, U8_128x128, U8_128x64, U8_64x64, U8_128x64_G2, U8_64x64_G4,
   DMA_256x192, DMA_256x160, DMA_256x128, DMA_128x256, DMA_128x192, DMA_128x128, DMA_128x64, DMA_64x64, DMA_64x64_K128, DMA_128x64_K128,
+  DMA_256x224, DMA_192x192, DMA_192x128, DMA_128x96, DMA_96x96,
   DMA_NN_256x128, DMA_NN_128x128, NN_ANYROW_128x128, NN_ANYROW_128x64,
   NN_ANYROW_64x64_G4, NN_ANYROW_32x64_G4,
   STAGE_256x128, STAGE_128x128, STAGE_64x64,
@@ -2415,11 +2443,40 @@ GemmChoice pick(const MatmulArgs& a, const Candidate* c, int n, double* cost_out
 // (the two large tiles run on 16x16x32 MFMAs: 9-16 % faster than on 32x32x16 on data that is not
 // constant -- qkv 170 -> 156 us, o 68 -> 58, down 162 -> 144 -- while the smaller tiles, which are
 // not bound by the power limit, gain nothing from it and stay on 32x32x16)
+// The last five fill rounds that the others leave partly empty: 128 x 96 and 96 x 96 where 128 x 128 would occupy
+// a half to three quarters of the compute units, 192 x 128, 192 x 192 and 256 x 224 where the next smaller tile needs
+// a second round.  us, weights from HBM, without / with them: K4096 N1024 m=2056 30.0 / 26.6, K4096 N4096 m=577 33.6 /
+// 30.3, 1028 47.1 / 41.2, K1280 N5120 m=836 21.9 / 19.3, K4096 N11008 m=1100 117 / 103, K5120 N13824 m=514 103 / 85, 1000
+// 152 / 126, 2048 263 / 248.  Their constants are fitted to one full round each, between those of the others.
 const Candidate DMA_TILES[] = {
     {DMA_256x192, 256, 192, 1, 1.24f}, {DMA_256x128, 256, 128, 1, 1.13f},
     {DMA_128x256, 128, 256, 1, 1.13f}, {DMA_128x192, 128, 192, 1, 0.85f}, {DMA_128x128, 128, 128, 2, 0.80f}, {DMA_128x64, 128, 64, 2, 0.60f},
-    {DMA_64x64, 64, 64, 4, 0.40f}, {DMA_256x160, 256, 160, 1, 1.19f}};
+    {DMA_64x64, 64, 64, 4, 0.40f}, {DMA_256x160, 256, 160, 1, 1.19f}, {DMA_256x224, 256, 224, 1, 1.20f},
+    {DMA_192x192, 192, 192, 1, 1.09f}, {DMA_192x128, 192, 128, 1, 0.99f}, {DMA_128x96, 128, 96, 1, 0.70f},
+    {DMA_96x96, 96, 96, 1, 0.58f}};
 constexpr int N_DMA_TILES = sizeof(DMA_TILES) / sizeof(DMA_TILES[0]);
+// Which of the last five a product is offered: none over batches (measured on weight matrices only); 192 x 128 above 384
+// rows, up to which 128 x 192 has no more tiles (it would be 4-6 % ahead at 330 and 384 rows against 12288 columns and 4 %
+// behind at 257); the two small ones, whose five stages are filled before the first slice, from 16 slices and for
+// more rows than one 64 x 64 tile has, and 128 x 96 where 128 x 128 occupies three quarters of the compute units only with
+// a longer K (192 tiles: K1024 N3072 m=900 11.4 -> 12.1 us, K4096 N12288 m=200 39.4 -> 37.1).
+GemmChoice pick_dma(const MatmulArgs& a, double* cost = nullptr) {
+  Candidate c[N_DMA_TILES];
+  int n = 0;
+  const int64_t tiles128 = (int64_t)((a.m + 127) / 128) * ((a.n + 127) / 128);
+  for (const Candidate& t : DMA_TILES) {
+    bool offered = true;
+    switch (t.id) {
+      case DMA_256x224: case DMA_192x192: offered = a.batches == 1; break;
+      case DMA_192x128: offered = a.batches == 1 && a.m > 384; break;
+      case DMA_128x96: offered = a.batches == 1 && a.m > 64 && (a.k >= 2048 || (a.k >= 1024 && 4 * tiles128 < 3 * num_cu())); break;
+      case DMA_96x96: offered = a.batches == 1 && a.m > 64 && a.k >= 1024; break;
+      default: break;
+    }
+    if (offered) c[n++] = t;
+  }
+  return pick(a, c, n, cost);
+}
 
 // The tiles of the u8-weight kernel.  One tile on every CU, weights from HBM, us at K 11008 / K 4096: 256x192 210 / 93
 // (176 and 232 tiles), 256x128 179 / 72, 128x128 114 / 47, 128x64 77 / 31 (two K groups; one: 87 / 35), 64x64
@@ -2442,6 +2499,12 @@ GemmChoice u8_k_groups(const MatmulArgs& a, GemmChoice c) {
   if (c == U8_128x64 && a.k % 128 == 0) return U8_128x64_G2;
   if (c == U8_64x64 && a.k % 256 == 0) return U8_64x64_G4;
   return c;
+}
+
+// Whether the rows of a tile lie within the 32 bits of gemm_nt_dma_kernel's descriptors (192 rows of 2^22 halves).
+bool buffer_rows(const MatmulArgs& a) {
+  constexpr int most = 1 << 22;
+  return a.stride_ly >= 0 && a.stride_ly < most && a.stride_rx >= 0 && a.stride_rx < most && a.k <= most;
 }
 
 // The MFMA family needs 16-byte aligned, K-contiguous rows on both operands.
@@ -2498,6 +2561,11 @@ GemmChoice choose(const MatmulArgs& a) {
   if (!a.rhs_q && (a.k == 64 || a.k == 128) && !(a.store == STORE_ACC_BETA && a.beta != 0.0f) &&
       a.m > 64 && (int64_t)((a.m + 127) / 128) * ((a.n + 127) / 128) * a.batches >= 2 * NUM_CU)
     return a.k == 64 ? SHORTK_64 : SHORTK_128;
+  if (plain && a.k % 64 == 0 && !buffer_rows(a)) {
+    static const Candidate wide[] = {{DMA_256x192, 256, 192, 1, 1.24f}, {DMA_256x128, 256, 128, 1, 1.13f},
+                                     {DMA_128x256, 128, 256, 1, 1.13f}};
+    return pick(a, wide, 3);
+  }
   if (plain && a.k % 64 == 0) {
     // Few K slices and too few tiles for the persistent kernel: a tile is dominated by its load
     // latency and its epilogue; two resident workgroups per CU overlap those phases
@@ -2509,7 +2577,7 @@ GemmChoice choose(const MatmulArgs& a) {
     // (tests and benchmarks can force a tile: adr_debug_knob)
     const int forced = knob(KNOB_GEMM_TILE);
     if (forced >= 1 && forced <= N_DMA_TILES) return DMA_TILES[forced - 1].id;
-    GemmChoice c = pick(a, DMA_TILES, N_DMA_TILES);
+    GemmChoice c = pick_dma(a);
     // Up to 64 rows against a matrix of a little more than one 64 x 64 tile per CU: the CUs that
     // hold two tiles finish as late as one 128 x 128 tile would, and that tile is 0-16 % ahead
     // (K6656 N17920 m=64: 72.8 -> 61.4 us, K3072 N24576: 37.9 -> 34.6, K8192 N22016: 86.2 -> 86.6);
@@ -2570,7 +2638,7 @@ SplitChoice choose_split_k64(const MatmulArgs& a, int64_t avail_bytes, GemmChoic
   const SplitChoice none = {GEMM_NONE, 1, 0, 0};
   const int NUM_CU = num_cu();
   double whole_cost;
-  pick(a, DMA_TILES, N_DMA_TILES, &whole_cost);
+  pick_dma(a, &whole_cost);
   whole_cost *= a.k;
   // With about one small tile per compute unit the time is set by the latency of the K slices,
   // not by the tile's arithmetic: 0.38 us per slice of 64 (measured: K4160 N4096 m=130 25.7 us).
@@ -2626,7 +2694,8 @@ SplitChoice search_split(const MatmulArgs& a, int64_t avail_bytes) {
   const GemmChoice whole = choose(a);
   const int NUM_CU = num_cu();
   if (a.k % 128 != 0)
-    return whole == DMA_128x128 || whole == DMA_128x64 || whole == DMA_64x64 || whole == DMA_256x128
+    return whole == DMA_128x128 || whole == DMA_128x64 || whole == DMA_64x64 || whole == DMA_256x128 ||
+                   whole == DMA_192x128 || whole == DMA_128x96 || whole == DMA_96x96
                ? choose_split_k64(a, avail_bytes, whole) : none;
   // us per slice of 64 with every compute unit busy and weights from HBM; the share of it that is left when
   // few tiles are in flight (`alone`); the rest goes with the tiles (three quarters on the large tiles)
@@ -2635,7 +2704,8 @@ SplitChoice search_split(const MatmulArgs& a, int64_t avail_bytes) {
   static const Whole wholes[] = {{DMA_64x64, 64, 64, 0.26, 0.55}, {DMA_64x64_K128, 64, 64, 0.26, 0.55},
                                  {DMA_128x64, 128, 64, 0.35, 0.40}, {DMA_128x64_K128, 128, 64, 0.35, 0.40},
                                  {DMA_128x128, 128, 128, 0.565, 0.23}, {DMA_128x192, 128, 192, 0.75, 0.23},
-                                 {DMA_256x128, 256, 128, 0.84, 0.23}};
+                                 {DMA_256x128, 256, 128, 0.84, 0.23}, {DMA_192x128, 192, 128, 0.70, 0.23},
+                                 {DMA_128x96, 128, 96, 0.49, 0.23}, {DMA_96x96, 96, 96, 0.52, 0.55}};
   auto tiles_of = [&](int bm, int bn) { return (int64_t)((a.m + bm - 1) / bm) * ((a.n + bn - 1) / bn) * a.batches; };
   const double weights_mb = 2e-6 * a.k * a.n * a.batches, slices = a.k / 64;
   double limit = 0;
@@ -2672,7 +2742,7 @@ SplitChoice search_split(const MatmulArgs& a, int64_t avail_bytes) {
 
 SplitChoice choose_split(const MatmulArgs& a, int64_t avail_bytes) {
   const SplitChoice none = {GEMM_NONE, 1, 0, 0};
-  if (avail_bytes <= 0 || a.rhs_q || a.load != ADR_LOAD_IDENTITY || a.k % 64 != 0 || a.k < 1024)
+  if (avail_bytes <= 0 || a.rhs_q || a.load != ADR_LOAD_IDENTITY || a.k % 64 != 0 || a.k < 1024 || !buffer_rows(a))
     return none;
   if (a.split == 0) return search_split(a, avail_bytes);
   const SplitChoice made = {(GemmChoice)(a.split >> 24), a.split & 0xff, (a.split >> 16 & 0xff) * 32, (a.split >> 8 & 0xff) * 32};
@@ -2710,6 +2780,11 @@ static bool choice_name(GemmChoice c, const char** name, bool u8 = false) {
     case DMA_64x64: *name = "gemm_nt_mfma_dma_64x64x64"; return true;
     case DMA_64x64_K128: *name = "gemm_nt_mfma_dma_64x64x128"; return true;
     case DMA_128x64_K128: *name = "gemm_nt_mfma_dma_128x64x128"; return true;
+    case DMA_256x224: *name = "gemm_nt_mfma_dma_256x224x64"; return true;
+    case DMA_192x192: *name = "gemm_nt_mfma_dma_192x192x64"; return true;
+    case DMA_192x128: *name = "gemm_nt_mfma_dma_192x128x64"; return true;
+    case DMA_128x96: *name = "gemm_nt_mfma_dma_128x96x64"; return true;
+    case DMA_96x96: *name = "gemm_nt_mfma_dma_96x96x64"; return true;
     case DMA_NN_256x128: *name = "gemm_nn_mfma_dma_256x128x64"; return true;
     case DMA_NN_128x128: *name = "gemm_nn_mfma_dma_128x128x64"; return true;
     case NN_ANYROW_128x128: *name = "gemm_nn_mfma_anyrow_128x128x64"; return true;
@@ -2749,6 +2824,14 @@ static hipError_t launch_choice(hipStream_t stream, const MatmulArgs& a, GemmCho
     case DMA_64x64: return launch_dma<64, 64, 2, 2, 3, 3>(stream, a);
     case DMA_64x64_K128: return launch_dma<64, 64, 2, 2, 3, 1, false, 128>(stream, a);
     case DMA_128x64_K128: return launch_dma<128, 64, 2, 2, 3, 1, false, 128>(stream, a);
+    // (256 x 224: two left and three right stages are what the LDS holds; 120 bytes a lane in scratch memory, none in
+    // the loop.  256 x 256 on the same stages spills 368 bytes and takes twice the time.  128 x 96 and 96 x 96: five
+    // stages of each operand, 2-4 % ahead of three and four where the inputs are cold)
+    case DMA_256x224: return launch_dma<256, 224, 4, 2, 4, 1, false, 64, true>(stream, a);
+    case DMA_192x192: return launch_dma<192, 192, 2, 4, 6, 1, false, 64, true>(stream, a);
+    case DMA_192x128: return launch_dma<192, 128, 2, 4, 7, 1, false, 64, true>(stream, a);
+    case DMA_128x96: return launch_dma<128, 96, 4, 2, 5, 1, false, 64, true>(stream, a);
+    case DMA_96x96: return launch_dma<96, 96, 3, 2, 5, 1, false, 64, true>(stream, a);
     case DMA_NN_256x128: return launch_dma<256, 128, 4, 2, 3, 1, true>(stream, a);
     case DMA_NN_128x128: return launch_dma<128, 128, 2, 2, 2, 2, true>(stream, a);
     case NN_ANYROW_128x128: return launch_nn_anyrow<128, 128, 4, 2, 1>(stream, a);
@@ -2781,15 +2864,15 @@ static bool split_m_tail(const MatmulArgs& a, MatmulArgs& head, MatmulArgs& tail
   const GemmChoice ca = choose(a), ch = choose(head), ct = choose(tail);
   auto dma_tile = [](GemmChoice c) {
     return c == DMA_256x192 || c == DMA_256x160 || c == DMA_256x128 || c == DMA_128x256 || c == DMA_128x192 || c == DMA_128x128 ||
-           c == DMA_128x64 || c == DMA_64x64;
+           c == DMA_128x64 || c == DMA_64x64 || (c >= DMA_256x224 && c <= DMA_96x96);
   };
   if (!dma_tile(ca) || !dma_tile(ch) || !dma_tile(ct)) return false;
   // pick()'s cost (tile area on the busiest CU over efficiency) times K is proportional to the
   // time of a launch; one more launch is priced at 3 us (2.9e6 of those units per us, measured)
   double whole, first, rest;
-  pick(a, DMA_TILES, N_DMA_TILES, &whole);
-  pick(head, DMA_TILES, N_DMA_TILES, &first);
-  pick(tail, DMA_TILES, N_DMA_TILES, &rest);
+  pick_dma(a, &whole);
+  pick_dma(head, &first);
+  pick_dma(tail, &rest);
   return (first + rest) * a.k + 8.7e6 < whole * a.k;
 }
 

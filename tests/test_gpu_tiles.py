@@ -1,0 +1,78 @@
+"""The tiles of the fp16 kernel that fill rounds the power-of-two tiles leave partly empty (256 x 224, 192 x 192,
+192 x 128, 128 x 96, 96 x 96), forced, at the edges of tiles, at every remainder of their stage periods and over batches
+with padded rows; and row pitches that their 32-bit row offsets do not hold.
+
+Inputs are multiples of 2^-6 up to 2^-4 in size: every product is a multiple of 2^-12 and every sum of up to 1088 of
+them below 2^2.1, exact in 32 bits in any order, so results are compared bit for bit."""
+import pytest
+import torch
+
+from adrastea_amd import _ffi
+
+pytestmark = pytest.mark.gpu
+
+TILES = {9: (256, 224), 10: (192, 192), 11: (192, 128), 12: (128, 96), 13: (96, 96)}
+
+
+def _draw(gen, shape):
+    return (torch.randint(-4, 5, shape, generator=gen, device="cuda").float() / 64).half()
+
+
+def _product(lib, B, M, K, N, ly, rx, oy, gen, tile):
+    lz, rz, oz = M * ly + 64, N * rx + 24, M * oy + 16
+    l, r = _draw(gen, (B * lz,)), _draw(gen, (B * rz,))
+    out = torch.full((B * oz,), 5.0, dtype=torch.float16, device="cuda")
+    want = out.clone()
+    for b in range(B):
+        x = torch.as_strided(l, (M, K), (ly, 1), b * lz).double()
+        w = torch.as_strided(r, (N, K), (rx, 1), b * rz).double()
+        torch.as_strided(want, (M, N), (oy, 1), b * oz).copy_((x @ w.t()).half())
+    try:
+        assert lib.adr_debug_knob(0, tile) == 0
+        assert lib.adr_matmul_f16(torch.cuda.current_stream().cuda_stream, out.data_ptr(), l.data_ptr(), r.data_ptr(),
+                                  B, M, K, N, 1, oy, oz, 1, ly, lz, rx, 1, rz, None, 0.0, 1.0, 0, 0, 0) == 0
+    finally:
+        lib.adr_debug_knob(0, 0)
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16)), (tile, B, M, K, N)
+
+
+@pytest.mark.parametrize("tile", TILES)
+def test_edges_of_tiles_and_every_remainder_of_the_stages(tile):
+    lib, gen = _ffi.lib(), torch.Generator(device="cuda").manual_seed(tile)
+    bm, bn = TILES[tile]
+    for slices in list(range(5, 18)):  # (fewer go to other kernels; periods of 4, 5, 6 and 12 slices)
+        _product(lib, 1, bm, 64 * slices, bn, 64 * slices, 64 * slices, bn, gen, tile)
+    for m in (1, 15, 17, bm - 1, bm + 1, 2 * bm + 31):
+        for n in (8, bn - 8, bn + 8, 2 * bn + 40, 3 * bn - 3):
+            _product(lib, 1, m, 384, n, 384, 384, n, gen, tile)
+    _product(lib, 2, bm + 37, 448, 2 * bn + 24, 456, 464, 2 * bn + 32, gen, tile)
+
+
+@pytest.mark.parametrize("M,K,N,tile", [(577, 4096, 4096, "128x96"), (1100, 4096, 4096, "192x128"),
+                                        (130, 4096, 12288, "96x96"), (514, 5120, 13824, "192x192"),
+                                        (1100, 4096, 11008, "256x224"), (2048, 4096, 12288, "256x192"),
+                                        (64, 4096, 17920, "128x128")])
+def test_the_choice_is_by_rounds(M, K, N, tile):
+    import ctypes as C
+    buf = C.create_string_buffer(96)
+    assert _ffi.lib().adr_matmul_f16_plan(buf, 96, 1, M, K, N, 1, N, 0, 1, K, 0, K, 1, 0, 0, 0, 0) == 0
+    assert buf.value.decode() == f"gemm_nt_mfma_dma_{tile}x64"
+
+
+@pytest.mark.parametrize("M,N", [(3, 200), (200, 5)])
+def test_row_pitches_beyond_32_bit_offsets(M, N):
+    """A pitch of 2^22 halves and more: 192 such rows are 2^31 bytes.  K 192 would go to the small tiles, 1088 to any."""
+    lib = _ffi.lib()
+    pitch = (1 << 22) + 8
+    for K in (192, 1088):
+        gen = torch.Generator(device="cuda").manual_seed(K)
+        rows = min(M, N)
+        big, small = _draw(gen, (rows * pitch,)), _draw(gen, (max(M, N), K))
+        wide = torch.as_strided(big, (rows, K), (pitch, 1))
+        out = torch.zeros(M, N, dtype=torch.float16, device="cuda")
+        l, r, ly, rx = (big, small, pitch, K) if M < N else (small, big, K, pitch)
+        assert lib.adr_matmul_f16(torch.cuda.current_stream().cuda_stream, out.data_ptr(), l.data_ptr(), r.data_ptr(),
+                                  1, M, K, N, 1, N, 0, 1, ly, 0, rx, 1, 0, None, 0.0, 1.0, 0, 0, 0) == 0
+        x, w = (wide, small) if M < N else (small, wide)
+        assert torch.equal(out, (x.double() @ w.double().t()).half())
