@@ -1563,9 +1563,13 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
 // leave (weights from HBM, us: K11008 N4096 m=160 55.0 -> 47.1, 384 81.5 -> 70.3, K13824 N5120 m=96 66.8 -> 57.7,
 // K4096 N12288 m=64 29.0 -> 27.1, 1536 179 -> 172); without the fence the left operand's moved back as well, and the
 // large tiles lost 10-15 %.
-template <int BM, int BN, int WM, int WN, bool MI16, int BK = 64, int G = 1>
-__global__ __launch_bounds__(WM* WN* G * 64, 1) void gemm_nt_u8_kernel(MatmulArgs a, TileMap map,
-                                                                      int block_shift) {
+// PAIRS: a lane's chunks are two by two neighbours in K, one request of 16 weights and one of the scale they share
+// (blocks of 16 weights and more), instead of a request of 8 and a scale for each chunk.  Half the weight requests of
+// the tiles with two chunks a lane, two thirds with three; weights from HBM, us: K4096 N4096 m=96 22.0 -> 21.2, 256 23.1 ->
+// 22.2, K11008 N4096 m=256 49.8 -> 47.7, 768 101.7 -> 98.6, K4096 N11008 m=64 26.1 -> 25.0, 2048 180.3 -> 178.6; the
+// LLaMA-7B layer of 2048 rows 820.7 -> 814.5.
+template <int BM, int BN, int WM, int WN, bool MI16, int BK, int G, bool PAIRS>
+__device__ __forceinline__ void gemm_nt_u8_body(const MatmulArgs& a, const TileMap& map, int block_shift) {
   constexpr int CPR = BK / 8, MI = MI16 ? 16 : 32, KG = 64 / MI, KK = CPR / KG;
   constexpr int NW = WM * WN, NT = NW * 64;  // wavefronts and lanes of one group
   constexpr int IA = BM * CPR / NT;   // DMA instructions per lane and slice
@@ -1575,6 +1579,8 @@ __global__ __launch_bounds__(WM* WN* G * 64, 1) void gemm_nt_u8_kernel(MatmulArg
   constexpr int FSTEP = MI * CPR * 16;         // bytes between the fragments of consecutive blocks
   constexpr int SLOT = 32 * (TN * 64 + 16);
   static_assert(BM * CPR % NT == 0 && BN * CPR % NT == 0, "slices must split evenly over lanes");
+  constexpr int NP = PAIRS ? LB / 2 : 0, NQ = LB - NP;  // pairs of chunks; requests of weights, and of scales, per slice
+  static_assert(NP * NT % (CPR / 2) == 0, "pairs fill whole rows");
   // epilogue slots lie in the stages of the operand with the larger ones, per stage half the
   // wavefronts where they fit (the 256-row tiles), else as many as fit
   constexpr bool SLOTS_IN_B = BN > BM;
@@ -1620,18 +1626,19 @@ __global__ __launch_bounds__(WM* WN* G * 64, 1) void gemm_nt_u8_kernel(MatmulArg
     lds_chunk_inv<CPR>((i * NW + wave) * 64 + lane, row, kc);
     gA[i] = (min((uint32_t)row, rows_a - 1) * (uint32_t)a.k + kc * 8) * 2;
   }
-  // weight chunk c = tid + i*NT -> (row, 8-weight group kc); rows beyond N are clamped
-  uint32_t gQ[LB], gS[LB];
+  // weight chunk c = tid + i*NT -> (row, 8-weight group kc), or the pairs of chunks first; rows beyond N are clamped
+  uint32_t gQ[NQ], gS[NQ];
   int offB[LB];
 #pragma unroll
-  for (int i = 0; i < LB; i++) {
-    const int c = tid + i * NT, row = c / CPR, kc = c % CPR;
+  for (int i = 0; i < NQ; i++) {
+    const int c = i < NP ? (tid + i * NT) * 2 : tid + (i + NP) * NT, row = c / CPR, kc = c % CPR;
     const uint32_t brow = min((uint32_t)row, rows_b - 1);
     gQ[i] = brow * (uint32_t)a.k + kc * 8;
     // block of weight k0 + 8*kc: k0 is a multiple of BK and 8*kc < BK, so the two parts of the
     // index add up exactly for any power-of-two block size
     gS[i] = (brow * (uint32_t)(a.k >> block_shift) + ((kc * 8) >> block_shift)) * 2;
-    offB[i] = lds_chunk_off<CPR>(row, kc);
+    offB[i < NP ? 2 * i : i + NP] = lds_chunk_off<CPR>(row, kc);
+    if (i < NP) offB[2 * i + 1] = lds_chunk_off<CPR>(row, kc + 1);
   }
   const int KT = a.k / (BK * G);
   int kloadA = 0, kloadQ = 0;
@@ -1646,18 +1653,25 @@ __global__ __launch_bounds__(WM* WN* G * 64, 1) void gemm_nt_u8_kernel(MatmulArg
   // of slice kt-1 (everything but that slice's own requests) already covers them and nothing in slice kt waits
   // for a load issued a moment ago
   u32x2_t rq[3][LB];
-  half_t rs[3][LB];
+  half_t rs[3][NQ];
   auto fetchQ = [&](int set) {
     const int k0 = (min(kloadQ, KT - 1) * G + grp) * BK;
     kloadQ++;
 #pragma unroll
-    for (int i = 0; i < LB; i++) {
-      rq[set][i] = __builtin_amdgcn_raw_buffer_load_b64(rQ, (int)gQ[i], k0, 0);
+    for (int i = 0; i < NQ; i++) {
+      if (i < NP) {
+        const u32x4_t q = __builtin_amdgcn_raw_buffer_load_b128(rQ, (int)gQ[i], k0, 0);
+        rq[set][2 * i] = u32x2_t{q[0], q[1]};
+        rq[set][2 * i + 1] = u32x2_t{q[2], q[3]};
+      } else {
+        rq[set][i + NP] = __builtin_amdgcn_raw_buffer_load_b64(rQ, (int)gQ[i], k0, 0);
+      }
       rs[set][i] = __builtin_bit_cast(half_t, __builtin_amdgcn_raw_buffer_load_b16(rS, (int)gS[i], (k0 >> block_shift) * 2, 0));
     }
   };
   auto dequant_store1 = [&](int set, unsigned char* dB, int i) {
-    const half2_t s2 = {rs[set][i], rs[set][i]};
+    const half_t scale = rs[set][i < 2 * NP ? i / 2 : i - NP];
+    const half2_t s2 = {scale, scale};
     *(half8_t*)(dB + goB + offB[i]) = dequant8(rq[set][i][0], rq[set][i][1], s2);
   };
   auto dequant_store = [&](int set, unsigned char* dB) {
@@ -1746,7 +1760,7 @@ __global__ __launch_bounds__(WM* WN* G * 64, 1) void gemm_nt_u8_kernel(MatmulArg
     // measured to: K11008 N4096 m=2048 174.2 us with three stages, 173.7 with four, 175.7 with four of either; K4096
     // N4096 70.5, 71.8, 71.6; K4096 N11008 m=512 58.5, 60.5, 60.4; K5120 N5120 m=1280 76.6, 78.3, 79.5.)
     __builtin_amdgcn_sched_barrier(0x38F);
-    constexpr int n = 2 * LB + IA;
+    constexpr int n = 2 * NQ + IA;
     __builtin_amdgcn_s_waitcnt(0x0070 | (n & 0xF) | ((n >> 4) << 14));
     __builtin_amdgcn_s_barrier();
     load_frags(0, nA, nB, 0);
@@ -1817,6 +1831,17 @@ __global__ __launch_bounds__(WM* WN* G * 64, 1) void gemm_nt_u8_kernel(MatmulArg
   unsigned char* slot = (SLOTS_IN_B ? (wave < SLOTS ? sB0 : sB1)
                                     : (wave < SLOTS ? sA0 : wave < 2 * SLOTS ? sA1 : sA2)) + (wave % SLOTS) * SLOT;
   wave_epilogue<TM, 2 * TN>(a, out, acc, m0 + wm * WTM, n0 + wn * WTN, slot, (half_t)a.scale, lane);
+}
+
+// Blocks of 8 weights: every chunk has a scale of its own.
+template <int BM, int BN, int WM, int WN, bool MI16, int BK = 64, int G = 1>
+__global__ __launch_bounds__(WM* WN * G * 64, 1) void gemm_nt_u8_kernel(MatmulArgs a, TileMap map, int block_shift) {
+  gemm_nt_u8_body<BM, BN, WM, WN, MI16, BK, G, false>(a, map, block_shift);
+}
+// Blocks of 16 weights and more.
+template <int BM, int BN, int WM, int WN, bool MI16, int BK = 64, int G = 1>
+__global__ __launch_bounds__(WM* WN * G * 64, 1) void gemm_nt_u8_pairs_kernel(MatmulArgs a, TileMap map, int block_shift) {
+  gemm_nt_u8_body<BM, BN, WM, WN, MI16, BK, G, true>(a, map, block_shift);
 }
 
 // =============================================================================================
@@ -2348,8 +2373,12 @@ template <int BM, int BN, int WM, int WN, bool MI16, int BK = 64, int G = 1>
 hipError_t launch_u8(hipStream_t stream, const MatmulArgs& a) {
   TileMap map = make_map(a, BM, BN);
   if (map.total < 0 || a.k % (BK * G) != 0) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((gemm_nt_u8_kernel<BM, BN, WM, WN, MI16, BK, G>), dim3((unsigned)map.total),
-                     dim3(WM * WN * G * 64), 0, stream, a, map, __builtin_ctz(a.block_size));
+  const dim3 grid((unsigned)map.total), block(WM * WN * G * 64);
+  const int shift = __builtin_ctz(a.block_size);
+  if (shift >= 4)
+    hipLaunchKernelGGL((gemm_nt_u8_pairs_kernel<BM, BN, WM, WN, MI16, BK, G>), grid, block, 0, stream, a, map, shift);
+  else
+    hipLaunchKernelGGL((gemm_nt_u8_kernel<BM, BN, WM, WN, MI16, BK, G>), grid, block, 0, stream, a, map, shift);
   return hipGetLastError();
 }
 
