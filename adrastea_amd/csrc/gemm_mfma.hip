@@ -1574,10 +1574,10 @@ __device__ __forceinline__ void gemm_nt_u8_body(const MatmulArgs& a, const TileM
   constexpr int NW = WM * WN, NT = NW * 64;  // wavefronts and lanes of one group
   constexpr int IA = BM * CPR / NT;   // DMA instructions per lane and slice
   constexpr int LB = BN * CPR / NT;   // 8-weight chunks per lane and slice
-  constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
+  constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN2 = WTN / 16;
   constexpr int FM = WTM / MI, FN = WTN / MI;  // MFMA blocks of the wavefront's sub-tile
   constexpr int FSTEP = MI * CPR * 16;         // bytes between the fragments of consecutive blocks
-  constexpr int SLOT = 32 * (TN * 64 + 16);
+  constexpr int SLOT = 32 * (TN2 * 32 + 16);
   static_assert(BM * CPR % NT == 0 && BN * CPR % NT == 0, "slices must split evenly over lanes");
   constexpr int NP = PAIRS ? LB / 2 : 0, NQ = LB - NP;  // pairs of chunks; requests of weights, and of scales, per slice
   static_assert(NP * NT % (CPR / 2) == 0, "pairs fill whole rows");
@@ -1830,10 +1830,10 @@ __device__ __forceinline__ void gemm_nt_u8_body(const MatmulArgs& a, const TileM
   }
   unsigned char* slot = (SLOTS_IN_B ? (wave < SLOTS ? sB0 : sB1)
                                     : (wave < SLOTS ? sA0 : wave < 2 * SLOTS ? sA1 : sA2)) + (wave % SLOTS) * SLOT;
-  wave_epilogue<TM, 2 * TN>(a, out, acc, m0 + wm * WTM, n0 + wn * WTN, slot, (half_t)a.scale, lane);
+  wave_epilogue<TM, TN2>(a, out, acc, m0 + wm * WTM, n0 + wn * WTN, slot, (half_t)a.scale, lane);
 }
 
-// Blocks of 8 weights: every chunk has a scale of its own.
+// Blocks of 8 weights, where every chunk has a scale of its own (and see launch_u8).
 template <int BM, int BN, int WM, int WN, bool MI16, int BK = 64, int G = 1>
 __global__ __launch_bounds__(WM* WN * G * 64, 1) void gemm_nt_u8_kernel(MatmulArgs a, TileMap map, int block_shift) {
   gemm_nt_u8_body<BM, BN, WM, WN, MI16, BK, G, false>(a, map, block_shift);
@@ -2375,7 +2375,10 @@ hipError_t launch_u8(hipStream_t stream, const MatmulArgs& a) {
   if (map.total < 0 || a.k % (BK * G) != 0) return hipErrorInvalidConfiguration;
   const dim3 grid((unsigned)map.total), block(WM * WN * G * 64);
   const int shift = __builtin_ctz(a.block_size);
-  if (shift >= 4)
+  // (128 x 128 on more than three quarters of the compute units is 1-2 % faster with its chunks apart: K5120 N13824 m=192
+  // 53.7 / 54.9 us, K1280 N5120 m=700 16.6 / 17.0; on fewer 1-3 % slower: K11008 N4096 m=768 101.7 / 98.6)
+  const bool apart = BM == 128 && BN == 128 && 4 * (int64_t)map.total > 3 * device_info_for_plan().cus;
+  if (shift >= 4 && !apart)
     hipLaunchKernelGGL((gemm_nt_u8_pairs_kernel<BM, BN, WM, WN, MI16, BK, G>), grid, block, 0, stream, a, map, shift);
   else
     hipLaunchKernelGGL((gemm_nt_u8_kernel<BM, BN, WM, WN, MI16, BK, G>), grid, block, 0, stream, a, map, shift);
@@ -2430,7 +2433,7 @@ hipError_t launch_shortk(hipStream_t stream, const MatmulArgs& a) {
 enum GemmChoice {
   GEMM_NONE = 0,
   SHORTK_64, SHORTK_128,
-  U8_256x192, U8_256x128, U8_128x128, U8_128x64, U8_64x64, U8_128x64_G2, U8_64x64_G4,
+  U8_256x192, U8_256x128, U8_128x128, U8_128x64, U8_64x64, U8_128x64_G2, U8_64x64_G4, U8_192x192, U8_192x128, U8_96x96,
   DMA_256x192, DMA_256x160, DMA_256x128, DMA_128x256, DMA_128x192, DMA_128x128, DMA_128x64, DMA_64x64, DMA_64x64_K128, DMA_128x64_K128,
   DMA_256x224, DMA_192x192, DMA_192x128, DMA_128x96, DMA_96x96,
   DMA_NN_256x128, DMA_NN_128x128, NN_ANYROW_128x128, NN_ANYROW_128x64,
@@ -2515,8 +2518,17 @@ GemmChoice pick_dma(const MatmulArgs& a, double* cost = nullptr) {
 // forced tile or within 3 % of it.
 const Candidate U8_TILES[] = {{U8_256x192, 256, 192, 1, 1.10f}, {U8_256x128, 256, 128, 1, 1.05f},
                               {U8_128x128, 128, 128, 1, 0.72f}, {U8_128x64, 128, 64, 2, 0.52f},
-                              {U8_64x64, 64, 64, 4, 0.37f}};
-constexpr int N_U8_TILES = sizeof(U8_TILES) / sizeof(U8_TILES[0]);
+                              {U8_64x64, 64, 64, 4, 0.37f}, {U8_192x192, 192, 192, 1, 0.98f},
+                              {U8_192x128, 192, 128, 1, 0.88f}, {U8_96x96, 96, 96, 1, 0.54f}};
+constexpr int N_U8_TILES = sizeof(U8_TILES) / sizeof(U8_TILES[0]), N_U8_FIRST = 5;
+// The last three fill rounds that the others leave partly empty, us without / with them: K4096 N12288 m=192 42.6 / 37.4
+// (96 x 96), 320 60.3 / 51.8, K5120 N13824 m=384 77.2 / 68.1, K4096 N4096 m=1280 57.9 / 54.4 (192 x 128), K4096 N12288 m=1408
+// 166 / 152, K5120 N13824 m=1280 203 / 186 (192 x 192).  Over 19 row counts x the eight (K, N) of the LLaMA-7B and 13B
+// layers the choice is the fastest of the ungrouped tiles or within 5 % of it.  (96 x 96 is no alternative to a single row
+// of 64 x 64 tiles, which other rules weigh against passes.)
+GemmChoice pick_u8(const MatmulArgs& a, double* cost = nullptr) {
+  return pick(a, U8_TILES, a.m > 64 ? N_U8_TILES : N_U8_TILES - 1, cost);
+}
 
 // With at most one tile per CU the two small tiles split K over groups of wavefronts inside the
 // workgroup (more slices in flight per CU; with more tiles than CUs several workgroups per CU do
@@ -2637,13 +2649,14 @@ GemmChoice choose(const MatmulArgs& a) {
   }
   // (the u8 kernel addresses the rows of a tile in 32 bits: 256 rows of 2^22 halves are 2^31 bytes)
   if (a.rhs_q && a.k % 64 == 0 && a.k <= 1 << 22 && a.block_size >= 8 && (a.block_size & (a.block_size - 1)) == 0) {
-    // (tests and benchmarks can force a tile: adr_debug_knob; 1 + N_U8_TILES: 128 x 64 with two K
-    // groups, 2 + N_U8_TILES: 64 x 64 with four, 3 + N_U8_TILES: the staged kernels below)
+    // (tests and benchmarks can force a tile: adr_debug_knob; 1 ... 5 the first of U8_TILES, 6: 128 x 64 with two K
+    // groups, 7: 64 x 64 with four, 8: the staged kernels below, from 10 on the rest of U8_TILES)
     const int forced = knob(KNOB_U8_TILE);
-    if (forced >= 1 && forced <= N_U8_TILES) return U8_TILES[forced - 1].id;
-    if (forced == N_U8_TILES + 1) return a.k % 128 == 0 ? U8_128x64_G2 : U8_128x64;
-    if (forced == N_U8_TILES + 2) return a.k % 256 == 0 ? U8_64x64_G4 : U8_64x64;
-    if (forced != N_U8_TILES + 3) return u8_k_groups(a, pick(a, U8_TILES, N_U8_TILES));
+    if (forced >= 1 && forced <= N_U8_FIRST) return U8_TILES[forced - 1].id;
+    if (forced == 6) return a.k % 128 == 0 ? U8_128x64_G2 : U8_128x64;
+    if (forced == 7) return a.k % 256 == 0 ? U8_64x64_G4 : U8_64x64;
+    if (forced >= 10 && forced < 10 + N_U8_TILES - N_U8_FIRST) return U8_TILES[N_U8_FIRST + forced - 10].id;
+    if (forced != 8) return u8_k_groups(a, pick_u8(a));
   }
   static const Candidate stage[] = {{STAGE_256x128, 256, 128, 2, 1.00f},
                                     {STAGE_128x128, 128, 128, 2, 0.85f},
@@ -2797,6 +2810,9 @@ static bool choice_name(GemmChoice c, const char** name, bool u8 = false) {
     case U8_128x128: *name = "gemm_nt_u8_mfma_128x128x64"; return true;
     case U8_128x64: *name = "gemm_nt_u8_mfma_128x64x64"; return true;
     case U8_64x64: *name = "gemm_nt_u8_mfma_64x64x64"; return true;
+    case U8_192x192: *name = "gemm_nt_u8_mfma_192x192x64"; return true;
+    case U8_192x128: *name = "gemm_nt_u8_mfma_192x128x64"; return true;
+    case U8_96x96: *name = "gemm_nt_u8_mfma_96x96x64"; return true;
     case U8_128x64_G2: *name = "gemm_nt_u8_mfma_128x64x64_k2"; return true;
     case U8_64x64_G4: *name = "gemm_nt_u8_mfma_64x64x64_k4"; return true;
     case DMA_256x192: *name = "gemm_nt_mfma_dma_256x192x64"; return true;
@@ -2836,6 +2852,9 @@ static hipError_t launch_choice(hipStream_t stream, const MatmulArgs& a, GemmCho
     case U8_128x128: return launch_u8<128, 128, 4, 2, true>(stream, a);
     case U8_128x64: return launch_u8<128, 64, 2, 2, true>(stream, a);
     case U8_64x64: return launch_u8<64, 64, 2, 2, true>(stream, a);
+    case U8_192x192: return launch_u8<192, 192, 2, 4, true>(stream, a);
+    case U8_192x128: return launch_u8<192, 128, 2, 4, true>(stream, a);
+    case U8_96x96: return launch_u8<96, 96, 3, 2, true>(stream, a);
     case U8_128x64_G2: return launch_u8<128, 64, 2, 2, true, 64, 2>(stream, a);
     case U8_64x64_G4: return launch_u8<64, 64, 2, 2, true, 64, 4>(stream, a);
     case DMA_256x192: return launch_dma<256, 192, 4, 2, 6, 1, false, 64, true>(stream, a);
@@ -2999,7 +3018,7 @@ double gemm_u8_mfma_estimate_us(int m, int p, int n, int block_size) {
   const MatmulArgs a = u8_args(nullptr, nullptr, (const uint8_t*)16, nullptr, m, p, n, block_size, 0.0f);
   if (!(p % 64 == 0 && block_size >= 8 && (block_size & (block_size - 1)) == 0)) return -1.0;
   double cost;
-  const GemmChoice c = pick(a, U8_TILES, N_U8_TILES, &cost);
+  const GemmChoice c = pick_u8(a, &cost);
   int64_t tiles = 0;
   for (const Candidate& t : U8_TILES)
     if (t.id == c) tiles = (int64_t)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);

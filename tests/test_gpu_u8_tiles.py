@@ -9,7 +9,7 @@ from adrastea_amd import GpuKernels, _ffi
 
 pytestmark = pytest.mark.gpu
 
-FORCED = {1: (256, 192), 2: (256, 128), 3: (128, 128), 4: (128, 64)}   # 5: 64 x 64, what they are compared with
+FORCED = {1: (256, 192), 2: (256, 128), 3: (128, 128), 4: (128, 64), 10: (192, 192), 11: (192, 128), 12: (96, 96)}  # 5: 64 x 64, what they are compared with
 
 
 def _run(kern, tile, x, q, s, block):

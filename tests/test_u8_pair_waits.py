@@ -7,7 +7,7 @@ from test_u8_waits import device_code, slices  # noqa: F401 (a fixture)
 
 # (rows, columns, wavefronts along them, groups)
 TILES = [(256, 192, 4, 2, 1), (256, 128, 4, 2, 1), (128, 128, 4, 2, 1), (128, 64, 2, 2, 1), (64, 64, 2, 2, 1),
-         (128, 64, 2, 2, 2), (64, 64, 2, 2, 4)]
+         (128, 64, 2, 2, 2), (64, 64, 2, 2, 4), (192, 192, 2, 4, 1), (192, 128, 2, 4, 1), (96, 96, 3, 2, 1)]
 
 
 @pytest.mark.parametrize("tile", TILES, ids=lambda t: "%dx%d_%dx%d_k%d" % t)
