@@ -249,18 +249,33 @@ __device__ __forceinline__ half8_t load8_any(const half_t* p, uintptr_t last) {
   return __builtin_bit_cast(half8_t, align5(d, (uint32_t)((uintptr_t)p & 2)));
 }
 
+// CACHED: plain stores instead of streaming ones, so that the L2 puts the lines together that two chunks share.
+template <bool CACHED = false>
 __device__ __forceinline__ void store8_any(half_t* p, half8_t v) {
+  typedef uint16_t ADR_GLOBAL_AS* gptr16_t;
+  typedef uint32_t ADR_GLOBAL_AS* gptr32_t;
+  typedef ADR_GLOBAL_AS u32x2_dword_aligned_t* gptr64_t;
+  typedef ADR_GLOBAL_AS u32x4_dword_aligned_t* gptr128_t;
   const uintptr_t u = (uintptr_t)p;
   const u32x4_t r = __builtin_bit_cast(u32x4_t, v);
   if ((u & 2) == 0) {
-    __builtin_nontemporal_store(r, (ADR_GLOBAL_AS u32x4_dword_aligned_t*)u);
+    if constexpr (CACHED) *(gptr128_t)u = r;
+    else __builtin_nontemporal_store(r, (gptr128_t)u);
   } else {
-    typedef uint16_t ADR_GLOBAL_AS* gptr16_t;
-    __builtin_nontemporal_store((uint16_t)(r[0] & 0xffffu), (gptr16_t)u);
+    const uint16_t first = (uint16_t)(r[0] & 0xffffu), last = (uint16_t)(r[3] >> 16);
     const u32x2_t m01 = {__builtin_amdgcn_alignbyte(r[1], r[0], 2u), __builtin_amdgcn_alignbyte(r[2], r[1], 2u)};
-    __builtin_nontemporal_store(m01, (ADR_GLOBAL_AS u32x2_dword_aligned_t*)(u + 2));
-    __builtin_nontemporal_store(__builtin_amdgcn_alignbyte(r[3], r[2], 2u), (ADR_GLOBAL_AS uint32_t*)(u + 10));
-    __builtin_nontemporal_store((uint16_t)(r[3] >> 16), (gptr16_t)(u + 14));
+    const uint32_t m2 = __builtin_amdgcn_alignbyte(r[3], r[2], 2u);
+    if constexpr (CACHED) {
+      *(gptr16_t)u = first;
+      *(gptr64_t)(u + 2) = m01;
+      *(gptr32_t)(u + 10) = m2;
+      *(gptr16_t)(u + 14) = last;
+    } else {
+      __builtin_nontemporal_store(first, (gptr16_t)u);
+      __builtin_nontemporal_store(m01, (gptr64_t)(u + 2));
+      __builtin_nontemporal_store(m2, (gptr32_t)(u + 10));
+      __builtin_nontemporal_store(last, (gptr16_t)(u + 14));
+    }
   }
 }
 

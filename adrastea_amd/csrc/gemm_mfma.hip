@@ -1130,8 +1130,9 @@ __device__ __forceinline__ void wait_vmcnt_at_most() {
 }
 
 // CPR: 16-byte chunks per row: 8 (K = 64) or 16 (K = 128).  DIRECT: the writers store the -inf of hidden tiles by
-// themselves (launch_shortk; a template parameter because a flag that they look at takes 10 % of a small result's time)
-template <int CPR, bool DIRECT>
+// themselves; CACHED: their stores go through the L2 instead of being streamed (launch_shortk; template parameters because a
+// flag that the writers look at takes 2-10 % of a small result's time)
+template <int CPR, bool DIRECT, bool CACHED>
 __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(MatmulArgs a,
                                                                            ShortKMap map) {
   constexpr int BM = 128, BN = 128, NWL = SHORTK_LOADERS, NWW = SHORTK_WRITERS;
@@ -1334,8 +1335,12 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
         half_t* const p = out + (int64_t)y0 * a.stride_oy + x;
         if (inside && walign == 8) {
 #pragma unroll
-          for (int it = 0; it < WIT; it++)
-            __builtin_nontemporal_store(v[it] * mul, (half8_t*)(p + (int64_t)(it * 4) * a.stride_oy));
+          for (int it = 0; it < WIT; it++) {
+            const half8_t r = v[it] * mul;
+            half_t* const q = p + (int64_t)(it * 4) * a.stride_oy;
+            if constexpr (CACHED) *(half8_t*)q = r;
+            else __builtin_nontemporal_store(r, (half8_t*)q);
+          }
         } else {
           // a ragged tile (rows or chunks past the matrix are skipped, a chunk across its last
           // column goes element by element), or rows that are not 16-byte aligned (a row length
@@ -1347,8 +1352,9 @@ __global__ __launch_bounds__(SHORTK_THREADS, 1) void gemm_nt_shortk_kernel(Matmu
             const half8_t r = v[it] * mul;
             half_t* const q = p + (int64_t)(it * 4) * a.stride_oy;
             if (whole) {
-              if (walign == 8) __builtin_nontemporal_store(r, (half8_t*)q);
-              else store8_any(q, r);
+              if (walign != 8) store8_any<CACHED>(q, r);
+              else if constexpr (CACHED) *(half8_t*)q = r;
+              else __builtin_nontemporal_store(r, (half8_t*)q);
             } else if (part) {
 #pragma unroll
               for (int e = 0; e < 8; e++)
@@ -2422,11 +2428,25 @@ hipError_t launch_shortk(hipStream_t stream, const MatmulArgs& a) {
   // themselves and staging is as good or better (32 heads of 128, 400 26.3 / 28.5, 513 50.1 / 51.4, 900 71.2 / 72.5; 40 of
   // 128, 800 69.9 / 73.7; 16 of 64, 1250 74.0 / 76.9; 12 of 64, 1100 56.8 / 55.3), and so it is for whole lines (32 of 128,
   // 2048 245.5 / 243.1, alone 72 / 94; 1600 of 40 heads 217 / 223; 1024 69.1 / 71.2).
+  // For the same reason large results of such rows are not streamed: a line goes out once, with what the tiles on both
+  // of its sides hold.  us, QK^T / the three calls, streamed -> cached: 16-byte aligned rows, 32 heads of 128, 1992 keys
+  // 124 / 298 -> 121 / 263, 1000 31 / 76 -> 19 / 71, 16 of 64, 1000 under the mask 15.6 / 42.0 -> 11.2 / 38.3; rows at any
+  // even address, 32 of 128, 2047 219 / 409 -> 165 / 346, under the mask 204 / 377 -> 136 / 317, 1500 76 / 197 -> 80 / 183, 40 of
+  // 128, 1333 96 / 206 -> 93 / 194.  Small results are a little better off streamed: 32 of 128, 400 26.6 / 27.3, and rows at
+  // any address 700 58.9 / 59.9, 1100 132.5 / 134.1, 16 of 64, 1111 66.2 / 66.9; hence the two lines.
   const bool lines = ((uintptr_t)a.output | 2 * (uintptr_t)a.stride_oy | (a.batches > 1 ? 2 * (uintptr_t)a.stride_oz : 0)) % 128 == 0;
-  if (a.mask == ADR_MASK_CAUSAL && !lines && (int64_t)a.batches * a.m * a.n >= 32 << 20)
-    hipLaunchKernelGGL((gemm_nt_shortk_kernel<CPR, true>), dim3(grid), dim3(SHORTK_THREADS), 0, stream, a, map);
+  const bool rows16 = (((uintptr_t)a.output >> 1 | (uintptr_t)a.stride_oy | (uintptr_t)a.stride_oz) & 7) == 0;
+  const int64_t results = (int64_t)a.batches * a.m * a.n;
+  const bool cached = !lines && results >= (rows16 ? 12 << 20 : 42 << 20), direct = a.mask == ADR_MASK_CAUSAL && !lines && results >= 32 << 20;
+  const dim3 block(SHORTK_THREADS);
+  if (direct && cached)
+    hipLaunchKernelGGL((gemm_nt_shortk_kernel<CPR, true, true>), dim3(grid), block, 0, stream, a, map);
+  else if (direct)
+    hipLaunchKernelGGL((gemm_nt_shortk_kernel<CPR, true, false>), dim3(grid), block, 0, stream, a, map);
+  else if (cached)
+    hipLaunchKernelGGL((gemm_nt_shortk_kernel<CPR, false, true>), dim3(grid), block, 0, stream, a, map);
   else
-    hipLaunchKernelGGL((gemm_nt_shortk_kernel<CPR, false>), dim3(grid), dim3(SHORTK_THREADS), 0, stream, a, map);
+    hipLaunchKernelGGL((gemm_nt_shortk_kernel<CPR, false, false>), dim3(grid), block, 0, stream, a, map);
   return hipGetLastError();
 }
 
