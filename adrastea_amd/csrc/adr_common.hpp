@@ -243,6 +243,23 @@ __device__ __forceinline__ u32x4_t load5_finish(const half_t* p, uintptr_t last,
   return align5(e, (uint32_t)((uintptr_t)p & 2));
 }
 
+// The same for chunks at 4-byte aligned addresses: the four dwords of the chunk, no shift.
+__device__ __forceinline__ u32x4_t load4_issue(const half_t* p, uintptr_t last) {
+  const uintptr_t base = (uintptr_t)p, lim = last - 12;
+  return *(const ADR_GLOBAL_AS u32x4_dword_aligned_t*)(base < lim ? base : lim);
+}
+__device__ __forceinline__ u32x4_t load4_finish(const half_t* p, uintptr_t last, u32x4_t q) {
+  const uintptr_t base = (uintptr_t)p, lim = last - 12;
+  if (__builtin_amdgcn_ballot_w64(base > lim) != 0) {
+    const uint32_t d0 = q[0], d1 = q[1], d2 = q[2], d3 = q[3];
+    const uintptr_t back = base > lim ? (base - lim) >> 2 : 0;  // (as in load5_finish)
+    q[0] = back == 0 ? d0 : back == 1 ? d1 : back == 2 ? d2 : d3;
+    q[1] = back == 0 ? d1 : back == 1 ? d2 : d3;
+    q[2] = back == 0 ? d2 : d3;
+  }
+  return q;
+}
+
 __device__ __forceinline__ half8_t load8_any(const half_t* p, uintptr_t last) {
   uint32_t d[5];
   load5_any(p, last, d);
