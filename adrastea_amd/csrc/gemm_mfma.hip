@@ -2495,13 +2495,14 @@ GemmChoice pick(const MatmulArgs& a, const Candidate* c, int n, double* cost_out
   GemmChoice best = GEMM_NONE;
   double best_cost = 0;
   const int NUM_CU = num_cu();
+  const double once = 1.0 / ((double)a.m * a.n * a.batches);
   for (int i = 0; i < n; i++) {
     const int64_t tiles = (int64_t)((a.m + c[i].bm - 1) / c[i].bm) * ((a.n + c[i].bn - 1) / c[i].bn) *
                           a.batches;
-    const int64_t per_cu = (tiles + NUM_CU - 1) / NUM_CU;
+    const int64_t per_cu = tiles < 1 << 30 ? ((uint32_t)tiles + NUM_CU - 1) / (uint32_t)NUM_CU : (tiles + NUM_CU - 1) / NUM_CU;
     // (between tiles that need equally many rounds, the one that pads the product less is a few
     // percent faster: M320 N11008 on 128 x 256 41.3 us, on 256 x 128 45.3)
-    const double padded = (double)tiles * c[i].bm * c[i].bn / ((double)a.m * a.n * a.batches);
+    const double padded = (double)tiles * c[i].bm * c[i].bn * once;
     const double cost = (double)per_cu * c[i].bm * c[i].bn / c[i].eff * (1.0 + 0.02 * (padded - 1.0));
     if (best == GEMM_NONE || cost < best_cost) {
       best = c[i].id;
@@ -2533,16 +2534,20 @@ constexpr int N_DMA_TILES = sizeof(DMA_TILES) / sizeof(DMA_TILES[0]);
 // more rows than one 64 x 64 tile has, and 128 x 96 where 128 x 128 occupies three quarters of the compute units only with
 // a longer K (192 tiles: K1024 N3072 m=900 11.4 -> 12.1 us, K4096 N12288 m=200 39.4 -> 37.1).
 GemmChoice pick_dma(const MatmulArgs& a, double* cost = nullptr) {
+  if (a.batches > 1 || (a.m <= 384 && a.k < 1024)) {
+    constexpr int first = N_DMA_TILES - 5;
+    if (a.batches > 1) return pick(a, DMA_TILES, first, cost);
+    return pick(a, DMA_TILES, first + 2, cost);  // (256 x 224 and 192 x 192)
+  }
   Candidate c[N_DMA_TILES];
   int n = 0;
   const int64_t tiles128 = (int64_t)((a.m + 127) / 128) * ((a.n + 127) / 128);
   for (const Candidate& t : DMA_TILES) {
     bool offered = true;
     switch (t.id) {
-      case DMA_256x224: case DMA_192x192: offered = a.batches == 1; break;
-      case DMA_192x128: offered = a.batches == 1 && a.m > 384; break;
-      case DMA_128x96: offered = a.batches == 1 && a.m > 64 && (a.k >= 2048 || (a.k >= 1024 && 4 * tiles128 < 3 * num_cu())); break;
-      case DMA_96x96: offered = a.batches == 1 && a.m > 64 && a.k >= 1024; break;
+      case DMA_192x128: offered = a.m > 384; break;
+      case DMA_128x96: offered = a.m > 64 && (a.k >= 2048 || (a.k >= 1024 && 4 * tiles128 < 3 * num_cu())); break;
+      case DMA_96x96: offered = a.m > 64 && a.k >= 1024; break;
       default: break;
     }
     if (offered) c[n++] = t;
