@@ -9,20 +9,20 @@
 //
 //  gemm_nt_dma_kernel   K % 64 == 0, plain fp16 operands.  K slices of depth 64 go from global
 //                       memory straight into LDS (global_load_lds_dwordx4, no register round
-//                       trip) into statically separate LDS stages (three per operand, or two /
-//                       three of the left and four of the right operand with the transfers split
-//                       by wavefront role), so the loads of the next slices are in flight while
+//                       trip) into statically separate LDS stages (three per operand, or, with the
+//                       transfers split by wavefront role, two to five of each), so the loads of the next slices are in flight while
 //                       the current slice feeds the MFMAs; one barrier per slice.  MFMA
 //                       fragments are prefetched one k-step ahead and interleaved with the
 //                       MFMAs by scheduling-group barriers.
-//  gemm_nt_u8_kernel    the same with u8 weights dequantised on their way into LDS; its two small
-//                       tiles can split K over groups of wavefronts inside the workgroup.
+//  gemm_nt_u8_pairs_kernel, gemm_nt_u8_kernel  the same with u8 weights dequantised on their way into
+//                       LDS (blocks of 16 and more, blocks of 8); the two small tiles can split K over groups of wavefronts inside the workgroup.
 //  gemm_nt_shortk_kernel  K = 64 / 128 (the attention score product): persistent workgroups;
 //                       also with the Load Scale operator (both operands scaled in fp16 on the
 //                       way into the MFMAs) and for score rows that are not 16-byte aligned.
 //  gemm_nn_anyrow_kernel  row-major x row-major products (P.V) whose left rows start at any even
 //                       address and whose K is no multiple of 64 (sequence lengths like 77, 257,
-//                       1500): left operand through registers, shifted into place.
+//                       1500): left operand through registers, shifted into place where its rows
+//                       start 2 bytes off a dword.
 //  gemm_nt_stage_kernel any K % 8 == 0, and the variants that must touch the data on the way
 //                       in: u8 weights dequantised while staging (a K that is no multiple of 64,
 //                       block sizes that are no power of two), and the Load Scale operator on
@@ -2521,7 +2521,7 @@ GemmChoice pick(const MatmulArgs& a, const Candidate* c, int n, double* cost_out
 // a second round.  us, weights from HBM, without / with them: K4096 N1024 m=2056 30.0 / 26.6, K4096 N4096 m=577 33.6 /
 // 30.3, 1028 47.1 / 41.2, K1280 N5120 m=836 21.9 / 19.3, K4096 N11008 m=1100 117 / 103, K5120 N13824 m=514 103 / 85, 1000
 // 152 / 126, 2048 263 / 248.  Their constants are fitted to one full round each, between those of the others.
-const Candidate DMA_TILES[] = {
+constexpr Candidate DMA_TILES[] = {
     {DMA_256x192, 256, 192, 1, 1.24f}, {DMA_256x128, 256, 128, 1, 1.13f},
     {DMA_128x256, 128, 256, 1, 1.13f}, {DMA_128x192, 128, 192, 1, 0.85f}, {DMA_128x128, 128, 128, 2, 0.80f}, {DMA_128x64, 128, 64, 2, 0.60f},
     {DMA_64x64, 64, 64, 4, 0.40f}, {DMA_256x160, 256, 160, 1, 1.19f}, {DMA_256x224, 256, 224, 1, 1.20f},
@@ -2534,6 +2534,10 @@ constexpr int N_DMA_TILES = sizeof(DMA_TILES) / sizeof(DMA_TILES[0]);
 // more rows than one 64 x 64 tile has, and 128 x 96 where 128 x 128 occupies three quarters of the compute units only with
 // a longer K (192 tiles: K1024 N3072 m=900 11.4 -> 12.1 us, K4096 N12288 m=200 39.4 -> 37.1).
 GemmChoice pick_dma(const MatmulArgs& a, double* cost = nullptr) {
+  // (at most one 64 x 64 tile per compute unit: no larger tile is cheaper, whatever it pads less; host time of small calls)
+  constexpr int smallest = 6;
+  static_assert(DMA_TILES[smallest].id == DMA_64x64, "the 64 x 64 tile");
+  if ((int64_t)((a.m + 63) / 64) * ((a.n + 63) / 64) * a.batches <= num_cu()) return pick(a, DMA_TILES + smallest, 1, cost);
   if (a.batches > 1 || (a.m <= 384 && a.k < 1024)) {
     constexpr int first = N_DMA_TILES - 5;
     if (a.batches > 1) return pick(a, DMA_TILES, first, cost);
