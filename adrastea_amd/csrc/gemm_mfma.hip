@@ -2491,10 +2491,9 @@ struct Candidate {
 // Estimated cost: the tiles of the busiest CU times the work of one tile over the efficiency of
 // a CU running this tile shape.  (With few long tiles the transfer rate into one CU's LDS, not
 // the matrix pipe, bounds a tile: spreading the same work over all CUs with smaller tiles wins.)
-GemmChoice pick(const MatmulArgs& a, const Candidate* c, int n, double* cost_out = nullptr) {
+GemmChoice pick(const MatmulArgs& a, const Candidate* c, int n, double* cost_out = nullptr, int NUM_CU = num_cu()) {
   GemmChoice best = GEMM_NONE;
   double best_cost = 0;
-  const int NUM_CU = num_cu();
   const double once = 1.0 / ((double)a.m * a.n * a.batches);
   for (int i = 0; i < n; i++) {
     const int64_t tiles = (int64_t)((a.m + c[i].bm - 1) / c[i].bm) * ((a.n + c[i].bn - 1) / c[i].bn) *
@@ -2534,14 +2533,15 @@ constexpr int N_DMA_TILES = sizeof(DMA_TILES) / sizeof(DMA_TILES[0]);
 // more rows than one 64 x 64 tile has, and 128 x 96 where 128 x 128 occupies three quarters of the compute units only with
 // a longer K (192 tiles: K1024 N3072 m=900 11.4 -> 12.1 us, K4096 N12288 m=200 39.4 -> 37.1).
 GemmChoice pick_dma(const MatmulArgs& a, double* cost = nullptr) {
+  const int cus = num_cu();
   // (at most one 64 x 64 tile per compute unit: no larger tile is cheaper, whatever it pads less; host time of small calls)
   constexpr int smallest = 6;
   static_assert(DMA_TILES[smallest].id == DMA_64x64, "the 64 x 64 tile");
-  if ((int64_t)((a.m + 63) / 64) * ((a.n + 63) / 64) * a.batches <= num_cu()) return pick(a, DMA_TILES + smallest, 1, cost);
+  if ((int64_t)((a.m + 63) / 64) * ((a.n + 63) / 64) * a.batches <= cus) return pick(a, DMA_TILES + smallest, 1, cost, cus);
   if (a.batches > 1 || (a.m <= 384 && a.k < 1024)) {
     constexpr int first = N_DMA_TILES - 5;
-    if (a.batches > 1) return pick(a, DMA_TILES, first, cost);
-    return pick(a, DMA_TILES, first + 2, cost);  // (256 x 224 and 192 x 192)
+    if (a.batches > 1) return pick(a, DMA_TILES, first, cost, cus);
+    return pick(a, DMA_TILES, first + 2, cost, cus);  // (256 x 224 and 192 x 192)
   }
   Candidate c[N_DMA_TILES];
   int n = 0;
@@ -2550,13 +2550,13 @@ GemmChoice pick_dma(const MatmulArgs& a, double* cost = nullptr) {
     bool offered = true;
     switch (t.id) {
       case DMA_192x128: offered = a.m > 384; break;
-      case DMA_128x96: offered = a.m > 64 && (a.k >= 2048 || (a.k >= 1024 && 4 * tiles128 < 3 * num_cu())); break;
+      case DMA_128x96: offered = a.m > 64 && (a.k >= 2048 || (a.k >= 1024 && 4 * tiles128 < 3 * cus)); break;
       case DMA_96x96: offered = a.m > 64 && a.k >= 1024; break;
       default: break;
     }
     if (offered) c[n++] = t;
   }
-  return pick(a, c, n, cost);
+  return pick(a, c, n, cost, cus);
 }
 
 // The tiles of the u8-weight kernel.  One tile on every CU, weights from HBM, us at K 11008 / K 4096: 256x192 210 / 93
