@@ -676,18 +676,20 @@ __global__ __launch_bounds__(WM* WN * 64, MINB) void gemm_nt_dma_kernel(MatmulAr
   // 256-column tiles.  The smaller ones address their rows through buffer descriptors, a lane's byte offset and the place
   // in K as the scalar offset: rows beyond the matrix lie past the descriptor's end and are no transfer, and no address
   // is computed per slice (us, clamped -> this: K1024 N2048 m=512 on 64x64 7.2 -> 7.05, K4096 N2048 m=1024 on 128x64
-  // 29.5 -> 29.0, K1024 N4096 m=1400 on 192x128 14.2 -> 14.0; the large ones lost 1 % with it, 128x256 8 %).  Row pitches
-  // that 32 bits do not hold stay off those tiles: buffer_rows() below.
-  constexpr bool BUFFER = !NN && BM <= 192 && BN <= 192;  // (the host's side of it: buffer_rows())
+  // 29.5 -> 29.0, K1024 N4096 m=1400 on 192x128 14.2 -> 14.0; the large ones lost 1 % with it, 128x256 8 %).  The offsets
+  // are unsigned: a view has fewer than 2^31 elements, so that the rows of every tile fit, whatever their pitch (the host's
+  // side of it: buffer_rows()).  Where the offset of a row beyond the matrix wraps, it lies inside the descriptor.
+  constexpr bool BUFFER = !NN && BM <= 192 && BN <= 192;
   const int dwave = ROLES ? wave % NWD : wave;  // index among the wavefronts issuing an operand
   const half_t* gA[BUFFER ? 1 : IA];
   const half_t* gB[BUFFER ? 1 : IB];
   uint32_t oA[BUFFER ? IA : 1], oB[BUFFER ? IB : 1];
   const uint32_t rows_a = min(BM, a.m - m0), rows_b = min(BN, a.n - n0);
+  const uint32_t depth = SPLIT ? (uint32_t)(kt_end - kt_begin) * BK : (uint32_t)a.k;  // elements of a row that are read
   auto rA = __builtin_amdgcn_make_buffer_rsrc((void*)(A + (int64_t)m0 * a.stride_ly), 0,
-                                              (int)(((rows_a - 1) * (uint32_t)a.stride_ly + (uint32_t)(a.k - kt_begin * BK)) * 2), 0x00020000);
+                                              (int)(((rows_a - 1) * (uint32_t)a.stride_ly + depth) * 2), 0x00020000);
   auto rB = __builtin_amdgcn_make_buffer_rsrc((void*)(B + (int64_t)n0 * a.stride_rx), 0,
-                                              (int)(((rows_b - 1) * (uint32_t)a.stride_rx + (uint32_t)(a.k - kt_begin * BK)) * 2), 0x00020000);
+                                              (int)(((rows_b - 1) * (uint32_t)a.stride_rx + depth) * 2), 0x00020000);
 #pragma unroll
   for (int i = 0; i < IA; i++) {
     int row, kc;
@@ -719,7 +721,7 @@ __global__ __launch_bounds__(WM* WN * 64, MINB) void gemm_nt_dma_kernel(MatmulAr
     for (int i = 0; i < IA; i++)
       if constexpr (BUFFER)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, ADR_LDS_PTR(dA + (i * NWD + dwave) * 1024), 16, (int)oA[i],
-                                                 ks * (BK * 2), 0, 0);
+                                                 (int)((uint32_t)ks * (BK * 2)), 0, 0);
       else
         __builtin_amdgcn_global_load_lds(ADR_GLB_PTR(gA[i] + ks * BK),
                                          ADR_LDS_PTR(dA + (i * NWD + dwave) * 1024), 16, 0, 0);
@@ -729,7 +731,7 @@ __global__ __launch_bounds__(WM* WN * 64, MINB) void gemm_nt_dma_kernel(MatmulAr
     for (int i = 0; i < IB; i++)
       if constexpr (BUFFER)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rB, ADR_LDS_PTR(dB + (i * NWD + dwave) * 1024), 16, (int)oB[i],
-                                                 ks * (BK * 2), 0, 0);
+                                                 (int)((uint32_t)ks * (BK * 2)), 0, 0);
       else
         __builtin_amdgcn_global_load_lds(ADR_GLB_PTR(gB[i] + ks * b_slice),
                                          ADR_LDS_PTR(dB + (i * NWD + dwave) * 1024), 16, 0, 0);
@@ -2591,10 +2593,14 @@ GemmChoice u8_k_groups(const MatmulArgs& a, GemmChoice c) {
   return c;
 }
 
-// Whether the rows of a tile lie within the 32 bits of gemm_nt_dma_kernel's descriptors (192 rows of 2^22 halves).
-bool buffer_rows(const MatmulArgs& a) {
-  constexpr int most = 1 << 22;
-  return a.stride_ly >= 0 && a.stride_ly < most && a.stride_rx >= 0 && a.stride_rx < most && a.k <= most;
+// Whether the rows of a tile, or of the pieces of a split one, lie within the 32 bits of gemm_nt_dma_kernel's descriptors.
+// Every entry point refuses views whose farthest element lies at or beyond 2^31: the only ones that do not fit are rows that
+// go backwards and an unsplit tile that ends on exactly the 2^31st element (4 GiB in at most 192 rows).
+bool buffer_rows(const MatmulArgs& a, bool split) {
+  auto fit = [&](int rows, int64_t pitch) {
+    return pitch >= 0 && (split || (std::min(rows, 192) - 1) * pitch + a.k < (int64_t)1 << 31);
+  };
+  return fit(a.m, a.stride_ly) && fit(a.n, a.stride_rx);
 }
 
 // The MFMA family needs 16-byte aligned, K-contiguous rows on both operands.
@@ -2651,7 +2657,8 @@ GemmChoice choose(const MatmulArgs& a) {
   if (!a.rhs_q && (a.k == 64 || a.k == 128) && !(a.store == STORE_ACC_BETA && a.beta != 0.0f) &&
       a.m > 64 && (int64_t)((a.m + 127) / 128) * ((a.n + 127) / 128) * a.batches >= 2 * NUM_CU)
     return a.k == 64 ? SHORTK_64 : SHORTK_128;
-  if (plain && a.k % 64 == 0 && !buffer_rows(a)) {
+  if (plain && a.k % 64 == 0 && !buffer_rows(a, false)) {
+    if (buffer_rows(a, true)) return DMA_256x128;  // (which a split is compared with)
     static const Candidate wide[] = {{DMA_256x192, 256, 192, 1, 1.24f}, {DMA_256x128, 256, 128, 1, 1.13f},
                                      {DMA_128x256, 128, 256, 1, 1.13f}};
     return pick(a, wide, 3);
@@ -2833,7 +2840,7 @@ SplitChoice search_split(const MatmulArgs& a, int64_t avail_bytes) {
 
 SplitChoice choose_split(const MatmulArgs& a, int64_t avail_bytes) {
   const SplitChoice none = {GEMM_NONE, 1, 0, 0};
-  if (avail_bytes <= 0 || a.rhs_q || a.load != ADR_LOAD_IDENTITY || a.k % 64 != 0 || a.k < 1024 || !buffer_rows(a))
+  if (avail_bytes <= 0 || a.rhs_q || a.load != ADR_LOAD_IDENTITY || a.k % 64 != 0 || a.k < 1024 || !buffer_rows(a, true))
     return none;
   if (a.split == 0) return search_split(a, avail_bytes);
   const SplitChoice made = {(GemmChoice)(a.split >> 24), a.split & 0xff, (a.split >> 16 & 0xff) * 32, (a.split >> 8 & 0xff) * 32};

@@ -62,7 +62,7 @@ def test_the_choice_is_by_rounds(M, K, N, tile):
 
 @pytest.mark.parametrize("M,N", [(3, 200), (200, 5)])
 def test_row_pitches_beyond_32_bit_offsets(M, N):
-    """A pitch of 2^22 halves and more: 192 such rows are 2^31 bytes.  K 192 would go to the small tiles, 1088 to any."""
+    """A pitch of 2^22 halves and more: 256 such rows are 2^31 bytes.  K 192 goes to the small tiles, 1088 to any."""
     lib = _ffi.lib()
     pitch = (1 << 22) + 8
     for K in (192, 1088):
@@ -76,3 +76,56 @@ def test_row_pitches_beyond_32_bit_offsets(M, N):
                                   1, M, K, N, 1, N, 0, 1, ly, 0, rx, 1, 0, None, 0.0, 1.0, 0, 0, 0) == 0
         x, w = (wide, small) if M < N else (small, wide)
         assert torch.equal(out, (x.double() @ w.double().t()).half())
+
+
+@pytest.mark.parametrize("side", ["left", "right"])
+@pytest.mark.parametrize("sign", [1, -1])
+def test_rows_gigabytes_apart(side, sign):
+    """Three rows a little under 2^30 halves apart: their byte offsets need all 32 bits.  On the 64 x 64 tile, on every
+    one of TILES, and with K split (K 8256; the view in the middle of its buffer, gigabytes from either end)."""
+    lib, R, O = _ffi.lib(), 3, 200
+    pitch, front = (1 << 30) - 16384, 1 << 30
+    big = torch.empty(front + 2 * pitch + 8256 + front, dtype=torch.float16, device="cuda")
+    first = front if sign > 0 else front + 2 * pitch  # of row 0
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    out = torch.empty(R * O, dtype=torch.float16, device="cuda")
+    for K, tiles in ((192, [0]), (1088, [0, *TILES]), (8256, [0])):
+        wide, small = _draw(gen, (R, K)), _draw(gen, (O, K))
+        if K > 1088:  # (so that sums of 8256 products stay exact)
+            wide[:, 1088:] = 0
+        for r in range(R):
+            big[first + r * sign * pitch:first + r * sign * pitch + K] = wide[r]
+        M, N = (R, O) if side == "left" else (O, R)
+        x, w = (wide, small) if side == "left" else (small, wide)
+        want = (x.double() @ w.double().t()).half()
+        at = big.data_ptr() + 2 * first
+        l, r, ly, rx = (at, small.data_ptr(), sign * pitch, K) if side == "left" else (small.data_ptr(), at, K, sign * pitch)
+        for tile in tiles:
+            out.fill_(5.0)
+            try:
+                assert lib.adr_debug_knob(0, tile) == 0
+                assert lib.adr_matmul_f16(torch.cuda.current_stream().cuda_stream, out.data_ptr(), l, r,
+                                          1, M, K, N, 1, N, 0, 1, ly, 0, rx, 1, 0, None, 0.0, 1.0, 0, 0, 0) == 0
+            finally:
+                lib.adr_debug_knob(0, 0)
+            assert torch.equal(out.view(M, N), want), (K, tile)
+
+
+@pytest.mark.parametrize("tile", [0, *TILES])
+def test_rows_that_overlap(tile):
+    """A pitch of 8 halves, the frames of a signal, and of none: the rows that a ragged tile is short of are not read."""
+    lib, gen = _ffi.lib(), torch.Generator(device="cuda").manual_seed(5)
+    for M, K, N, ly, rx in ((70, 1088, 200, 8, 1088), (200, 1088, 70, 1088, 8), (70, 448, 130, 0, 8), (70, 192, 200, 8, 192),
+                            (70, 8256, 200, 8, 8)):
+        l, r = _draw(gen, ((M - 1) * ly + K,)), _draw(gen, ((N - 1) * rx + K,))
+        if K > 1088:
+            l[600:-600] = 0  # (at most 1200 products that are not zero)
+        x, w = torch.as_strided(l, (M, K), (ly, 1)), torch.as_strided(r, (N, K), (rx, 1))
+        out = torch.full((M, N), 5.0, dtype=torch.float16, device="cuda")
+        try:
+            assert lib.adr_debug_knob(0, tile) == 0
+            assert lib.adr_matmul_f16(torch.cuda.current_stream().cuda_stream, out.data_ptr(), l.data_ptr(), r.data_ptr(),
+                                      1, M, K, N, 1, N, 0, 1, ly, 0, rx, 1, 0, None, 0.0, 1.0, 0, 0, 0) == 0
+        finally:
+            lib.adr_debug_knob(0, 0)
+        assert torch.equal(out, (x.double() @ w.double().t()).half()), (M, K, N, ly, rx)
