@@ -269,6 +269,8 @@ static bool skinny_ok(const MatmulArgs& a) {
   // against 32.8); from five rows on also ahead of the dot-product kernel (m=8, K4096 N12288:
   // 20.5 against 24.9)
   if (a.k % 128 != 0 || a.k < 1024 || (int64_t)a.n * a.k < (1 << 22)) return false;
+  // (unsigned 32-bit row offsets)
+  if (a.stride_ly < 0 || a.stride_rx < 0) return false;
   // four blocks of activation rows leave room for two groups of weight rows per workgroup; on a
   // wide matrix every workgroup then re-reads more activations than weights and the tiled
   // kernels are ahead (K4096 N12288 m=64: 38.8 against 29 us; N8192 and narrower: 38.7 against

@@ -129,3 +129,18 @@ def test_rows_that_overlap(tile):
         finally:
             lib.adr_debug_knob(0, 0)
         assert torch.equal(out, (x.double() @ w.double().t()).half()), (M, K, N, ly, rx)
+
+
+@pytest.mark.parametrize("M,K,N", [(3, 4096, 1100), (16, 4096, 1100), (64, 1024, 4096), (300, 1088, 700), (200, 8192, 520)])
+def test_rows_that_go_backwards(M, K, N):
+    """A negative pitch on either side, alone and on both: few rows, tiles, and sums that would be split."""
+    lib, gen = _ffi.lib(), torch.Generator(device="cuda").manual_seed(M)
+    x, w = _draw(gen, (M, K)), _draw(gen, (N, K))
+    x[:, 1088:] = 0  # (so that longer sums stay exact)
+    for ly, rx in ((-K, K), (K, -K), (-K, -K)):
+        l, r = x.data_ptr() + (2 * (M - 1) * K if ly < 0 else 0), w.data_ptr() + (2 * (N - 1) * K if rx < 0 else 0)
+        out = torch.full((M, N), 5.0, dtype=torch.float16, device="cuda")
+        assert lib.adr_matmul_f16(torch.cuda.current_stream().cuda_stream, out.data_ptr(), l, r,
+                                  1, M, K, N, 1, N, 0, 1, ly, 0, rx, 1, 0, None, 0.0, 1.0, 0, 0, 0) == 0
+        want = ((x.flip(0) if ly < 0 else x).double() @ (w.flip(0) if rx < 0 else w).double().t()).half()
+        assert torch.equal(out, want), (ly, rx)

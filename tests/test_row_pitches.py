@@ -50,3 +50,13 @@ def test_rows_that_go_backwards_are_addressed_in_64_bits(K):
     for M, N, ly, rx in ((300, 700, -K, K), (300, 700, K, -K), (300, 700, -(1 << 22), -K)):
         assert _plan(M, K, N, ly, rx) in ("gemm_nt_mfma_dma_256x192x64", "gemm_nt_mfma_dma_256x128x64",
                                           "gemm_nt_mfma_dma_128x256x64")
+
+
+@pytest.mark.parametrize("M", [3, 16, 33, 64])
+def test_few_rows_that_go_backwards_stay_off_the_unsigned_offsets(M):
+    """The kernel for up to 64 rows adds a row's unsigned 32-bit offset to the operand's address: a negative pitch would read
+    4 GiB further on."""
+    K, N = 4096, 4096
+    assert _plan(M, K, N, K, K) == "skinny_f16_mfma16_regstream"
+    for ly, rx in ((-K, K), (K, -K)):
+        assert not _plan(M, K, N, ly, rx).startswith("skinny")
