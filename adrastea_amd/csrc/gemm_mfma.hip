@@ -2450,16 +2450,27 @@ hipError_t launch_shortk(hipStream_t stream, const MatmulArgs& a) {
   // themselves and staging is as good or better (32 heads of 128, 400 26.3 / 28.5, 513 50.1 / 51.4, 900 71.2 / 72.5; 40 of
   // 128, 800 69.9 / 73.7; 16 of 64, 1250 74.0 / 76.9; 12 of 64, 1100 56.8 / 55.3), and so it is for whole lines (32 of 128,
   // 2048 245.5 / 243.1, alone 72 / 94; 1600 of 40 heads 217 / 223; 1024 69.1 / 71.2).
-  // For the same reason large results of such rows are not streamed: a line goes out once, with what the tiles on both
-  // of its sides hold.  us, QK^T / the three calls, streamed -> cached: 16-byte aligned rows, 32 heads of 128, 1992 keys
-  // 124 / 298 -> 121 / 263, 1000 31 / 76 -> 19 / 71, 16 of 64, 1000 under the mask 15.6 / 42.0 -> 11.2 / 38.3; rows at any
-  // even address, 32 of 128, 2047 219 / 409 -> 165 / 346, under the mask 204 / 377 -> 136 / 317, 1500 76 / 197 -> 80 / 183, 40 of
-  // 128, 1333 96 / 206 -> 93 / 194.  Small results are a little better off streamed: 32 of 128, 400 26.6 / 27.3, and rows at
-  // any address 700 58.9 / 59.9, 1100 132.5 / 134.1, 16 of 64, 1111 66.2 / 66.9; hence the two lines.
-  const bool lines = ((uintptr_t)a.output | 2 * (uintptr_t)a.stride_oy | (a.batches > 1 ? 2 * (uintptr_t)a.stride_oz : 0)) % 128 == 0;
-  const bool rows16 = (((uintptr_t)a.output >> 1 | (uintptr_t)a.stride_oy | (uintptr_t)a.stride_oz) & 7) == 0;
+  // For the same reason large results of such rows are not streamed: a line goes out once, with what the tiles on both of
+  // its sides hold, and is still cached when the next launch reads it.  How much that gains goes with `piece`, the power of two
+  // that every row's place is a multiple of.  us, streamed -> cached, QK^T over three buffers in turn / the three calls:
+  //   any even address  32 heads of 128, 2047 keys 213 / 410 -> 158 / 345, 1501 87 / 208 -> 81 / 194; 40 of 128, 1590 129 / 302 ->
+  //                     135 / 273; masked 2047 204 / 375 -> 135 / 318, 1333 x 40 77 / 191 -> 81 / 186
+  //   16 bytes          1992 125 / 289 -> 113 / 252, 1000 31 / 76 -> 19 / 68; 16 of 64, 1000 15.1 / 41.2 -> 11.3 / 37.4; masked 1800
+  //                     91 / 200 -> 79 / 188
+  //   32 bytes          1840 86 / 225 -> 93 / 209, 2000 106 / 269 -> 111 / 251; 40 of 128, 1200 49 / 142 -> 56 / 136; 20 of 64, 1200
+  //                     24 / 65 -> 19 / 61
+  // Half lines are streamed as well as whole ones (64 bytes: 1824 54 / 213 -> 83 / 203, 40 of 128, 1376 42 / 171 -> 67 / 168, 800
+  // 14.9 / 51.2 -> 17.2 / 51.9), and so are results below which QK^T loses what the calls gain, or more: masked ones with
+  // their hidden tiles written directly (32 bytes, 1328 39 / 127 -> 50 / 124, 1680 74 / 182 -> 75 / 179; 16 bytes, 1352 44 / 134 ->
+  // 51 / 129, 40 of 128, 1400 70 / 171 -> 69 / 166; any address, 1101 51 / 153 -> 58 / 150, 16 of 64, 2001 60 / 151 -> 56 / 140), and
+  // small ones (32 bytes, 720 15.6 / 47.6 -> 16.3 / 48.0, 848 19.8 / 56.2 -> 17.8 / 54.8; any address, 1100 132.5 -> 134.1).
+  const uint64_t places = (uintptr_t)a.output | 2 * (uint64_t)a.stride_oy | (a.batches > 1 ? 2 * (uint64_t)a.stride_oz : 0);
+  const uint64_t piece = places & (0 - places);
+  const bool lines = places % 128 == 0;
   const int64_t results = (int64_t)a.batches * a.m * a.n;
-  const bool cached = !lines && results >= (rows16 ? 12 << 20 : 42 << 20), direct = a.mask == ADR_MASK_CAUSAL && !lines && results >= 32 << 20;
+  const bool direct = a.mask == ADR_MASK_CAUSAL && !lines && results >= 32 << 20;
+  const int from = piece <= 8 ? (direct ? 56 : 42) : piece == 16 ? (direct ? 70 : 12) : (direct ? 84 : 18);  // Mi results
+  const bool cached = piece <= 32 && results >= (int64_t)from << 20;
   const dim3 block(SHORTK_THREADS);
   if (direct && cached)
     hipLaunchKernelGGL((gemm_nt_shortk_kernel<CPR, true, true>), dim3(grid), block, 0, stream, a, map);

@@ -1,6 +1,6 @@
 """Score products so large that their results go through the L2 instead of being streamed: rows that are no whole 128-byte
-lines, 16-byte aligned (from 12 * 2^20 results on) and at any even address (from 42 * 2^20 on), masked and not, by themselves
-and as views with a pitch.  Inputs are multiples of 2^-3 up to 1/2 in size: every sum of 128 products is a multiple of 2^-6
+lines, 16-byte aligned (from 12 * 2^20 results on), at any even address (from 42 * 2^20 on) and 32-byte aligned, masked and
+not, by themselves and as views with a pitch.  Inputs are multiples of 2^-3 up to 1/2 in size: every sum of 128 products is a multiple of 2^-6
 below 2^5, exact in 32 bits in any order, and so is its one rounding to fp16."""
 import pytest
 import torch
@@ -17,6 +17,12 @@ pytestmark = pytest.mark.gpu
     (8, 64, 2350, 2350, 2350, False),      # rows at every fourth, eighth, twelfth and sixteenth byte
     (8, 128, 2347, 2347, 2347, True),      # at any even address
     (8, 64, 2347, 2351, 2353, False),      # with a pitch: what lies between the rows stays
+    (15, 128, 2304, 2200, 2200, True),     # as the third, from 70 * 2^20 on, where masked results are not streamed either
+    (11, 128, 2347, 2347, 2347, True),     # as the fifth, from 56 * 2^20 on
+    (13, 64, 2400, 2352, 2352, False),     # 32-byte aligned rows: from 18 * 2^20 on
+    (16, 128, 2400, 2352, 2352, True),     # (masked: from 84 * 2^20 on)
+    (8, 128, 2400, 2336, 2336, True),      # rows of whole half lines: streamed
+    (9, 64, 2300, 2312, 2336, False),      # (with a pitch)
 ])
 def test_large_scores(heads, d, m, n, pitch, causal):
     gen = torch.Generator(device="cuda").manual_seed(heads * n + d)

@@ -128,3 +128,31 @@ def test_chosen_u8_tile_is_within_seven_percent_of_the_best_forced_one(case):
         if ratio <= 1.07:
             break
     assert ratio <= 1.07, (case, {("chosen" if t == 0 else U8_TILES[t - 1]): round(v * 1e3, 1) for t, v in best.items()})
+
+
+@pytest.mark.parametrize("heads,d,n,lines", [(40, 128, 1376, 1408), (32, 128, 1824, 1856), (16, 64, 1888, 1920)])
+def test_score_rows_of_half_lines_are_as_fast_as_rows_of_whole_lines(heads, d, n, lines):
+    """The score product by itself, over three buffers in turn: rows of whole 64-byte pieces take no longer for a result
+    than rows of whole 128-byte lines, both streamed (through the L2 the former took half as long again)."""
+    lib = _ffi.lib()
+
+    def ready(n):
+        gen = torch.Generator(device="cuda").manual_seed(n)
+        q, k = (torch.randn(n, heads * d, generator=gen, device="cuda").half() for _ in range(2))
+        outs = [torch.zeros(heads, n, n, dtype=torch.float16, device="cuda") for _ in range(3)]
+
+        def fn():
+            for out in outs:
+                rc = lib.adr_matmul_f16(torch.cuda.current_stream().cuda_stream, out.data_ptr(), q.data_ptr(), k.data_ptr(),
+                                        heads, n, d, n, 1, n, n * n, 1, heads * d, d, heads * d, 1, d, None, 0.0,
+                                        d ** -0.5, 4, 0, 0)
+                assert rc == 0
+        return fn
+    half, whole = ready(n), ready(lines)
+    ratio = None
+    for attempt in range(3):
+        times = [min(_time(fn, 40) for _ in range(3)) for fn in (half, whole)]
+        ratio = times[0] / times[1] * (lines / n) ** 2
+        if ratio <= 1.15:
+            break
+    assert ratio <= 1.15, (times, ratio)
