@@ -2795,6 +2795,11 @@ SplitChoice choose_split_k64(const MatmulArgs& a, int64_t avail_bytes, GemmChoic
 // us, before the second launch was spread over the chip and the large tiles could split -> now, weights from
 // HBM: K11008 N4096 m=128 37 -> 31, 256 45 -> 41, 512 67 -> 55, 640 101 -> 71, 768 101 -> 81, 1024 105 -> 89;
 // K13824 N5120 m=512 124 -> 77; K4096 N4096 m=96 18.7 -> 16.0; K5120 N1280 m=100 23.3 -> 11.5.
+// 192 x 128 and 256 x 128 in several rounds are priced from products of their own (priced like the other tiles, 192 x 128 was 14 %
+// too cheap on three quarters of the compute units and 256 x 128 13 % in two rounds; us, that choice / this, weights from
+// HBM: K28672 N8192 m=513 316 -> 278 (whole -> three pieces), 1024 434 -> 403 (two pieces -> whole), 641 331 -> 341; K14336 N4096
+// m=2048 212 -> 185; K11008 N4096 m=1200 124 -> 102, 1280 125 -> 118 (three pieces -> whole; with resident weights 121 -> 101).
+// 192 x 192 and 256 x 224 have no price: where they are chosen they are ahead of the pieces (K8192 N8192 m=1281 161 / 197).
 SplitChoice search_split(const MatmulArgs& a, int64_t avail_bytes) {
   const SplitChoice none = {GEMM_NONE, 1, 0, 0};
 #ifdef ADR_PHASE_STAMPS
@@ -2813,7 +2818,7 @@ SplitChoice search_split(const MatmulArgs& a, int64_t avail_bytes) {
   static const Whole wholes[] = {{DMA_64x64, 64, 64, 0.26, 0.55}, {DMA_64x64_K128, 64, 64, 0.26, 0.55},
                                  {DMA_128x64, 128, 64, 0.35, 0.40}, {DMA_128x64_K128, 128, 64, 0.35, 0.40},
                                  {DMA_128x128, 128, 128, 0.565, 0.23}, {DMA_128x192, 128, 192, 0.75, 0.23},
-                                 {DMA_256x128, 256, 128, 0.84, 0.23}, {DMA_192x128, 192, 128, 0.70, 0.23},
+                                 {DMA_256x128, 256, 128, 0.84, 0.23}, {DMA_192x128, 192, 128, 0.715, 0.50},
                                  {DMA_128x96, 128, 96, 0.49, 0.23}, {DMA_96x96, 96, 96, 0.52, 0.55}};
   auto tiles_of = [&](int bm, int bn) { return (int64_t)((a.m + bm - 1) / bm) * ((a.n + bn - 1) / bn) * a.batches; };
   const double weights_mb = 2e-6 * a.k * a.n * a.batches, slices = a.k / 64;
@@ -2826,10 +2831,10 @@ SplitChoice search_split(const MatmulArgs& a, int64_t avail_bytes) {
     }
   const double least = 6.7 + 0.067 * weights_mb;
   if (least >= limit) return none;  // (as for most products: no host time for the search)
-  struct Piece { GemmChoice id; int bm, bn; double us; };
-  static const Piece pieces[] = {{DMA_64x64_K128, 64, 64, 0.19}, {DMA_128x64_K128, 128, 64, 0.296},
-                                 {DMA_128x128, 128, 128, 0.439}, {DMA_128x256, 128, 256, 0.766},
-                                 {DMA_256x128, 256, 128, 0.659}};
+  struct Piece { GemmChoice id; int bm, bn; double us, us2; };  // us2: where the pieces need more than one round
+  static const Piece pieces[] = {{DMA_64x64_K128, 64, 64, 0.19, 0.19}, {DMA_128x64_K128, 128, 64, 0.296, 0.296},
+                                 {DMA_128x128, 128, 128, 0.439, 0.439}, {DMA_128x256, 128, 256, 0.766, 0.766},
+                                 {DMA_256x128, 256, 128, 0.659, 0.745}};
   SplitChoice best = none;
   for (const Piece& t : pieces) {
     const int64_t nt = tiles_of(t.bm, t.bn);
@@ -2839,7 +2844,7 @@ SplitChoice search_split(const MatmulArgs& a, int64_t avail_bytes) {
       const int64_t bytes = nt * sp * t.bm * t.bn * 4;
       if (bytes > avail_bytes) break;
       const int rounds = ((int)nt * sp + NUM_CU - 1) / NUM_CU;
-      const double us = least - 1.4 + rounds * (1.4 + (a.k / 64 + sp - 1) / sp * t.us) + 0.28e-6 * bytes;
+      const double us = least - 1.4 + rounds * (1.4 + (a.k / 64 + sp - 1) / sp * (rounds > 1 ? t.us2 : t.us)) + 0.28e-6 * bytes;
       if (us < limit) {
         limit = us;
         best = {t.id, sp, t.bm, t.bn};
