@@ -2659,7 +2659,7 @@ GemmChoice choose(const MatmulArgs& a) {
   if (a.k % 8 != 0 || a.k < 8) return GEMM_NONE;
   if ((a.stride_ly % 8) | (a.stride_rx % 8) | (a.stride_lz % 8) | (a.stride_rz % 8)) return GEMM_NONE;
   if (a.lhs && ((uintptr_t)a.lhs % 16 != 0 || (uintptr_t)a.rhs % 16 != 0 ||
-                (uintptr_t)a.rhs_q % 8 != 0)) return GEMM_NONE;
+                (uintptr_t)a.rhs_q % 16 != 0)) return GEMM_NONE;
   const bool plain = !a.rhs_q && a.load == ADR_LOAD_IDENTITY;
   // One or two K slices (the attention score product): the persistent kernel, which also scales
   // its operands on the way in where the caller asks for that (whisper.rs:424-430)
