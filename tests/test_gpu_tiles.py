@@ -49,6 +49,39 @@ def test_edges_of_tiles_and_every_remainder_of_the_stages(tile):
     _product(lib, 2, bm + 37, 448, 2 * bn + 24, 456, 464, 2 * bn + 32, gen, tile)
 
 
+@pytest.mark.parametrize("store", [0, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("tile", TILES)
+def test_every_store_with_and_without_the_mask(tile, store):
+    """The epilogues of the tiles' sub-tile widths against the step-for-step kernel, whose sums are the same bits: result
+    rows of 16-byte pieces, with a last column tile that ends inside the matrix, and rows at any even address.  The GELU
+    stores evaluate their function to 2e-6 of its value, here at most 4, and either side rounds once to fp16."""
+    lib, gen = _ffi.lib(), torch.Generator(device="cuda").manual_seed(100 * tile + store)
+    bm, bn = TILES[tile]
+    K, stream = 384, torch.cuda.current_stream().cuda_stream
+    for M, N, oy in ((2 * bm + 31, 2 * bn + 40, 2 * bn + 40), (bm + 17, 2 * bn, 2 * bn + 8), (bm + 33, bn + 13, bn + 13),
+                     (2 * bm, 2 * bn, 2 * bn + 5)):
+        l, r = _draw(gen, (M, K)), _draw(gen, (N, K))
+        bias, prev = (torch.randint(-8, 9, shape, generator=gen, device="cuda").div(4).half() for shape in ((N,), (M, oy)))
+        for mask in (0, 1):
+            got, want = prev.clone(), prev.clone()
+            for fn, out, knob in ((lib.adr_matmul_f16, got, tile), (lib.adr_matmul_f16_slow, want, 0)):
+                try:
+                    assert lib.adr_debug_knob(0, knob) == 0
+                    assert fn(stream, out.data_ptr(), l.data_ptr(), r.data_ptr(), 1, M, K, N, 1, oy, 0, 1, K, 0, K, 1, 0,
+                              bias.data_ptr(), 0.5, 0.25, store, 0, mask) == 0
+                finally:
+                    lib.adr_debug_knob(0, 0)
+            torch.cuda.synchronize()
+            if store in (2, 6):
+                shown = want.isfinite()
+                assert torch.equal(got[~shown].view(torch.int16), want[~shown].view(torch.int16)), (M, N, mask)
+                assert shown.all() == (mask == 0)
+                g, w = got[shown].double(), want[shown].double()
+                assert ((g - w).abs() <= w.abs() * 2.0 ** -10 + 8e-6 + 2.0 ** -24).all(), (M, N, mask)
+            else:
+                assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (M, N, mask)
+
+
 @pytest.mark.parametrize("M,K,N,tile", [(577, 4096, 4096, "128x96"), (1100, 4096, 4096, "192x128"),
                                         (130, 4096, 12288, "96x96"), (514, 5120, 13824, "192x192"),
                                         (1100, 4096, 11008, "256x224"), (2048, 4096, 12288, "256x192"),

@@ -25,7 +25,7 @@ def test_longer_rows_are_staged_through_registers(m):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tile,p", [(tile, EDGE) for tile in range(8)] + [(0, EDGE + 64), (1, EDGE + 64)])
+@pytest.mark.parametrize("tile,p", [(tile, EDGE) for tile in (*range(8), 10, 11, 12)] + [(0, EDGE + 64), (1, EDGE + 64)])
 def test_products_over_the_longest_rows(tile, p):
     """(a forced tile is no tile for longer rows: they have the staged kernels only)"""
     m, n = 257, 200

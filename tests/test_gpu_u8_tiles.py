@@ -40,3 +40,31 @@ def test_tiles_give_one_result(block):
             ref = x.double() @ w.double().t()
             rms = ref.pow(2).mean().sqrt()
             assert ((want.double() - ref).abs() / torch.maximum(ref.abs(), rms)).max() <= 2.0 ** -11 + 1e-5
+
+
+@pytest.mark.parametrize("beta", [0.5, 1.0])
+def test_tiles_add_to_the_result(beta):
+    """beta times the previous result, added to the 32-bit sum before its one rounding: the same bits from every tile, rows of
+    16-byte pieces and at any even address."""
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    lib, k = _ffi.lib(), 640
+    for tile, (bm, bn) in FORCED.items():
+        for m, n in ((bm + 1, 2 * bn + 8), (2 * bm - 5, bn + 13)):
+            q = torch.randint(0, 256, (n, k), dtype=torch.uint8, device="cuda", generator=gen)
+            s = (torch.rand(n, k // 32, device="cuda", generator=gen) * 0.019 + 0.001).half()
+            x, prev = (torch.randn(*shape, device="cuda", generator=gen).half() for shape in ((m, k), (m, n)))
+            outs = []
+            for knob in (5, tile):
+                outs.append(prev.clone())
+                try:
+                    assert lib.adr_debug_knob(1, knob) == 0
+                    assert lib.adr_matmul_nt_fp16u8(torch.cuda.current_stream().cuda_stream, outs[-1].data_ptr(),
+                                                    x.data_ptr(), q.data_ptr(), s.data_ptr(), m, k, n, 32, beta) == 0
+                finally:
+                    lib.adr_debug_knob(1, 0)
+            assert torch.equal(outs[1].view(torch.int16), outs[0].view(torch.int16)), (tile, m, n)
+            w = torch.zeros(n, k, dtype=torch.float16, device="cuda")
+            GpuKernels().dequantize_absmax_uint8(w, s, q)
+            ref = x.double() @ w.double().t() + beta * prev.double()
+            rms = ref.pow(2).mean().sqrt()
+            assert ((outs[0].double() - ref).abs() / torch.maximum(ref.abs(), rms)).max() <= 2.0 ** -11 + 1e-5

@@ -52,7 +52,8 @@ def slices(device_code, kernel):
 
 # (rows, columns, wavefronts along them, groups)
 @pytest.mark.parametrize("tile", [(256, 192, 4, 2, 1), (256, 128, 4, 2, 1), (128, 128, 4, 2, 1), (128, 64, 2, 2, 1),
-                                  (64, 64, 2, 2, 1), (128, 64, 2, 2, 2), (64, 64, 2, 2, 4)],
+                                  (64, 64, 2, 2, 1), (128, 64, 2, 2, 2), (64, 64, 2, 2, 4),
+                                  (192, 192, 2, 4, 1), (192, 128, 2, 4, 1), (96, 96, 3, 2, 1)],
                          ids=lambda t: "%dx%d_%dx%d_k%d" % t)
 def test_a_slice_waits_for_the_transfers_of_the_slice_before(device_code, tile):
     rows, columns, wm, wn, groups = tile

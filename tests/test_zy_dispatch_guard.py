@@ -12,10 +12,13 @@ from adrastea_amd import _ffi
 
 pytestmark = pytest.mark.gpu
 
-TILES = ["256x192", "256x128", "128x256", "128x192", "128x128", "128x64", "64x64", "256x160"]
+# by value of adr_debug_knob(0, ...)
+TILES = dict(enumerate(["256x192", "256x128", "128x256", "128x192", "128x128", "128x64", "64x64", "256x160",
+                        "256x224", "192x192", "192x128", "128x96", "96x96"], 1))
 SHAPES = [("clip_mlp_up", 2056, 1024, 4096), ("clip_mlp_down", 2056, 4096, 1024),
           ("llama_qkv", 2048, 4096, 12288), ("llama_o", 2048, 4096, 4096),
-          ("llama_gate_up", 2048, 4096, 11008), ("llama_down", 2048, 11008, 4096)]
+          ("llama_gate_up", 2048, 4096, 11008), ("llama_down", 2048, 11008, 4096),
+          ("llama_o_m1100", 1100, 4096, 4096), ("llama_gate_up_m1100", 1100, 4096, 11008)]
 
 
 def _time(fn, iters, warm=8):
@@ -31,13 +34,13 @@ def _time(fn, iters, warm=8):
     return e0.elapsed_time(e1) / iters
 
 
-def _measure(lib, fn, passes, knob=0, tiles=len(TILES)):
+def _measure(lib, fn, passes, knob=0, tiles=TILES):
     # (every measurement spans some ten milliseconds: shorter ones see the clock wander)
     iters = max(40, int(10.0 / max(_time(fn, 20), 1e-3)))
     best = {}
     try:
         for _ in range(passes):
-            for t in range(tiles + 1):
+            for t in (0, *tiles):
                 assert lib.adr_debug_knob(knob, t) == 0
                 best[t] = min(best.get(t, 1e30), _time(fn, iters))
     finally:
@@ -55,12 +58,12 @@ def test_forced_tile_changes_the_plan_and_not_the_result():
     buf = C.create_string_buffer(96)
     names = set()
     try:
-        for t in range(len(TILES) + 1):
+        for t in (0, *TILES):
             assert lib.adr_debug_knob(0, t) == 0
             assert lib.adr_matmul_f16_plan(buf, 96, 1, M, K, N, 1, N, 0, 1, K, 0, K, 1, 0, 0, 0, 0) == 0
             if t:
                 names.add(buf.value.decode())
-                assert buf.value.decode() == f"gemm_nt_mfma_dma_{TILES[t - 1]}x64"
+                assert buf.value.decode() == f"gemm_nt_mfma_dma_{TILES[t]}x64"
             out = torch.zeros(M, N, dtype=torch.float16, device="cuda")
             assert lib.adr_matmul_f16(torch.cuda.current_stream().cuda_stream, out.data_ptr(), a.data_ptr(),
                                       w.data_ptr(), 1, M, K, N, 1, N, 0, 1, K, 0, K, 1, 0, None, 0.0, 1.0,
@@ -93,13 +96,15 @@ def test_chosen_tile_is_within_five_percent_of_the_best_forced_one(case):
         ratio = best[0] / min(v for t, v in best.items() if t)
         if ratio <= 1.05:
             break
-    assert ratio <= 1.05, (case, {("chosen" if t == 0 else TILES[t - 1]): round(v * 1e3, 1) for t, v in best.items()})
+    assert ratio <= 1.05, (case, {("chosen" if t == 0 else TILES[t]): round(v * 1e3, 1) for t, v in best.items()})
 
 
-# the u8-weight kernel's tiles in the order of adr_debug_knob(1, 1 + i)
-U8_TILES = ["256x192", "256x128", "128x128", "128x64", "64x64", "128x64_k2", "64x64_k4"]
+# the u8-weight kernel's tiles by value of adr_debug_knob(1, ...)
+U8_TILES = {**dict(enumerate(["256x192", "256x128", "128x128", "128x64", "64x64", "128x64_k2", "64x64_k4"], 1)),
+            10: "192x192", 11: "192x128", 12: "96x96"}
 U8_SHAPES = [("down_m256", 256, 11008, 4096), ("o_m512", 512, 4096, 4096), ("down_m1024", 1024, 11008, 4096),
-             ("qkv_m128", 128, 4096, 12288), ("gate_m384", 384, 4096, 11008), ("qkv_m2048", 2048, 4096, 12288)]
+             ("qkv_m128", 128, 4096, 12288), ("gate_m384", 384, 4096, 11008), ("qkv_m2048", 2048, 4096, 12288),
+             ("qkv_m192", 192, 4096, 12288), ("o_m1280", 1280, 4096, 4096), ("qkv_m1408", 1408, 4096, 12288)]
 
 
 @pytest.mark.parametrize("case", U8_SHAPES, ids=[c[0] for c in U8_SHAPES])
@@ -123,11 +128,11 @@ def test_chosen_u8_tile_is_within_seven_percent_of_the_best_forced_one(case):
         fn()
     ratio = None
     for attempt in range(3):
-        best = _measure(lib, fn, passes=3, knob=1, tiles=len(U8_TILES))
+        best = _measure(lib, fn, passes=3, knob=1, tiles=U8_TILES)
         ratio = best[0] / min(v for t, v in best.items() if t)
         if ratio <= 1.07:
             break
-    assert ratio <= 1.07, (case, {("chosen" if t == 0 else U8_TILES[t - 1]): round(v * 1e3, 1) for t, v in best.items()})
+    assert ratio <= 1.07, (case, {("chosen" if t == 0 else U8_TILES[t]): round(v * 1e3, 1) for t, v in best.items()})
 
 
 @pytest.mark.parametrize("heads,d,n,lines", [(40, 128, 1376, 1408), (32, 128, 1824, 1856), (16, 64, 1888, 1920)])
