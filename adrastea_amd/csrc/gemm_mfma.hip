@@ -2399,8 +2399,10 @@ hipError_t launch_u8(hipStream_t stream, const MatmulArgs& a) {
   if (map.total < 0 || a.k % (BK * G) != 0) return hipErrorInvalidConfiguration;
   const dim3 grid((unsigned)map.total), block(WM * WN * G * 64);
   const int shift = __builtin_ctz(a.block_size);
-  // (128 x 128 on more than three quarters of the compute units is 1-2 % faster with its chunks apart: K5120 N13824 m=192
-  // 53.7 / 54.9 us, K1280 N5120 m=700 16.6 / 17.0; on fewer 1-3 % slower: K11008 N4096 m=768 101.7 / 98.6)
+  // (128 x 128 on more than three quarters of the compute units is faster with its chunks apart, by 1.1 % in the mean of 23
+  // products with resident weights and 0.1 % with cold ones; us: K5120 N13824 m=129 46.4 / 47.6 and 52.6 / 54.1, K13824 N5120
+  // m=520 115.9 / 118.3 and 122.0 / 122.1, K4096 N4096 m=900 42.7 / 43.1 and 44.0 / 43.4; on fewer units 1-3 % slower: K11008
+  // N4096 m=768 101.7 / 98.6)
   const bool apart = BM == 128 && BN == 128 && 4 * (int64_t)map.total > 3 * device_info_for_plan().cus;
   if (shift >= 4 && !apart)
     hipLaunchKernelGGL((gemm_nt_u8_pairs_kernel<BM, BN, WM, WN, MI16, BK, G>), grid, block, 0, stream, a, map, shift);
@@ -2525,9 +2527,8 @@ GemmChoice pick(const MatmulArgs& a, const Candidate* c, int n, double* cost_out
   return best;
 }
 
-// (the two large tiles run on 16x16x32 MFMAs: 9-16 % faster than on 32x32x16 on data that is not
-// constant -- qkv 170 -> 156 us, o 68 -> 58, down 162 -> 144 -- while the smaller tiles, which are
-// not bound by the power limit, gain nothing from it and stay on 32x32x16)
+// (the tiles run on 16x16x32 MFMAs: 9-16 % faster than on 32x32x16 on data that is not constant where the power limit
+// bounds them -- qkv 170 -> 156 us, o 68 -> 58, down 162 -> 144 -- but for 128 x 192, 128 x 64 and 64 x 64, which gain nothing from it)
 // The last five fill rounds that the others leave partly empty: 128 x 96 and 96 x 96 where 128 x 128 would occupy
 // a half to three quarters of the compute units, 192 x 128, 192 x 192 and 256 x 224 where the next smaller tile needs
 // a second round.  us, weights from HBM, without / with them: K4096 N1024 m=2056 30.0 / 26.6, K4096 N4096 m=577 33.6 /
