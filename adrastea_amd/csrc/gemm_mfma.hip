@@ -678,7 +678,8 @@ __global__ __launch_bounds__(WM* WN * 64, MINB) void gemm_nt_dma_kernel(MatmulAr
   // is computed per slice (us, clamped -> this: K1024 N2048 m=512 on 64x64 7.2 -> 7.05, K4096 N2048 m=1024 on 128x64
   // 29.5 -> 29.0, K1024 N4096 m=1400 on 192x128 14.2 -> 14.0; the large ones lost 1 % with it, 128x256 8 %).  The offsets
   // are unsigned: a view has fewer than 2^31 elements, so that the rows of every tile fit, whatever their pitch (the host's
-  // side of it: buffer_rows()).  Where the offset of a row beyond the matrix wraps, it lies inside the descriptor.
+  // side of it: buffer_rows()).  A row beyond the matrix whose offset wraps, or whose pitch is short, reads inside the
+  // descriptor at most: the range check of a buffer without stride counts the scalar offset.
   constexpr bool BUFFER = !NN && BM <= 192 && BN <= 192;
   const int dwave = ROLES ? wave % NWD : wave;  // index among the wavefronts issuing an operand
   const half_t* gA[BUFFER ? 1 : IA];
